@@ -4,8 +4,8 @@
 // scale multiply rounded to the activation dtype) needs x.A once per call.  lora_prep computes it
 // together with the transposed, zero-padded up-projection so the GEMM epilogue can run the
 // rank-R product as one more MFMA K-step.  linear_epilogue applies bias / LoRA / activation to an
-// already computed y for the paths that do not fuse them (GEMV, f32 activations, ranks above 16
-// and every result MLX's dtype promotion makes f32 from a bf16 product).
+// already computed y for the paths that do not fuse them (GEMV, f32 activations, ranks above 16,
+// further adapters and every result MLX's dtype promotion makes f32 from a bf16 product).
 #include "mlxq_common.h"
 
 namespace mlxq {
@@ -190,6 +190,7 @@ __global__ __launch_bounds__(kXaWaves * 64) void lora_xa_kernel(const uint16_t* 
 
 // DR = f32 (an f32 or fp16 activation, or f32 factors): xa[M,R] = x . A and lbt[N,R] = B^T in f32,
 // x and the factors widened exactly (MLX promotes the 16-bit operands of a mixed matmul to f32).
+// One thread per output element: the general form (K not a multiple of 16, unaligned x).
 template <typename XT, typename FT>
 __global__ void lora_prep_f32_kernel(const XT* __restrict__ x, int64_t M, int64_t K,
                                      const FT* __restrict__ A, const FT* __restrict__ B, int64_t N,
@@ -212,6 +213,133 @@ __global__ void lora_prep_f32_kernel(const XT* __restrict__ x, int64_t M, int64_
   }
 }
 
+// The same on v_mfma_f32_16x16x4_f32, whose products and sums are f32's own.  A workgroup owns 16
+// rows of x and 16 * NCB columns of xa; its 8 waves split K and reduce through LDS.  Bound by the
+// x stream and by the loads of A: per 16 k, a lane loads 4 consecutive x values of its row and, for
+// each of those 4 k, the NCB adjacent columns (16 columns x NCB) of A its column index owns, so
+// MFMA t multiplies k = 4 q + t of both sides with no transpose, and NCB = 2 or 4 (rank a multiple
+// of it, A aligned to the wider load) halves or quarters both the loads of A and the passes over x.
+// One thread per output, walking K alone, had taken 576 us for x [4608, 3072] f32, rank 32, where
+// x's bytes take 11.5 us at copy speed; with lora_epilogue_kernel below, the whole linear
+// [4608, 3072] x [12288, 3072]^T with rank 32 and GELU went from 7196 to 1043 us.
+// Workgroups past xa_blocks write lbt, eight ranks of one n per thread (loads coalesced over n).
+template <typename XT, typename FT, int NCB>
+__global__ __launch_bounds__(kXaWaves * 64) void lora_xa_f32_kernel(
+    const XT* __restrict__ x, int64_t M, int64_t K, const FT* __restrict__ A, const FT* __restrict__ B,
+    int64_t N, int rank, int R, float* __restrict__ xa, float* __restrict__ lbt, int xa_blocks) {
+  __shared__ float red[NCB][kXaWaves][16 * 16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if ((int)blockIdx.x >= xa_blocks) {
+    if (blockIdx.y != 0) return;
+    const int64_t u = ((int64_t)blockIdx.x - xa_blocks) * (kXaWaves * 64) + tid;
+    if (u < N * (R / 8)) {
+      const int64_t n = u % N;
+      const int r8 = (int)(u / N) * 8;
+      f32x4 v[2];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[j >> 2][j & 3] = r8 + j < rank ? Act<FT>::ld(B, (int64_t)(r8 + j) * N + n) : 0.0f;
+#pragma unroll
+      for (int h = 0; h < 2; ++h) *reinterpret_cast<f32x4*>(lbt + n * R + r8 + 4 * h) = v[h];
+    }
+    return;
+  }
+  constexpr int U = NCB == 4 ? 2 : 4;  // 16-deep steps per chunk, double-buffered
+  struct alignas(4 * sizeof(XT)) XV { XT v[4]; };
+  struct alignas(NCB * sizeof(FT)) AV { FT v[NCB]; };
+  struct Chunk {
+    XV x[U];
+    AV a[U][4];
+  };
+  const int c16 = lane & 15, q = lane >> 4;
+  const int64_t m0 = (int64_t)blockIdx.x * 16;
+  const int r0 = blockIdx.y * 16 * NCB;
+  const int col = r0 + c16 * NCB;  // this lane's first column; rank is a multiple of NCB
+  const int KS = (int)(K / 16);
+  const int ks0 = __builtin_amdgcn_readfirstlane((int)((int64_t)wave * KS / kXaWaves));
+  const int ks1 = __builtin_amdgcn_readfirstlane((int)((int64_t)(wave + 1) * KS / kXaWaves));
+  const XT* xp = x + (m0 + c16 < M ? m0 + c16 : M - 1) * K + 4 * q;
+  const FT* ap = A + (int64_t)(4 * q) * rank + (col < rank ? col : 0);  // padding columns: not stored
+  auto load1 = [&](int ks, XV& xv, AV (&av)[4]) {
+    xv = *reinterpret_cast<const XV*>(xp + (int64_t)ks * 16);
+#pragma unroll
+    for (int t = 0; t < 4; ++t) av[t] = *reinterpret_cast<const AV*>(ap + ((int64_t)ks * 16 + t) * rank);
+  };
+  f32x4 acc[NCB];
+#pragma unroll
+  for (int c = 0; c < NCB; ++c) acc[c] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  auto mac1 = [&](const XV& xv, const AV (&av)[4]) {
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+#pragma unroll
+      for (int c = 0; c < NCB; ++c)
+        acc[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(Act<XT>::ld(xv.v, t), Act<FT>::ld(av[t].v, c), acc[c], 0, 0, 0);
+  };
+  auto load = [&](int ks, Chunk& c) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load1(ks + u, c.x[u], c.a[u]);
+  };
+  auto mac = [&](const Chunk& c) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) mac1(c.x[u], c.a[u]);
+  };
+  // Whole chunks, the next one's loads ahead of this one's products, then single steps; every
+  // condition is wave-uniform.
+  const int full = (ks1 - ks0) / U;
+  if (full > 0) {
+    Chunk c0, c1;
+    load(ks0, c0);
+    for (int i = 0; i < full; i += 2) {
+      if (i + 1 < full) load(ks0 + (i + 1) * U, c1);
+      mac(c0);
+      if (i + 1 < full) {
+        if (i + 2 < full) load(ks0 + (i + 2) * U, c0);
+        mac(c1);
+      }
+    }
+  }
+  for (int ks = ks0 + full * U; ks < ks1; ++ks) {
+    XV xv;
+    AV av[4];
+    load1(ks, xv, av);
+    mac1(xv, av);
+  }
+#pragma unroll
+  for (int c = 0; c < NCB; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) red[c][wave][(4 * q + e) * 16 + c16] = acc[c][e];
+  __syncthreads();
+  for (int i = tid; i < 256 * NCB; i += kXaWaves * 64) {
+    const int m = i / (16 * NCB), cc = i % (16 * NCB);  // cc: column r0 + cc = block cc % NCB, index cc / NCB
+    float v = 0.0f;
+#pragma unroll
+    for (int w = 0; w < kXaWaves; ++w) v += red[cc % NCB][w][m * 16 + cc / NCB];
+    if (m0 + m < M && r0 + cc < R) xa[(m0 + m) * R + r0 + cc] = r0 + cc < rank ? v : 0.0f;
+  }
+}
+
+template <typename XT, typename FT>
+static int lora_prep_f32(const void* x, int64_t M, int64_t K, const void* A, const void* B, int64_t N, int rank,
+                         int R, void* xa, void* lbt, hipStream_t st) {
+  const auto aligned = [](const void* p, size_t a) { return reinterpret_cast<uintptr_t>(p) % a == 0; };
+  const int64_t xa_blocks = (M + 15) / 16, bt_blocks = (N * (R / 8) + kXaWaves * 64 - 1) / (kXaWaves * 64);
+  if (K % 16 == 0 && aligned(x, 4 * sizeof(XT)) && K < (1LL << 31) && xa_blocks + bt_blocks < (1LL << 31)) {
+#define MLXQ_XA(C)                                                                                               \
+  hipLaunchKernelGGL((lora_xa_f32_kernel<XT, FT, C>), dim3((unsigned)(xa_blocks + bt_blocks), (unsigned)((R + 16 * C - 1) / (16 * C))), \
+                     dim3(kXaWaves * 64), 0, st, (const XT*)x, M, K, (const FT*)A, (const FT*)B, N, rank, R,     \
+                     (float*)xa, (float*)lbt, (int)xa_blocks)
+    if (R > 32 && rank % 4 == 0 && aligned(A, 4 * sizeof(FT))) MLXQ_XA(4);
+    else if (R > 16 && rank % 2 == 0 && aligned(A, 2 * sizeof(FT))) MLXQ_XA(2);
+    else MLXQ_XA(1);
+#undef MLXQ_XA
+    return check_launch("lora_prep");
+  }
+  const int64_t blocks = (M * R + N * R + 255) / 256;
+  if (blocks > 0x7fffffff) return set_error(MLXQ_EINVAL, "lora: problem too large");
+  hipLaunchKernelGGL((lora_prep_f32_kernel<XT, FT>), dim3((unsigned)blocks), dim3(256), 0, st, (const XT*)x, M, K,
+                     (const FT*)A, (const FT*)B, N, rank, R, (float*)xa, (float*)lbt);
+  return check_launch("lora_prep");
+}
+
 int run_lora_prep(const void* x, int x_dtype, int64_t M, int64_t K, const void* A, const void* B,
                   int lora_dtype, int64_t N, int rank, int R, void* xa, void* lbt, hipStream_t st) {
   const int64_t total = M * R + N * R;
@@ -219,24 +347,13 @@ int run_lora_prep(const void* x, int x_dtype, int64_t M, int64_t K, const void* 
   const int64_t blocks = (total + 255) / 256;
   if (blocks > 0x7fffffff) return set_error(MLXQ_EINVAL, "lora: problem too large");
   if (x_dtype != MLXQ_BFLOAT16 || lora_dtype != MLXQ_BFLOAT16) {
-    const dim3 g((unsigned)blocks), b(256);
-    if (x_dtype == MLXQ_FLOAT16) {
-      if (lora_dtype == MLXQ_BFLOAT16)
-        hipLaunchKernelGGL((lora_prep_f32_kernel<_Float16, uint16_t>), g, b, 0, st, (const _Float16*)x, M, K,
-                           (const uint16_t*)A, (const uint16_t*)B, N, rank, R, (float*)xa, (float*)lbt);
-      else
-        hipLaunchKernelGGL((lora_prep_f32_kernel<_Float16, float>), g, b, 0, st, (const _Float16*)x, M, K,
-                           (const float*)A, (const float*)B, N, rank, R, (float*)xa, (float*)lbt);
-    } else if (x_dtype == MLXQ_BFLOAT16)
-      hipLaunchKernelGGL((lora_prep_f32_kernel<uint16_t, float>), g, b, 0, st, (const uint16_t*)x, M, K,
-                         (const float*)A, (const float*)B, N, rank, R, (float*)xa, (float*)lbt);
-    else if (lora_dtype == MLXQ_BFLOAT16)
-      hipLaunchKernelGGL((lora_prep_f32_kernel<float, uint16_t>), g, b, 0, st, (const float*)x, M, K,
-                         (const uint16_t*)A, (const uint16_t*)B, N, rank, R, (float*)xa, (float*)lbt);
-    else
-      hipLaunchKernelGGL((lora_prep_f32_kernel<float, float>), g, b, 0, st, (const float*)x, M, K,
-                         (const float*)A, (const float*)B, N, rank, R, (float*)xa, (float*)lbt);
-    return check_launch("lora_prep");
+    const bool fb = lora_dtype == MLXQ_BFLOAT16;
+    if (x_dtype == MLXQ_FLOAT16)
+      return fb ? lora_prep_f32<_Float16, uint16_t>(x, M, K, A, B, N, rank, R, xa, lbt, st)
+                : lora_prep_f32<_Float16, float>(x, M, K, A, B, N, rank, R, xa, lbt, st);
+    if (x_dtype == MLXQ_BFLOAT16) return lora_prep_f32<uint16_t, float>(x, M, K, A, B, N, rank, R, xa, lbt, st);
+    return fb ? lora_prep_f32<float, uint16_t>(x, M, K, A, B, N, rank, R, xa, lbt, st)
+              : lora_prep_f32<float, float>(x, M, K, A, B, N, rank, R, xa, lbt, st);
   }
   const int64_t bt_blocks = (N * R + kXaWaves * 64 - 1) / (kXaWaves * 64);
   if (K % 32 == 0 && M < (1LL << 31) / 16 && K < (1LL << 31) && bt_blocks < (1LL << 30)) {
@@ -280,22 +397,10 @@ __device__ __forceinline__ float rnd_if(bool bf16, float v) { return bf16 ? roun
 // sequence of LinearBase::forward's bias add and AdaptableLinear::forward's residual sum
 // (reference src/adapters.rs:318-320,543-549, Adapter::residual :260-270).  A bf16 activation is
 // the bf16 table's entry of its input; in f32 it is evaluated (GELU and the exact GELU as the
-// f32 erf form, the tanh GELU op by op).
-template <typename YI, typename YO>
-__global__ void linear_epilogue_kernel(LinearEpilogueArgs a) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.M * a.N) return;
-  const int64_t m = t / a.N, n = t % a.N;
-  float o = Act<YI>::ld(static_cast<const YI*>(a.y_in), t);
+// f32 erf form, the tanh GELU op by op).  has_r: r is the residual's product, before rounding.
+__device__ __forceinline__ float epilogue_finish(const LinearEpilogueArgs& a, float o, int64_t n, bool has_r, float r) {
   if (a.bias) o = rnd_if(a.d1_bf16, o + ld_any(a.bias, a.bias_bf16, n));
-  if (a.R > 0) {
-    float r = 0.0f;
-    for (int k = 0; k < a.R; ++k)
-      r = fmaf(ld_any(a.xa, a.dr_bf16, m * a.R + k), ld_any(a.lbt, a.dr_bf16, n * a.R + k), r);
-    o = rnd_if(a.d2_bf16, o + rnd_if(a.dr_bf16, rnd_if(a.dr_bf16, r) * a.lora_scale));
-  } else if (a.res) {
-    o = rnd_if(a.d2_bf16, o + rnd_if(a.dr_bf16, rnd_if(a.dr_bf16, a.res[t]) * a.lora_scale));
-  }
+  if (has_r) o = rnd_if(a.d2_bf16, o + rnd_if(a.dr_bf16, rnd_if(a.dr_bf16, r) * a.lora_scale));
   const bool act_bf16 = a.d2_bf16;  // the activation's input dtype
   if (a.act == MLXQ_ACT_GELU) {
     o = gelu_erf(o);
@@ -303,7 +408,84 @@ __global__ void linear_epilogue_kernel(LinearEpilogueArgs a) {
     if (act_bf16) o = bf16_bits_to_f32(a.act_table[f32_to_bf16_bits(o)]);
     else o = a.act == MLXQ_ACT_GELU_TANH ? gelu_tanh<false>(o) : gelu_erf(o);
   }
-  Act<YO>::st(static_cast<YO*>(a.y_out), t, o);
+  return o;
+}
+
+// Without LoRA (R == 0): one thread per output.
+template <typename YI, typename YO>
+__global__ void linear_epilogue_kernel(LinearEpilogueArgs a) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.M * a.N) return;
+  const float o = Act<YI>::ld(static_cast<const YI*>(a.y_in), t);
+  Act<YO>::st(static_cast<YO*>(a.y_out), t, epilogue_finish(a, o, t % a.N, a.res != nullptr, a.res ? a.res[t] : 0.0f));
+}
+
+// With LoRA (R > 0): r = xa . lbt^T on the matrix cores (bf16 operands for DR = bf16, f32 operands
+// for DR = f32, the products and sums f32's own), one 32 x 64 block of outputs per wave.  Meant to
+// run at the rate of reading y_in and writing y_out; one thread per output, reading 2 R operands
+// for each, had taken 5.7 ms for [4608, 12288] f32 at R = 32, where y's 453 MB take 92 us.  The
+// activation rows are the MFMA's A side, so a lane holds 16 rows m of one column; its two columns
+// are neighbours (n = 2 (lane & 31) + j), so a wave's access to a row of y is 64 contiguous
+// elements.
+template <typename YI, typename YO, bool DRB>
+__global__ __launch_bounds__(256) void lora_epilogue_kernel(LinearEpilogueArgs a, int64_t tiles_n) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r32 = lane & 31, half = lane >> 5;
+  const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * 32;
+  const int64_t n0 = (int64_t)(blockIdx.x % tiles_n) * 256 + wave * 64;
+  const int64_t mr = m0 + r32 < a.M ? m0 + r32 : a.M - 1;  // rows and columns past the ends repeat
+  int64_t nr[2];                                           // the last one and are never stored
+#pragma unroll
+  for (int j = 0; j < 2; ++j) nr[j] = n0 + 2 * r32 + j < a.N ? n0 + 2 * r32 + j : a.N - 1;
+  f32x16 r[2] = {f32x16{}, f32x16{}};
+  for (int k = 0; k < a.R; k += 16) {
+    if constexpr (DRB) {
+      const bf16x8 xv = *reinterpret_cast<const bf16x8*>(static_cast<const uint16_t*>(a.xa) + mr * a.R + k + 8 * half);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const bf16x8 bv = *reinterpret_cast<const bf16x8*>(static_cast<const uint16_t*>(a.lbt) + nr[j] * a.R + k + 8 * half);
+        r[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xv, bv, r[j], 0, 0, 0);
+      }
+    } else {
+      const float* xp = static_cast<const float*>(a.xa) + mr * a.R + k + 8 * half;
+      const f32x4 x0 = *reinterpret_cast<const f32x4*>(xp), x1 = *reinterpret_cast<const f32x4*>(xp + 4);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        const float* bp = static_cast<const float*>(a.lbt) + nr[j] * a.R + k + 8 * half;
+        const f32x4 b0 = *reinterpret_cast<const f32x4*>(bp), b1 = *reinterpret_cast<const f32x4*>(bp + 4);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          r[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x0[t], b0[t], r[j], 0, 0, 0);
+          r[j] = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[t], b1[t], r[j], 0, 0, 0);
+        }
+      }
+    }
+  }
+  const int64_t n = n0 + 2 * r32;
+  if (n >= a.N) return;
+  const YI* const yi = static_cast<const YI*>(a.y_in);
+  YO* const yo = static_cast<YO*>(a.y_out);
+  struct alignas(2 * sizeof(YI)) VI { YI v[2]; };
+  struct alignas(2 * sizeof(YO)) VO { YO v[2]; };
+  // Pairs need an even N (a row's start aligned to two elements); both pointers are.
+  const bool pairs = a.N % 2 == 0 && reinterpret_cast<uintptr_t>(a.y_in) % sizeof(VI) == 0 &&
+                     reinterpret_cast<uintptr_t>(a.y_out) % sizeof(VO) == 0;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const int64_t m = m0 + 8 * (v >> 2) + 4 * half + (v & 3);
+    if (m >= a.M) continue;
+    const int64_t t = m * a.N + n;
+    if (pairs) {
+      const VI in = *reinterpret_cast<const VI*>(yi + t);
+      VO out;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) Act<YO>::st(out.v, j, epilogue_finish(a, Act<YI>::ld(in.v, j), n + j, true, r[j][v]));
+      *reinterpret_cast<VO*>(yo + t) = out;
+    } else {
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+        if (n + j < a.N) Act<YO>::st(yo, t + j, epilogue_finish(a, Act<YI>::ld(yi, t + j), n + j, true, r[j][v]));
+    }
+  }
 }
 
 int run_linear_epilogue(const LinearEpilogueArgs& a, hipStream_t st) {
@@ -314,7 +496,23 @@ int run_linear_epilogue(const LinearEpilogueArgs& a, hipStream_t st) {
   const bool table_act = a.act == MLXQ_ACT_GELU_TANH || a.act == MLXQ_ACT_GELU_EXACT;
   if (table_act && a.d2_bf16 && a.act_table == nullptr)
     return set_error(MLXQ_EINVAL, "linear epilogue: activation table missing");
-  const dim3 g((unsigned)blocks), b(256);
+  const dim3 b(256);
+  if (a.R > 0) {
+    const int64_t tiles_n = (a.N + 255) / 256, tiles = (a.M + 31) / 32 * tiles_n;
+    const dim3 g((unsigned)tiles);
+#define MLXQ_LE(YI, YO)                                                                             \
+  do {                                                                                              \
+    if (a.dr_bf16) hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, true>), g, b, 0, st, a, tiles_n); \
+    else hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, false>), g, b, 0, st, a, tiles_n);        \
+  } while (0)
+    if (a.y_in_bf16 && a.y_out_bf16) MLXQ_LE(uint16_t, uint16_t);
+    else if (a.y_in_bf16) MLXQ_LE(uint16_t, float);
+    else if (a.y_out_bf16) MLXQ_LE(float, uint16_t);
+    else MLXQ_LE(float, float);
+#undef MLXQ_LE
+    return check_launch("linear_epilogue");
+  }
+  const dim3 g((unsigned)blocks);
   if (a.y_in_bf16 && a.y_out_bf16) hipLaunchKernelGGL((linear_epilogue_kernel<uint16_t, uint16_t>), g, b, 0, st, a);
   else if (a.y_in_bf16) hipLaunchKernelGGL((linear_epilogue_kernel<uint16_t, float>), g, b, 0, st, a);
   else if (a.y_out_bf16) hipLaunchKernelGGL((linear_epilogue_kernel<float, uint16_t>), g, b, 0, st, a);
