@@ -601,13 +601,20 @@ int mlxq_linear(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t
     if ((rc = epilogue_table(a, st))) return rc;
     return run_linear_epilogue(a, st);
   }
-  // An f32 product at GEMM size fuses the bias and the activation (all in f32) unless a LoRA
-  // adapter needs the elementwise epilogue.
-  if (!p.d0_bf16 && M > 8 && !p.lora) {
+  // An f32 product at GEMM size fuses the bias, an f32 LoRA residual and the activation (all in
+  // f32); a bf16 residual (bf16 x and factors against f32 scales) and the shapes of the three-pass
+  // kernel need the elementwise epilogue.
+  if (!p.d0_bf16 && M > 8 && (!p.lora || (!p.dr_bf16 && qmm_f32_strip_fits(K, N)))) {
     F32Epilogue fe;
     fe.bias = p.bias ? ep->bias : nullptr;
     fe.bias_bf16 = p.bias && ep->bias_dtype == MLXQ_BFLOAT16;
     fe.act = p.act;
+    if (p.lora) {
+      fe.xa = (const float*)xa;
+      fe.lbt = (const float*)lbt;
+      fe.R = p.R;
+      fe.lora_scale = scale;
+    }
     return run_qmm_f32(x, x_dtype, M, K, wq, scales, biases, sb_dtype, N, group_size, bits, y, st, fe);
   }
   // The product in D0, straight into y when y has that dtype; a bf16 product whose result

@@ -109,12 +109,20 @@ struct F32Epilogue {
   const void* bias = nullptr;  // [N]
   bool bias_bf16 = false;
   int act = 0;                 // mlxq_activation
+  const float* xa = nullptr;   // [M, R] x . A and [N, R] B^T of a LoRA residual in f32
+  const float* lbt = nullptr;
+  int R = 0;                   // padded rank, 0 = no LoRA
+  float lora_scale = 1.0f;
 };
 // Large-M GEMM for operands MLX computes in f32 (f32 x and/or f32 scales), f32 y, as three bf16
 // MFMA passes over two-term bf16 splits of x and of the f32-dequantized weights.
 int run_qmm_f32(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                 const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, hipStream_t st,
                 const F32Epilogue& epi = F32Epilogue{});
+bool qmm_f32_strip_fits(int64_t K, int64_t N);
+int run_qmm_f32_strip(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
+                      const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, const F32Epilogue& epi,
+                      hipStream_t st);
 // y[M, N] f32 = x[M, K] . d^T for a dense d [N, K] in d_dtype, cast to bf16 against bf16 x, on
 // the matrix cores (bf16 passes over two-term splits of the f32 operands).  K % 32 == 0.
 int run_dense_f32(const void* x, int x_dtype, int64_t M, int64_t K, const void* d, int d_dtype,

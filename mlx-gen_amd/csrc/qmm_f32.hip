@@ -14,12 +14,11 @@
 // The dropped x_lo.w_lo term and the two representation errors are each below 2^-16 of |x.w|, so
 // the result is within ~1e-5 relative (Frobenius) of the f32 product, against ~1e-3 for a plain
 // bf16 product.  With bf16 activations (f32 scales) x_lo is zero and the third pass is skipped;
-// fp16 activations split exactly (x_hi + x_lo == x), so against exact bf16 code operands (the
-// factored kernel) their products are exact.
+// fp16 activations split exactly (x_hi + x_lo == x).
 // Weights are dequantized exactly as fma(code, scale, bias) in f32 (scale and bias widened
-// exactly from bf16), then split.  That three-pass kernel serves group size 32 and the LoKr dense
-// product; group sizes 64 and 128 take the factored kernel further down (qmm_f32c_kernel: the
-// codes themselves as exact bf16 operands, two passes for f32 x).
+// exactly from bf16), then split.  This kernel serves K % 64 == 32 (group size 32), widths past the
+// factored kernel's reach and the LoKr dense product; everything else takes the factored kernel
+// (qmm_f32_strip.hip: the codes themselves as exact operands, one pass for fp16 x, two for f32 x).
 //
 // Structure: a workgroup of 8 waves (2 x 4, 64 x 64 each) per 128 x 256 output tile (the LoKr
 // dense product: 4 waves, 2 x 2, per 128 x 128 tile), K advanced BK = 32 at a time through a
@@ -433,345 +432,6 @@ __global__ __launch_bounds__(WAVES * 64) void qmm_f32_kernel(const XT* __restric
   f32_store_dispatch<EPI>(epi.act, store);
 }
 
-// The factored form for group sizes 64 and 128: since
-//     x . w = sum_g ( s_g * sum_{k in g} x_k c_k  +  b_g * X_g ),   X_g = sum_{k in g} x_k,
-// the codes c (small integers, exact in bf16) are the weight operand and only the activations are
-// split: x_hi.c + x_lo.c is two MFMA passes for f32 x (one for bf16 x) instead of three, with no
-// dequantization or weight split.  Each group's product accumulates in `acc` (the first MFMA of a
-// group starts from zero) and is folded into the running f32 sum y by two FMAs per output with the
-// group's scale and bias (one per weight row) and activation sum (one per activation row), which
-// the staging threads leave in two small LDS tables next to the step's tiles (with bf16 scales and
-// K / GS a multiple of 16, one FMA: the bias term runs on the matrix cores, see BMF).  The loop is
-// unrolled by the group's GS/32 steps, so group starts and ends are compile-time positions.
-// Tiles, waves, buffers and the load pipeline are those of qmm_f32_kernel (128 x 256, 8 waves of
-// 64 x 64, 32-deep K steps, loads two steps ahead).
-template <typename XT, typename SB, int BITS, int GS, bool EPI, bool BMF, int WAVES, int BN>
-__global__ __launch_bounds__(WAVES * 64, 8 / WAVES) void qmm_f32c_kernel(const XT* __restrict__ x, int64_t M, int64_t K,
-                                                   const uint32_t* __restrict__ wq,
-                                                   const SB* __restrict__ scales,
-                                                   const SB* __restrict__ biases, int64_t N,
-                                                   float* __restrict__ y, F32Epilogue epi) {
-  constexpr bool XLO = XStore<XT>::LO;  // activations carry a low part
-  constexpr int BK = 32;
-  constexpr int BM = kF32BM, NT = WAVES * 64;
-  constexpr int WGN = WAVES / 2;
-  constexpr int WM = BM / 2, WN = BN / WGN, TM = WM / 32, TN = WN / 32;
-  constexpr int CPR = BK / 8;                // 16-byte bf16 chunks per tile row
-  constexpr int A_LD = BM * CPR / NT;        // activation chunks per thread per step (1 or 2)
-  constexpr int CPT = BN * BK / NT;          // codes per thread per step (16)
-  constexpr int WPT = CPT * BITS / 32;       // their packed words
-  constexpr int PPR = BK / CPT;              // threads per weight row (2)
-  constexpr int GSTEP = GS / BK;             // steps per group (2 or 4)
-  constexpr int TA = BM * BK * 2, TB = BN * BK * 2;
-  constexpr int OFF_SB = 2 * TA + TB, OFF_X = OFF_SB + BN * 8, BUF = OFF_X + BM * 4;
-  static_assert(A_LD * NT == BM * CPR && CPT == 16 && GSTEP >= 2 && GSTEP % 2 == 0 && WPT >= 1, "tile shape");
-  // Per buffer: x_hi, x_lo, codes, then the (s, b) pairs of the tile's weight rows and the
-  // activation sums of its rows for the group the buffer's step closes.
-  __shared__ __attribute__((aligned(16))) unsigned char smem[2][BUF];
-  // BMF (bf16 scales, K / GS a multiple of 16): the bias term b.X goes to the matrix cores, 16
-  // groups at a time: each group's bf16 biases per weight row and hi/lo split activation sums per
-  // activation row wait in 16-group tables (rows of 32 bytes), and every 16th group adds
-  // b[n, g..g+15] . X[g..g+15, m] into y with one MFMA pair per block.  The per-group fold is then
-  // one FMA per output, y += s * acc.
-  constexpr int BT = BN * 32, XT_ = BM * 32;
-  static_assert(!BMF || std::is_same<SB, uint16_t>::value, "bias MFMA needs bf16 biases (exact bf16 operands)");
-  __shared__ __attribute__((aligned(16))) unsigned char btab[BMF ? BT + 2 * XT_ : 16];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
-  const int wm = wave / WGN, wn = wave % WGN;
-  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
-  int64_t tm, tn;
-  f32_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int64_t bm0 = tm * BM, bn0 = tn * BN;
-  const int64_t kwords = K * BITS / 32;
-  const int64_t groups = K / GS;
-  const int ksteps = (int)(K / BK);  // a multiple of GSTEP (K % GS == 0)
-
-  // Staging registers, two slots (see qmm_f32_kernel): thread tid stages activation chunks
-  // id = tid + NT i (row id / 4, chunk id % 4), and codes CPT of weight row tid / 2 with that row's
-  // scale and bias.
-  u32x4 a_reg[2][A_LD][XStore<XT>::W];
-  uint32_t b_reg[2][WPT];
-  float s_reg[2], z_reg[2];
-  float xrun[A_LD];  // each staged row's activation sum over the current group's steps so far
-
-  auto load_global = [&](int kt, auto SLOT) {
-    constexpr int sl = decltype(SLOT)::value;
-    const int64_t k0 = (int64_t)kt * BK;
-#pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      const int id = tid + NT * i;
-      const int row = id / CPR, c = id % CPR;
-      const int64_t m = bm0 + row < M ? bm0 + row : M - 1;
-#pragma unroll
-      for (int h = 0; h < XStore<XT>::W; ++h)
-        a_reg[sl][i][h] = reinterpret_cast<const u32x4*>(x + m * K + k0 + c * 8)[h];
-    }
-    const int row = tid / PPR, part = tid % PPR;
-    const int64_t n = bn0 + row < N ? bn0 + row : N - 1;
-    const int64_t kc = k0 + part * CPT;
-    const uint32_t* src = wq + n * kwords + kc * BITS / 32;
-    if constexpr (WPT == 1) {
-      b_reg[sl][0] = src[0];
-    } else {
-#pragma unroll
-      for (int q = 0; q < WPT; q += 2) {
-        const u32x2 v = *reinterpret_cast<const u32x2*>(src + q);
-        b_reg[sl][q] = v[0];
-        b_reg[sl][q + 1] = v[1];
-      }
-    }
-    const int64_t g = n * groups + kc / GS;
-    s_reg[sl] = SBLoad<SB>::ld(scales, g);
-    z_reg[sl] = SBLoad<SB>::ld(biases, g);
-  };
-
-  // Step `POS` (its position in its group `grp`) from register slot SLOT into LDS buffer buf.
-  auto store_lds = [&](int buf, auto SLOT, auto POS, int grp) {
-    constexpr int sl = decltype(SLOT)::value;
-    constexpr int pos = decltype(POS)::value;
-    unsigned char* Ah = smem[buf];
-    unsigned char* Al = smem[buf] + TA;
-    unsigned char* Bc = smem[buf] + 2 * TA;
-#pragma unroll
-    for (int i = 0; i < A_LD; ++i) {
-      const int id = tid + NT * i;
-      const int row = id / CPR, c = id % CPR;
-      float t = 0.0f;
-      if constexpr (XLO) {
-        u32x4 hi, lo;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float v0, v1;
-          XStore<XT>::pair(a_reg[sl][i], e, v0, v1);
-          t += v0 + v1;
-          const u32x2 p = split2(v0, v1);
-          hi[e] = p[0];
-          lo[e] = p[1];
-        }
-        *reinterpret_cast<u32x4*>(Ah + swz32<BK>(row, c)) = hi;
-        *reinterpret_cast<u32x4*>(Al + swz32<BK>(row, c)) = lo;
-      } else {
-        const u32x4 v = a_reg[sl][i][0];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) t += __uint_as_float(v[e] << 16) + __uint_as_float(v[e] & 0xffff0000u);
-        *reinterpret_cast<u32x4*>(Ah + swz32<BK>(row, c)) = v;
-      }
-      // the row's sum over this step: its 4 chunks sit in 4 consecutive lanes
-      t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0xb1, 0xf, 0xf, true));
-      t += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(t), 0x4e, 0xf, 0xf, true));
-      xrun[i] = pos == 0 ? t : xrun[i] + t;
-      if constexpr (pos == GSTEP - 1) {
-        if (c == 0) {
-          reinterpret_cast<float*>(smem[buf] + OFF_X)[row] = xrun[i];
-          if constexpr (BMF) {
-            const uint16_t hb = f32_to_bf16_bits(xrun[i]);
-            const uint16_t lb = f32_to_bf16_bits(xrun[i] - bf16_bits_to_f32(hb));
-            reinterpret_cast<uint16_t*>(btab + BT)[row * 16 + (grp & 15)] = hb;
-            reinterpret_cast<uint16_t*>(btab + BT + XT_)[row * 16 + (grp & 15)] = lb;
-          }
-        }
-      }
-    }
-    const int row = tid / PPR, part = tid % PPR;
-    const int c0 = part * CPT / 8;  // LDS chunk c holds k [8c, 8c + 8) of the step
-    if constexpr (BITS == 4) {
-      // word q: codes 8q..8q+7 in natural order (low nibble first) -> chunk c0 + q, as bf16(c).
-      // The nibbles are split into bytes and interleaved back into code order (bytes c0..c3 and
-      // c4..c7); a byte c <= 15 read as OCP fp8 E4M3 is exactly c * 2^-9, so one scaled convert
-      // turns two code bytes into two exact bf16 values: 9 VALU ops per word instead of 20.
-#pragma unroll
-      for (int q = 0; q < WPT; ++q) {
-        const uint32_t w = b_reg[sl][q];
-        const uint32_t ev = w & 0x0f0f0f0fu, od = (w >> 4) & 0x0f0f0f0fu;  // c0 c2 c4 c6 / c1 c3 c5 c7
-        const uint32_t n0 = __builtin_amdgcn_perm(od, ev, 0x05010400u);     // c0 c1 c2 c3
-        const uint32_t n1 = __builtin_amdgcn_perm(od, ev, 0x07030602u);     // c4 c5 c6 c7
-        u32x4 cv;
-        cv[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n0, 512.0f, false));
-        cv[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n0, 512.0f, true));
-        cv[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n1, 512.0f, false));
-        cv[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n1, 512.0f, true));
-        *reinterpret_cast<u32x4*>(Bc + swz32<BK>(row, c0 + q)) = cv;
-      }
-    } else {
-#pragma unroll
-      for (int p = 0; p < WPT / 2; ++p) {
-        u32x4 cv;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const uint32_t w = b_reg[sl][2 * p + h];
-          cv[2 * h] = pack_bf16x2((float)(w & 0xffu), (float)((w >> 8) & 0xffu));
-          cv[2 * h + 1] = pack_bf16x2((float)((w >> 16) & 0xffu), (float)(w >> 24));
-        }
-        *reinterpret_cast<u32x4*>(Bc + swz32<BK>(row, c0 + p)) = cv;
-      }
-    }
-    if constexpr (pos == GSTEP - 1) {
-      if (part == 0) {
-        *reinterpret_cast<f32x2*>(smem[buf] + OFF_SB + row * 8) = f32x2{s_reg[sl], z_reg[sl]};
-        if constexpr (BMF)
-          reinterpret_cast<uint16_t*>(btab)[row * 16 + (grp & 15)] = (uint16_t)(__float_as_uint(z_reg[sl]) >> 16);
-      }
-    }
-  };
-
-  f32x16 acc[TM][TN], yv[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; ++i)
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) yv[i][j][v] = 0.0f;
-
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, 1>;
-  const int r32 = lane & 31, half = lane >> 5;
-  // Step products from LDS buffer buf; the first MFMA of a group's first step starts from zero.
-  auto mfma_step = [&](int buf, auto FIRST) {
-    constexpr bool first = decltype(FIRST)::value;
-    const unsigned char* Ah = smem[buf];
-    const unsigned char* Al = smem[buf] + TA;
-    const unsigned char* Bc = smem[buf] + 2 * TA;
-#pragma unroll
-    for (int kk = 0; kk < BK / 16; ++kk) {
-      const int c = kk * 2 + half;
-      bf16x8 ah[TM], al[TM], bc[TN];
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        ah[i] = *reinterpret_cast<const bf16x8*>(Ah + swz32<BK>(wm * WM + i * 32 + r32, c));
-        if constexpr (XLO) al[i] = *reinterpret_cast<const bf16x8*>(Al + swz32<BK>(wm * WM + i * 32 + r32, c));
-      }
-#pragma unroll
-      for (int j = 0; j < TN; ++j) bc[j] = *reinterpret_cast<const bf16x8*>(Bc + swz32<BK>(wn * WN + j * 32 + r32, c));
-#pragma unroll
-      for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j) {
-          if (first && kk == 0) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bc[j], ah[i], f32x16{}, 0, 0, 0);
-          else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bc[j], ah[i], acc[i][j], 0, 0, 0);
-        }
-      if constexpr (XLO) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bc[j], al[i], acc[i][j], 0, 0, 0);
-      }
-    }
-  };
-  // y += s * acc + b * X for the group closed by buffer buf's step.  Element v of acc[i][j]:
-  // activation row wm WM + 32 i + r32, weight row wn WN + 32 j + 8 (v >> 2) + 4 half + (v & 3).
-  auto fold = [&](int buf, int grp) {
-    const float* sb = reinterpret_cast<const float*>(smem[buf] + OFF_SB);
-    const float* xs = reinterpret_cast<const float*>(smem[buf] + OFF_X);
-    float xg[TM];
-    if constexpr (!BMF) {
-#pragma unroll
-      for (int i = 0; i < TM; ++i) xg[i] = xs[wm * WM + i * 32 + r32];
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const int n0 = wn * WN + j * 32 + 8 * t + 4 * half;
-        const f32x4 p0 = *reinterpret_cast<const f32x4*>(sb + 2 * n0);
-        const f32x4 p1 = *reinterpret_cast<const f32x4*>(sb + 2 * n0 + 4);
-        const float sv[4] = {p0[0], p0[2], p1[0], p1[2]}, zv[4] = {p0[1], p0[3], p1[1], p1[3]};
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            if constexpr (BMF) yv[i][j][4 * t + u] = fmaf(sv[u], acc[i][j][4 * t + u], yv[i][j][4 * t + u]);
-            else yv[i][j][4 * t + u] = fmaf(sv[u], acc[i][j][4 * t + u], fmaf(zv[u], xg[i], yv[i][j][4 * t + u]));
-          }
-      }
-    if constexpr (BMF) {
-      if ((grp & 15) == 15) {  // the 16-group batch is complete: y += b . X on the matrix cores
-        const unsigned char* bt = btab;
-        const unsigned char* xh = btab + BT;
-        const unsigned char* xl = btab + BT + XT_;
-        bf16x8 bf[TN];
-#pragma unroll
-        for (int j = 0; j < TN; ++j) bf[j] = *reinterpret_cast<const bf16x8*>(bt + (wn * WN + j * 32 + r32) * 32 + half * 16);
-#pragma unroll
-        for (int i = 0; i < TM; ++i) {
-          const int rr = (wm * WM + i * 32 + r32) * 32 + half * 16;
-          const bf16x8 ah = *reinterpret_cast<const bf16x8*>(xh + rr);
-          const bf16x8 al = *reinterpret_cast<const bf16x8*>(xl + rr);
-#pragma unroll
-          for (int j = 0; j < TN; ++j) {
-            yv[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[j], ah, yv[i][j], 0, 0, 0);
-            yv[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[j], al, yv[i][j], 0, 0, 0);
-          }
-        }
-      }
-    }
-  };
-  // One group: GSTEP steps, loads two steps ahead (clamped to the last step past the end).
-  auto body = [&](int kt, auto SLOT, auto NSLOT, auto POS) {
-    constexpr int pos = decltype(POS)::value;
-    load_global(kt + 2 < ksteps ? kt + 2 : ksteps - 1, SLOT);
-    mfma_step(kt & 1, std::integral_constant<bool, pos == 0>{});
-    if constexpr (pos == GSTEP - 1) fold(kt & 1, kt / GSTEP);
-    store_lds((kt + 1) & 1, NSLOT, std::integral_constant<int, (pos + 1) % GSTEP>{}, (kt + 1) / GSTEP);
-    __syncthreads();
-  };
-  load_global(0, S0{});
-  load_global(ksteps > 1 ? 1 : 0, S1{});
-  store_lds(0, S0{}, std::integral_constant<int, 0>{}, 0);
-  __syncthreads();
-  for (int kt = 0; kt < ksteps; kt += GSTEP) {
-    body(kt, S0{}, S1{}, std::integral_constant<int, 0>{});
-    body(kt + 1, S1{}, S0{}, std::integral_constant<int, 1>{});
-    if constexpr (GSTEP == 4) {
-      body(kt + 2, S0{}, S1{}, std::integral_constant<int, 2>{});
-      body(kt + 3, S1{}, S0{}, std::integral_constant<int, 3>{});
-    }
-  }
-
-  // Epilogue as in qmm_f32_kernel: y + bias in f32, then the activation in f32.
-  const bool vec_ok = (N % 4) == 0;
-  [[maybe_unused]] float bcol[TN][16];
-  if constexpr (EPI) {
-#pragma unroll
-    for (int j = 0; j < TN; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int64_t n = bn0 + wn * WN + j * 32 + 8 * (v >> 2) + 4 * half + (v & 3);
-        const int64_t nc = n < N ? n : N - 1;  // columns past N are never stored
-        bcol[j][v] = epi.bias == nullptr ? -0.0f
-                     : epi.bias_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(epi.bias)[nc])
-                                     : static_cast<const float*>(epi.bias)[nc];
-      }
-  }
-  auto store = [&](auto A) {
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-      const int64_t m = bm0 + wm * WM + i * 32 + r32;
-      if (m >= M) continue;
-      float* yrow = y + m * N;
-#pragma unroll
-      for (int j = 0; j < TN; ++j) {
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int64_t n = bn0 + wn * WN + j * 32 + 8 * a + 4 * half;
-          f32x4 v;
-#pragma unroll
-          for (int b = 0; b < 4; ++b) v[b] = f32_finish<EPI, decltype(A)::value>(yv[i][j][4 * a + b], EPI ? bcol[j][4 * a + b] : 0.0f);
-          if (vec_ok && n + 3 < N) {
-            *reinterpret_cast<f32x4*>(yrow + n) = v;
-          } else {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-              if (n + b < N) yrow[n + b] = v[b];
-          }
-        }
-      }
-    }
-  };
-  f32_store_dispatch<EPI>(epi.act, store);
-}
-
 template <typename XT, typename SB, int BITS, int GS>
 static int launch_qmm_f32(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                           const void* b, int64_t N, void* y, const F32Epilogue& epi, hipStream_t st) {
@@ -785,29 +445,6 @@ static int launch_qmm_f32(const void* x, int64_t M, int64_t K, const uint32_t* w
   const int64_t tiles = ((M + kF32BM - 1) / kF32BM) * ((N + BN - 1) / BN);
   if (tiles == 0) return MLXQ_OK;
   if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "qmm_f32: problem too large");
-  if constexpr (GS >= 64) {  // the factored form (codes as the weight operand)
-    const bool epi_on = epi.bias || epi.act != MLXQ_ACT_NONE;
-    const bool bmf = std::is_same<SB, uint16_t>::value && (K / GS) % 16 == 0;
-    // 8 waves on 128 x 256 tiles, as the three-pass kernel.  4 waves on 128 x 128 (two workgroups
-    // per CU, so the two waves of a SIMD fold at different times) measured slower on the FLUX
-    // shapes (same box: up 0.850 -> 0.926 ms, down 0.948 -> 1.020 ms).
-    constexpr int CW = 8, CBN = 256;
-    const int64_t ctiles = ((M + kF32BM - 1) / kF32BM) * ((N + CBN - 1) / CBN);
-#define MLXQ_F32C(E, B)                                                                                 \
-  hipLaunchKernelGGL((qmm_f32c_kernel<XT, SB, BITS, GS, E, B, CW, CBN>), dim3((unsigned)ctiles), dim3(CW * 64), 0, st, \
-                     (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N, (float*)y, epi)
-    if constexpr (std::is_same<SB, uint16_t>::value) {
-      if (bmf) {
-        if (epi_on) MLXQ_F32C(true, true);
-        else MLXQ_F32C(false, true);
-        return check_launch("qmm_f32");
-      }
-    }
-    if (epi_on) MLXQ_F32C(true, false);
-    else MLXQ_F32C(false, false);
-#undef MLXQ_F32C
-    return check_launch("qmm_f32");
-  }
   if (epi.bias || epi.act != MLXQ_ACT_NONE)
     hipLaunchKernelGGL((qmm_f32_kernel<XT, SB, BITS, GS, WAVES, BN, BK, true>), dim3((unsigned)tiles),
                        dim3(WAVES * 64), 0, st, (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N,
@@ -835,6 +472,9 @@ int run_qmm_f32(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t
                 const F32Epilogue& epi) {
   if (x_dtype == MLXQ_BFLOAT16 && sb_dtype == MLXQ_BFLOAT16)
     return set_error(MLXQ_EINVAL, "qmm_f32: bf16 operands take the bf16 GEMM");
+  if (qmm_f32_strip_fits(K, N))
+    return run_qmm_f32_strip(x, x_dtype, M, K, wq, s, b, sb_dtype, N, gs, bits, y, epi, st);
+  if (epi.R > 0) return set_error(MLXQ_EINVAL, "qmm_f32: the three-pass kernel fuses no LoRA residual");
   if (x_dtype == MLXQ_FLOAT32) {
     if (sb_dtype == MLXQ_BFLOAT16)
       return qmm_f32_bits_gs<float, uint16_t>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);

@@ -1,0 +1,600 @@
+// qmm_f32_strip.hip — the large-M quantized GEMM in f32 (y[M,N] = x[M,K] . W^T, K % 64 == 0) for the
+// operand mixes MLX computes in f32: fp16 or f32 activations, and bf16 ones against f32 scales.
+//
+// Since
+//     x . w = sum_g ( s_g * sum_{k in g} x_k c_k  +  b_g * X_g ),   X_g = sum_{k in g} x_k,
+// the codes c (integers below 256, exact in bf16 and fp16) are one MFMA operand and the activations
+// the other, with no dequantization: fp16 and bf16 activations as they are (one pass, every product
+// exact), f32 ones as two bf16 values whose sum holds them to 16 significant bits (two passes,
+// v_hi = bf16(v), v_lo = bf16(v - v_hi)).  Each group's product accumulates in `acc`, whose first
+// MFMA starts from zero, and is folded into the running sum by one FMA per output, y += s_g * acc.
+// The bias term runs on the f32 matrix cores, two groups per MFMA, between the two groups' folds.
+// s_g * acc and b_g * X_g are large and of opposite sign, so how many groups have only one of them in
+// the running sum sets the error: [4096, 1280] fp16 x Q4 was 2.1e-7 off the 64-bit product with 16
+// groups per bf16 MFMA (X in three bf16 terms), 1.7e-7 with four, 1.6e-7 with two after both folds,
+// and is 1.4e-7 in this form, as with two FMAs per output and group.
+//
+// Workgroup: 8 waves, tile BM (128 or 64) x 256, K advanced 64 per step; wave w owns columns
+// [32 w, 32 w + 32) of all BM rows.  What bounds it is the LDS port: a wave reads 1 KB of activations
+// per MFMA (32 cycles of one SIMD's matrix core; four SIMDs against 128 bytes per cycle).  Hence the
+// weights never pass through LDS: a lane loads its own column's packed words two steps ahead and
+// converts them straight into its MFMA operand, each code once per workgroup, and with the codes
+// as the MFMA's B side a lane holds 16 rows of ONE column, so the fold's scale is a single register.
+// fp16 and bf16 activations go global -> LDS by direct-to-LDS loads three steps ahead into a 4-stage
+// ring; f32 ones through registers, where they are split and summed, one step ahead.
+// The fold of a group is interleaved with the next group's first MFMAs block by block, so the vector
+// work of one block runs under the MFMAs of the others.
+//
+// Same-process A/B against the kernel it replaces (128 x 256 tiles of 64 x 64 per wave, codes and
+// split activations through LDS, fp16 split into two bf16 passes; LoRA in a launch of its own):
+// [4096, 1280] fp16 x Q4 [10240, 1280]^T with bias 281 -> 154 us; [77, 1280] fp16 x Q8 [5120, 1280]^T
+// with bias and GELU 50.5 -> 21.0; [4608, 3072] f32 x Q4 [12288, 3072]^T with bias, rank-32 LoRA and
+// GELU 1043 -> 795.
+//
+// All buffer resources start at the tile's own first row, so 32-bit offsets reach any operand, and
+// rows past M or N read as zero.
+#include <type_traits>
+
+#include "mlxq_common.h"
+
+namespace mlxq {
+
+namespace {
+
+constexpr int kStripBN = 256;
+constexpr int kStripGroupM = 8;  // M-tiles per group of the tile order
+constexpr int kStripFlags = 0x00020000;  // raw buffer resource word 3 for gfx9-family loads
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// Consecutive workgroup ids are spread over the 8 XCDs, so each XCD is given a contiguous slice of
+// an order that walks groups of 8 M-tiles by all N-tiles, M fastest: the workgroups in flight on
+// an XCD share weight and activation panels in its L2.
+__device__ __forceinline__ void strip_coords(int64_t bid, int64_t tiles_m, int64_t tiles_n, int64_t& tm, int64_t& tn) {
+  const int64_t T = tiles_m * tiles_n, per = T / 8;
+  const int64_t L = bid < per * 8 ? (bid % 8) * per + bid / 8 : bid;
+  const int64_t span = kStripGroupM * tiles_n;
+  const int64_t g = L / span, gm0 = g * kStripGroupM;
+  const int64_t gsz = tiles_m - gm0 < kStripGroupM ? tiles_m - gm0 : kStripGroupM;
+  const int64_t idx = L - g * span;
+  tm = gm0 + idx % gsz;
+  tn = idx / gsz;
+}
+
+// Workgroup barrier that waits for this wave's LDS operations only (a release fence would also wait
+// for every direct-to-LDS load in flight; the loop waits for exactly those it needs).
+__device__ __forceinline__ void strip_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(15 | (7 << 4) | (0 << 8) | (3 << 14));  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+// A copy the compiler cannot elide: the word taken from a ring register must not share the register
+// the next load in flight writes.
+__device__ __forceinline__ uint32_t take(uint32_t v) {
+  uint32_t r;
+  asm volatile("v_mov_b32 %0, %1" : "=v"(r) : "v"(v));
+  return r;
+}
+
+// Eight codes as exact fp16 or bf16 values in code order: word kk of w (Q4), words 2kk, 2kk+1 (Q8).
+// Q4: the nibbles become bytes in code order, and a byte c <= 15 read as OCP fp8 E4M3 is c * 2^-9, so
+// one scaled convert makes two exact values (9 VALU ops).  Q8 to fp16: bytes under 0x64 are 1024 + c.
+template <int BITS, bool F16>
+__device__ __forceinline__ u32x4 codes8(const uint32_t* w, int kk) {
+  u32x4 o;
+  if constexpr (BITS == 4) {
+    const uint32_t v = w[kk], ev = v & 0x0f0f0f0fu, od = (v >> 4) & 0x0f0f0f0fu;
+    const uint32_t n0 = __builtin_amdgcn_perm(od, ev, 0x05010400u), n1 = __builtin_amdgcn_perm(od, ev, 0x07030602u);
+    if constexpr (F16) {
+      o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(n0, 512.0f, false));
+      o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(n0, 512.0f, true));
+      o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(n1, 512.0f, false));
+      o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(n1, 512.0f, true));
+    } else {
+      o[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n0, 512.0f, false));
+      o[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n0, 512.0f, true));
+      o[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n1, 512.0f, false));
+      o[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(n1, 512.0f, true));
+    }
+  } else {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const uint32_t v = w[2 * kk + h];
+      if constexpr (F16) {
+        const f16x2 k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+        const f16x2 a = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u)) - k1024;
+        const f16x2 b = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u)) - k1024;
+        o[2 * h] = __builtin_bit_cast(uint32_t, a);
+        o[2 * h + 1] = __builtin_bit_cast(uint32_t, b);
+      } else {
+        o[2 * h] = pack_bf16x2(ubyte<0>(v), ubyte<1>(v));
+        o[2 * h + 1] = pack_bf16x2(ubyte<2>(v), ubyte<3>(v));
+      }
+    }
+  }
+  return o;
+}
+
+// sum + the low (0) or high (1) fp16 half of w, in one instruction.
+template <int H>
+__device__ __forceinline__ float add_f16(uint32_t w, float sum) {
+  if constexpr (H == 0) asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel_hi:[1,0,0]" : "+v"(sum) : "v"(w));
+  else asm("v_fma_mix_f32 %0, %1, 1.0, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(sum) : "v"(w));
+  return sum;
+}
+
+}  // namespace
+
+// XT: activation storage (float, _Float16, or uint16_t bf16 bits); SB: scale/bias storage.
+template <typename XT, typename SB, int BITS, int GS, int BM>
+__global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict__ x, int64_t M, int64_t K,
+                                                            const uint32_t* __restrict__ wq,
+                                                            const SB* __restrict__ scales,
+                                                            const SB* __restrict__ biases, int64_t N,
+                                                            float* __restrict__ y, F32Epilogue epi) {
+  constexpr bool F16 = std::is_same<XT, _Float16>::value;
+  constexpr bool XF32 = std::is_same<XT, float>::value;
+  constexpr bool SBF = std::is_same<SB, float>::value;
+  constexpr int P = XF32 ? 2 : 1;             // passes: activation parts in LDS
+  constexpr int TM = BM / 32;                 // 32-row blocks per wave
+  constexpr int PART = BM * 128;              // bytes of one part of one stage (BM rows of 64 values)
+  constexpr int STAGE = P * PART;
+  constexpr int GPB = 16;                     // groups per scale / bias table
+  constexpr int SPB = GPB * GS / 64;          // K steps per table
+  constexpr int SPP = SPB / 8;                // K steps per pair of groups
+  constexpr int STAGES = XF32 ? 3 : 4;        // activation ring
+  constexpr int A_LD = BM / 64;               // 8-value chunks per thread (f32), or direct-to-LDS rounds
+  constexpr int NW = GS == 32 ? 2 : BITS / 4; // weight loads per lane per step (8 or 16 bytes)
+  constexpr int OFF_X = STAGES * STAGE;       // [group % 8][BM rows] f32 sums
+  constexpr int OFF_S = OFF_X + 8 * BM * 4;
+  constexpr int SW = 32 * GPB * (int)sizeof(SB);  // per wave: [half][32 columns][8 groups] scales, then biases
+  __shared__ __attribute__((aligned(16))) unsigned char lds[OFF_S + 8 * 2 * SW];
+  auto stage_at = [&](int t) { return lds + (XF32 ? t % 3 : t & 3) * STAGE; };
+
+  const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + kStripBN - 1) / kStripBN;
+  int64_t tm, tn;
+  strip_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
+  const int64_t bm0 = tm * BM, bn0 = tn * kStripBN;
+  const int rows_m = (int)(M - bm0 < BM ? M - bm0 : BM), rows_n = (int)(N - bn0 < kStripBN ? N - bn0 : kStripBN);
+  const uint32_t kwords = (uint32_t)(K * BITS / 32);
+  const int groups = (int)(K / GS), T = (int)(K / 64);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<XT*>(x + bm0 * K), (short)0, (int)(uint32_t)(rows_m * K * (int64_t)sizeof(XT)), kStripFlags);
+  const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<uint32_t*>(wq + bn0 * kwords), (short)0, (int)(uint32_t)(rows_n * (int64_t)kwords * 4), kStripFlags);
+  const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<SB*>(scales + bn0 * groups), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups * (int64_t)sizeof(SB)), kStripFlags);
+  const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<SB*>(biases + bn0 * groups), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups * (int64_t)sizeof(SB)), kStripFlags);
+
+  // ---- activations.  16-byte chunk c (8 values) of row r sits at chunk c ^ swz_f(r) of its row.
+  // fp16 / bf16: round i of wave w fills rows 64 i + 8 w .. + 7, lane L the chunk that belongs at
+  // position L & 7 of row 64 i + 8 w + (L >> 3).  f32: thread t loads chunk t & 7 (32 bytes) of rows
+  // t / 8 + 64 i.
+  uint32_t x_off[A_LD];
+#pragma unroll
+  for (int i = 0; i < A_LD; ++i) {
+    if constexpr (XF32) {
+      x_off[i] = (uint32_t)(((tid >> 3) + 64 * i) * K * 4 + (tid & 7) * 32);
+    } else {
+      const int r = 64 * i + 8 * wave + (lane >> 3);
+      x_off[i] = (uint32_t)((r * K + ((lane & 7) ^ swz_f(r)) * 8) * 2);
+    }
+  }
+  auto dma_x = [&](int t) {  // !XF32
+#if defined(__HIP_DEVICE_COMPILE__)
+    unsigned char* const base = stage_at(t);
+    const uint32_t tc = (uint32_t)(t < T ? t : T - 1);
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(base + (64 * i + 8 * wave) * 128),
+                                               16, x_off[i] + tc * 128u, 0, 0, 0);
+#else
+    (void)t;
+#endif
+  };
+  u32x4 xr[XF32 ? A_LD : 1][2];
+  auto load_x = [&](int t) {  // XF32
+    const uint32_t tc = (uint32_t)(t < T ? t : T - 1);
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i)
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        xr[i][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, x_off[i] + tc * 256u + 16u * q, 0, 0));
+  };
+  float* const xtab = reinterpret_cast<float*>(lds + OFF_X);
+  float xrun[XF32 ? A_LD : 1];  // GS 128: a row's sum over its group's first step
+  // X of group g for tile row `row`; the lanes that share a row write the same value.
+  auto put_x = [&](int row, int g, float v) { xtab[(g & 7) * BM + row] = v; };
+  // f32: split step t's registers into its stage and leave the group sums.  POS: t's position in its
+  // 128-wide group.
+  auto stage_x = [&](int t, auto POS) {
+    unsigned char* const base = stage_at(t);
+#pragma unroll
+    for (int i = 0; i < A_LD; ++i) {
+      const int row = (tid >> 3) + 64 * i, c = tid & 7;
+      u32x4 hi, lo;
+      float sum = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const float v0 = __uint_as_float(xr[i][e >> 1][2 * (e & 1)]), v1 = __uint_as_float(xr[i][e >> 1][2 * (e & 1) + 1]);
+        sum += v0 + v1;
+        hi[e] = pack_bf16x2(v0, v1);
+        lo[e] = pack_bf16x2(v0 - __uint_as_float(hi[e] << 16), v1 - __uint_as_float(hi[e] & 0xffff0000u));
+      }
+      unsigned char* const p = base + row * 128 + ((c ^ swz_f(row)) << 4);
+      *reinterpret_cast<u32x4*>(p) = hi;
+      *reinterpret_cast<u32x4*>(p + PART) = lo;
+      // the row's 8 chunks sit in 8 consecutive lanes
+      sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xb1, 0xf, 0xf, true));
+      sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4e, 0xf, 0xf, true));
+      if constexpr (GS == 32) {
+        put_x(row, 2 * t + (c >> 2), sum);
+      } else {
+        sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x141, 0xf, 0xf, true));
+        if constexpr (GS == 64) {
+          put_x(row, t, sum);
+        } else if constexpr (decltype(POS)::value == 0) {
+          xrun[i] = sum;
+        } else {
+          put_x(row, t >> 1, xrun[i] + sum);
+        }
+      }
+    }
+  };
+  // fp16 / bf16: the group sums of step t from its landed stage, BM / 8 rows per wave, four lanes a row
+  // (two chunks each).
+  auto sum_x = [&](int t, auto POS) {
+    const int row = wave * (BM / 8) + ((lane >> 2) & (BM / 8 - 1)), q = lane & 3;
+    const unsigned char* const base = stage_at(t) + row * 128;
+    float part[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const u32x4 v = *reinterpret_cast<const u32x4*>(base + (((2 * q + h) ^ swz_f(row)) << 4));
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        if constexpr (F16) {
+          part[0] = add_f16<0>(v[e], part[0]);
+          part[1] = add_f16<1>(v[e], part[1]);
+        } else {
+          part[0] += __uint_as_float(v[e] << 16);
+          part[1] += __uint_as_float(v[e] & 0xffff0000u);
+        }
+      }
+    }
+    // Every lane of a row ends with the same sum and writes it: no branch.
+    float sum = part[0] + part[1];
+    sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xb1, 0xf, 0xf, true));
+    if constexpr (GS == 32) {
+      put_x(row, 2 * t + (q >> 1), sum);
+    } else {
+      sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4e, 0xf, 0xf, true));
+      if constexpr (GS == 64) put_x(row, t, sum);
+      else if constexpr (decltype(POS)::value == 0) xrun[0] = sum;
+      else put_x(row, t >> 1, xrun[0] + sum);
+    }
+  };
+
+  // ---- weights: column n = 32 w + r32 of the tile.  Lane half h covers, for MFMA kk of a step, 16-byte
+  // chunk 4 h + kk of k (group 64 and 128), or 4 (kk >> 1) + 2 h + (kk & 1) (group 32, so that MFMAs 0, 1
+  // and 2, 3 stay inside one group): its packed words are contiguous, one or two loads.
+  const uint32_t ncol = (uint32_t)(32 * wave + r32);
+  const uint32_t w_off = (ncol * kwords + (uint32_t)half * (GS == 32 ? BITS / 2 : BITS)) * 4u;
+  auto chunk_of = [&](int kk) { return GS == 32 ? 4 * (kk >> 1) + 2 * half + (kk & 1) : 4 * half + kk; };
+  uint32_t wr[2][BITS], wc[BITS];
+  auto load_w = [&](int t, auto SLOT) {
+    constexpr int sl = decltype(SLOT)::value;
+    const uint32_t at = w_off + (uint32_t)(t < T ? t : T - 1) * (8u * BITS);
+    constexpr int EACH = BITS / NW;  // words per load
+#pragma unroll
+    for (int q = 0; q < NW; ++q) {
+      const uint32_t o = at + (GS == 32 ? 4u * BITS * q : 16u * q);
+      if constexpr (EACH == 2) {
+        const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 2; ++e) wr[sl][2 * q + e] = v[e];
+      } else {
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wr[sl][4 * q + e] = v[e];
+      }
+    }
+  };
+  auto take_w = [&](auto SLOT) {
+    constexpr int sl = decltype(SLOT)::value;
+#pragma unroll
+    for (int e = 0; e < BITS; ++e) wc[e] = take(wr[sl][e]);
+  };
+
+  // ---- scales and biases, 16 groups at a time: lane (h, r32) loads groups 16 b + 8 h .. + 7 of its
+  // column into the wave's LDS tables, from which each group's scale and bias are read back.  Groups past the last are zero.
+  struct Batch { uint32_t s[SBF ? 8 : 4], z[SBF ? 8 : 4]; };
+  auto load_batch = [&](int b, Batch& d) {
+    const int g0 = 16 * b + 8 * half;
+    const uint32_t at = (ncol * (uint32_t)groups + (uint32_t)g0) * (uint32_t)sizeof(SB);
+    if (16 * b + 16 <= groups && (SBF || (groups & 1) == 0)) {  // whole and dword-aligned
+#pragma unroll
+      for (int q = 0; q < (SBF ? 2 : 1); ++q) {
+        const u32x4 s = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, at + 16u * q, 0, 0));
+        const u32x4 z = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rz, at + 16u * q, 0, 0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          d.s[4 * q + e] = s[e];
+          d.z[4 * q + e] = z[e];
+        }
+      }
+    } else {
+      uint32_t s[8], z[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t idx = g0 + e < groups ? ncol * (uint32_t)groups + (uint32_t)(g0 + e) : 0xffffffffu / (uint32_t)sizeof(SB);
+        s[e] = load_sb_bits<SB>(rs, idx);  // past the resource: zero
+        z[e] = load_sb_bits<SB>(rz, idx);
+      }
+#pragma unroll
+      for (int e = 0; e < (SBF ? 8 : 4); ++e) {
+        d.s[e] = SBF ? s[e] : (s[2 * e] & 0xffffu) | (s[2 * e + 1] << 16);
+        d.z[e] = SBF ? z[e] : (z[2 * e] & 0xffffu) | (z[2 * e + 1] << 16);
+      }
+    }
+  };
+  unsigned char* const stab = lds + OFF_S + wave * 2 * SW;
+  auto put_tables = [&](const Batch& d) {
+    unsigned char* const p = stab + half * (SW / 2) + r32 * (8 * (int)sizeof(SB));
+#pragma unroll
+    for (int q = 0; q < (SBF ? 2 : 1); ++q) {
+      *reinterpret_cast<u32x4*>(p + 16 * q) = u32x4{d.s[4 * q], d.s[4 * q + 1], d.s[4 * q + 2], d.s[4 * q + 3]};
+      *reinterpret_cast<u32x4*>(p + SW + 16 * q) = u32x4{d.z[4 * q], d.z[4 * q + 1], d.z[4 * q + 2], d.z[4 * q + 3]};
+    }
+  };
+  auto scale_of = [&](int g) {
+    return SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + ((g >> 3) & 1) * (SW / 2)) + r32 * 8, g & 7);
+  };
+
+  f32x16 acc[TM], yv[TM];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      acc[i][v] = 0.0f;
+      yv[i][v] = 0.0f;
+    }
+  // y += b . X over the groups 2 p and 2 p + 1; this half's operands are those of group 2 p + half.
+  auto bias_pair = [&](int p) {
+    const int g = 2 * p + half;
+    const float z = SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + SW + ((p >> 2) & 1) * (SW / 2)) + r32 * 8, 2 * (p & 3) + half);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      const float xg = xtab[(g & 7) * BM + 32 * i + r32];
+      yv[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(g < groups ? xg : 0.0f, z, yv[i], 0, 0, 0);
+    }
+  };
+
+  // ---- the loop.  Sub-step u = kk * P + part of a step multiplies fragments of one activation part
+  // by the codes of MFMA kk; its fragments were read one sub-step earlier.
+  constexpr int NSUB = 4 * P;
+  u32x4 af[2][TM], cf[2];
+  int a_off[4];
+#pragma unroll
+  for (int kk = 0; kk < 4; ++kk) a_off[kk] = r32 * 128 + ((chunk_of(kk) ^ swz_f(r32)) << 4);
+  auto read_a = [&](int slot, const unsigned char* base, int u) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+      af[slot][i] = *reinterpret_cast<const u32x4*>(base + (u % P) * PART + i * 4096 + a_off[u / P]);
+  };
+  float s_prev = 0.0f, s_next[2] = {0.0f, 0.0f};
+  auto mfma = [&](const u32x4& a, const u32x4& c, const f32x16& d) {
+    if constexpr (F16)
+      return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, c), d, 0, 0, 0);
+    else
+      return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, c), d, 0, 0, 0);
+  };
+  // Sub-step U (position POS of the step in a 128-wide group): a group's first sub-step folds the
+  // group before, block by block, and starts its own sums from zero.
+  auto sub = [&](auto U, auto POS) {
+    constexpr int u = decltype(U)::value, kk = u / P;
+    constexpr bool start = u % P == 0 && (GS == 32 ? kk % 2 == 0 : GS == 64 ? kk == 0 : kk == 0 && decltype(POS)::value == 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      if constexpr (start) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) yv[i][v] = fmaf(s_prev, acc[i][v], yv[i][v]);
+        // Pinned here (else the folds sink to where y is next read), and vector and matrix instructions
+        // stay on their side, so a block's old sums die before its new ones are born.
+        asm volatile("" : "+v"(yv[i]));
+        __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80);
+        acc[i] = mfma(af[u & 1][i], cf[kk & 1], f32x16{});
+      } else {
+        acc[i] = mfma(af[u & 1][i], cf[kk & 1], acc[i]);
+      }
+    }
+    if constexpr (start) s_prev = s_next[GS == 32 ? kk / 2 : 0];
+  };
+  using I0 = std::integral_constant<int, 0>;
+  using I1 = std::integral_constant<int, 1>;
+  Batch nb;
+  // Step t: before its middle barrier the first half of its sub-steps, and (f32) the staging of step
+  // t + 1; after it the loads of later steps, the rest, and the first fragments of step t + 1.
+  auto step = [&](int t, auto PAR) __attribute__((always_inline)) {
+    using NPAR = std::integral_constant<int, 1 - decltype(PAR)::value>;
+    const unsigned char* const As = stage_at(t);
+    const unsigned char* const An = stage_at(t + 1);
+    if constexpr (GS == 32) {
+      s_next[0] = scale_of(2 * t);
+      s_next[1] = scale_of(2 * t + 1);
+    } else if constexpr (GS == 64 || decltype(PAR)::value == 0) {
+      s_next[0] = scale_of(GS == 64 ? t : t >> 1);
+    }
+    if constexpr (XF32) stage_x(t + 1, NPAR{});
+    auto half1 = [&](auto U) {
+      constexpr int u = decltype(U)::value;
+      read_a((u + 1) & 1, As, u + 1);
+      if constexpr ((u + 1) % P == 0) cf[((u + 1) / P) & 1] = codes8<BITS, F16>(wc, (u + 1) / P);
+      sub(U, PAR);
+    };
+    half1(std::integral_constant<int, 0>{});
+    half1(std::integral_constant<int, 1>{});
+    if constexpr (P == 2) {
+      half1(std::integral_constant<int, 2>{});
+      half1(std::integral_constant<int, 3>{});
+    }
+    // x(t + 1) was issued in step t - 2, whatever its order against w(t + 1); x(t + 2) and w(t + 2) in
+    // step t - 1.
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (!XF32) mlxq_vmcnt<NW + A_LD>();
+    strip_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XF32) load_x(t + 2);
+    else dma_x(t + 3);
+    half1(std::integral_constant<int, 2 * P>{});
+    if constexpr (P == 2) half1(std::integral_constant<int, 5>{});
+    if constexpr (P == 2) half1(std::integral_constant<int, 6>{});
+    if constexpr (!XF32) sum_x(t + 1, NPAR{});
+    take_w(NPAR{});
+    load_w(t + 3, NPAR{});
+    read_a(0, An, 0);
+    cf[0] = codes8<BITS, F16>(wc, 0);
+    sub(std::integral_constant<int, NSUB - 1>{}, PAR);
+    __builtin_amdgcn_sched_barrier(0);
+    // A pair of groups ends with this step: their X sums were left during the step before, so all are
+    // visible since the barrier, and the second group is folded in the step after.
+    if (SPP == 1 || decltype(PAR)::value == 1) {
+      if ((t + 1) % SPP == 0) bias_pair(t / SPP);
+      if ((t + 1) % SPB == 0) {
+        put_tables(nb);
+        load_batch((t + 1) / SPB + 1, nb);
+      }
+    }
+  };
+
+  // ---- prologue: batch 0's scales, x and w of the first steps (issued x(0) w(0) x(1) w(1) x(2) w(2)).
+  load_batch(0, nb);
+  if constexpr (XF32) load_x(0);
+  else dma_x(0);
+  load_w(0, I0{});
+  if constexpr (!XF32) dma_x(1);
+  load_w(1, I1{});
+  if constexpr (!XF32) dma_x(2);
+  put_tables(nb);
+  if constexpr (XF32) {
+    stage_x(0, I0{});
+    load_x(1);
+  }
+  take_w(I0{});
+  load_batch(1, nb);
+  load_w(2, I0{});
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (!XF32) mlxq_vmcnt<NW + 2 * A_LD>();  // x(0) is older than w(1), x(1), x(2) and w(2)
+  strip_barrier();
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (!XF32) sum_x(0, I0{});
+  read_a(0, lds, 0);
+  cf[0] = codes8<BITS, F16>(wc, 0);
+  int t = 0;
+  for (; t + 1 < T; t += 2) {
+    step(t, I0{});
+    step(t + 1, I1{});
+  }
+  if (t < T) step(t, I0{});
+  // The last pair's bias term when its second group does not exist, and the last group's fold.
+  if (T % SPP != 0) bias_pair((T - 1) / SPP);
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) yv[i][v] = fmaf(s_prev, acc[i][v], yv[i][v]);
+  mlxq_vmcnt<0>();  // no direct-to-LDS load outlives the workgroup
+
+  // ---- epilogue: lane holds column n and rows m = 32 i + 8 (v >> 2) + 4 half + (v & 3): y + bias in
+  // f32, the LoRA residual (xa . lbt^T on the f32 matrix cores) times its scale, the activation.
+  const bool n_ok = (int)ncol < rows_n;
+  const int64_t n = bn0 + (n_ok ? (int)ncol : 0);
+  const float bv = epi.bias == nullptr ? -0.0f
+                   : epi.bias_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(epi.bias)[n])
+                                   : static_cast<const float*>(epi.bias)[n];
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
+      y + bm0 * N, (short)0, (int)(uint32_t)(rows_m * N * 4), kStripFlags);
+  auto finish = [&](auto ACT) {
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+      f32x16 o;
+#pragma unroll
+      for (int v = 0; v < 16; ++v) o[v] = yv[i][v] + bv;
+      if (epi.R > 0) {
+        f32x16 r = {};
+        const int mr = 32 * i + r32 < rows_m ? 32 * i + r32 : rows_m - 1;
+        for (int k = 0; k < epi.R; k += 16) {
+          const f32x4* const xp = reinterpret_cast<const f32x4*>(epi.xa + (bm0 + mr) * epi.R + k + 8 * half);
+          const f32x4* const lp = reinterpret_cast<const f32x4*>(epi.lbt + n * epi.R + k + 8 * half);
+          const f32x4 x0 = xp[0], x1 = xp[1], l0 = lp[0], l1 = lp[1];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            r = __builtin_amdgcn_mfma_f32_32x32x2f32(x0[e], l0[e], r, 0, 0, 0);
+            r = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[e], l1[e], r, 0, 0, 0);
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[v] += r[v] * epi.lora_scale;
+      }
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        float ov = o[v];
+        if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_EXACT) ov = gelu_erf(ov);
+        else if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_TANH) ov = gelu_tanh<false>(ov);
+        const int row = 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
+        const uint32_t at = n_ok ? (uint32_t)(row * N + n) * 4u : 0xfffffffcu;  // rows past M fall past the resource
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ov), ry, at, 0, 0);
+      }
+    }
+  };
+  if (epi.act == MLXQ_ACT_GELU || epi.act == MLXQ_ACT_GELU_EXACT) finish(std::integral_constant<int, MLXQ_ACT_GELU_EXACT>{});
+  else if (epi.act == MLXQ_ACT_GELU_TANH) finish(std::integral_constant<int, MLXQ_ACT_GELU_TANH>{});
+  else finish(std::integral_constant<int, MLXQ_ACT_NONE>{});
+}
+
+template <typename XT, typename SB, int BITS, int GS, int BM>
+static int launch_strip(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
+                        int64_t N, void* y, const F32Epilogue& epi, hipStream_t st) {
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + kStripBN - 1) / kStripBN);
+  if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "qmm_f32: problem too large");
+  hipLaunchKernelGGL((qmm_f32_strip_kernel<XT, SB, BITS, GS, BM>), dim3((unsigned)tiles), dim3(512), 0, st, (const XT*)x,
+                     M, K, wq, (const SB*)s, (const SB*)b, N, (float*)y, epi);
+  return check_launch("qmm_f32");
+}
+
+template <typename XT, typename SB>
+static int strip_bits_gs(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
+                         int64_t N, int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st) {
+  const bool big = ((M + 127) / 128) * ((N + kStripBN - 1) / kStripBN) >= device_cu_count() * 3 / 4;
+#define MLXQ_ST(B, G)                                                                             \
+  if (bits == B && gs == G)                                                                       \
+    return big ? launch_strip<XT, SB, B, G, 128>(x, M, K, wq, s, b, N, y, epi, st)                \
+               : launch_strip<XT, SB, B, G, 64>(x, M, K, wq, s, b, N, y, epi, st);
+  MLXQ_ST(4, 32) MLXQ_ST(4, 64) MLXQ_ST(4, 128) MLXQ_ST(8, 32) MLXQ_ST(8, 64) MLXQ_ST(8, 128)
+#undef MLXQ_ST
+  return set_error(MLXQ_EINVAL, "qmm_f32: unsupported bits=%d group_size=%d", bits, gs);
+}
+
+// Whether a tile's rows fit 32-bit byte offsets (operands of any number of rows do).
+bool qmm_f32_strip_fits(int64_t K, int64_t N) { return K % 64 == 0 && K < (1LL << 22) && N < (1LL << 22); }
+
+int run_qmm_f32_strip(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
+                      const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, const F32Epilogue& epi,
+                      hipStream_t st) {
+  if (M == 0 || N == 0) return MLXQ_OK;
+  if (x_dtype == MLXQ_FLOAT32) {
+    if (sb_dtype == MLXQ_BFLOAT16) return strip_bits_gs<float, uint16_t>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+    return strip_bits_gs<float, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+  }
+  if (x_dtype == MLXQ_FLOAT16) {
+    if (sb_dtype == MLXQ_BFLOAT16) return strip_bits_gs<_Float16, uint16_t>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+    return strip_bits_gs<_Float16, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+  }
+  return strip_bits_gs<uint16_t, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+}
+
+}  // namespace mlxq
