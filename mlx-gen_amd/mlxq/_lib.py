@@ -137,6 +137,24 @@ def load():
     return lib
 
 
+_fast = None
+
+
+def fast():
+    """The native call path of the operators (_fast.so, host/fast.cpp): each function returns None for
+    a call whose operands need preparation or that failed, and the caller takes its general path."""
+    global _fast
+    if _fast is None:
+        load()
+        try:
+            from . import _fast as module
+        except ImportError as e:
+            raise ImportError(f"mlxq._fast is missing or does not load ({e}): build it with "
+                              "`make -C mlx-gen_amd/csrc` (or __graft_entry__.build())") from e
+        _fast = module
+    return _fast
+
+
 def check(status: int) -> None:
     if status != MLXQ_OK:
         raise MlxqError(status, load().mlxq_last_error().decode())

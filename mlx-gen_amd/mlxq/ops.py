@@ -13,6 +13,8 @@ dtype; a matmul returns promote(x, scales) (bf16 only when both are bf16; fp16 a
 is f32); a bias add or a LoRA residual in f32 promotes the result to f32.  Every operand's shape and dtype is checked
 against x before anything is launched, as MLX's quantized_matmul checks them; failures raise
 ``MlxqError`` with status MLXQ_EINVAL, and library errors carry the library's status and message.
+The decode-sized calls go through the native module (_lib.fast) when their operands need no
+preparation; the code here is the general path and the one that reports errors.
 """
 from __future__ import annotations
 
@@ -229,6 +231,10 @@ def quantized_matmul(x, wq, scales, biases, transpose: bool = True,
                      group_size: int = DEFAULT_GROUP_SIZE, bits: int = 4, out=None):
     """y = x . dequantize(W)^T (transpose=True, the only form the reference uses), in
     promote(x, scales)."""
+    if transpose and out is None:
+        y = _lib.fast().quantized_matmul(x, wq, scales, biases, group_size, bits)
+        if y is not None:
+            return y
     return _mm("mlxq_quantized_matmul", x, wq, scales, biases, group_size, bits, transpose, out=out)
 
 
@@ -253,6 +259,10 @@ def embedding(ids, wq, scales, biases, group_size: int = DEFAULT_GROUP_SIZE, bit
     """TokenEmbedding::forward's quantized arm (src/nn.rs:42-58): gather the packed rows of ids
     (any shape, int32/int64), dequantize, cast to out_dtype (f32 like the reference).  Ids outside
     [0, vocab) give NaN rows."""
+    if out_dtype is torch.bfloat16 or out_dtype is torch.float32:
+        y = _lib.fast().embedding(ids, wq, scales, biases, group_size, bits, int(out_dtype is torch.bfloat16))
+        if y is not None:
+            return y
     if out_dtype not in (torch.bfloat16, torch.float32):
         raise TypeError(f"embedding: out_dtype must be bfloat16 or float32, got {out_dtype}")
     if bits not in (4, 8):
@@ -274,6 +284,10 @@ def swiglu(x, gate, up, group_size: int = DEFAULT_GROUP_SIZE, bits: int = 4, out
     """Fused decode SwiGLU h = silu(gate(x)) * up(x) (mlx-gen-sensenova/src/qwen3.rs:178-181), gate
     and up given as packed (wq, scales, biases) triples of shape [F, K].  Decode form only (bf16,
     M <= 8); other shapes raise MlxqError with status MLXQ_EUNSUPPORTED."""
+    if out is None:
+        h = _lib.fast().swiglu(x, gate, up, group_size, bits)
+        if h is not None:
+            return h
     _float_dtype("swiglu", "x", x)
     K = x.shape[-1]
     lead = x.shape[:-1]
@@ -386,6 +400,10 @@ def linear(x, wq, scales, biases, group_size: int = DEFAULT_GROUP_SIZE, bits: in
     """Quantized AdaptableLinear forward with optional bias, one LoRA adapter and an activation,
     rounded at the same points as the reference's separate ops.  bias and the LoRA factors keep
     their own dtypes; the result is in MLX's promoted dtype (linear_out_dtype)."""
+    if workspace is None:
+        y = _lib.fast().linear(x, wq, scales, biases, group_size, bits, bias, lora_a, lora_b, lora_scale, activation)
+        if y is not None:
+            return y
     _float_dtype("linear", "x", x)
     K = x.shape[-1]
     lead = x.shape[:-1]
