@@ -5,12 +5,12 @@
 // the epilogue's ops rounded to bf16 where the reference's separate ops round.
 //
 // When M x N gives few tiles, a tile kernel leaves most CUs idle and each workgroup walks all of
-// K one latency-bound step after another.  Here a workgroup of 8 waves owns a 64x64 output tile
-// and the waves split K: wave w takes K steps [w*KT/8, (w+1)*KT/8), so a tile has eight
-// independent load chains of KT/8 steps instead of one of KT.  Each wave moves its activation
+// K one latency-bound step after another.  Here a workgroup of 8 waves (4 when the
+// tiles outnumber the CUs) owns a 64x64 output tile and the waves split K: wave w of W takes K steps
+// [w*KT/W, (w+1)*KT/W), so a tile has W independent load chains of KT/W steps instead of one of KT.  Each wave moves its activation
 // rows global -> LDS with direct-to-LDS loads one step ahead (a private 2-stage ring, 8 rows x
 // 128 bytes per load, i.e. whole cache lines) and reads MFMA fragments back with ds_read_b128;
-// its weight fragments go straight into registers two steps ahead.  The eight partial tiles meet
+// its weight fragments go straight into registers two steps ahead.  The partial tiles meet
 // in LDS (over the rings) and are added in wave order (deterministic); waves 0-3 then finish one
 // 32x32 sub-tile each.
 // MFMA roles (as in qmm_wide.hip): weights are the A operand (rows n), activations the B operand
@@ -30,7 +30,6 @@ namespace mlxq {
 namespace {
 
 constexpr int kTile = 64;   // output tile rows and columns
-constexpr int kWaves = 8;   // waves per workgroup, splitting K
 constexpr int kBufferFlags = 0x00020000;
 
 template <typename SB, int BITS>
@@ -39,7 +38,7 @@ struct SmallOps {           // one K step of one lane's register operands
   uint32_t s[2], z[2];      // raw scale / bias bits of sub-tile j
 };
 
-template <typename SB, int BITS, int GS, int EPI, bool SZS>
+template <typename SB, int BITS, int GS, int EPI, bool SZS, int kWaves>
 __global__ __launch_bounds__(kWaves * 64, 1) void qmm_small_kernel(
     const uint16_t* __restrict__ x, int64_t M, int64_t K, const uint32_t* __restrict__ wq,
     const SB* __restrict__ scales, const SB* __restrict__ biases, int64_t N,
@@ -238,7 +237,7 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qmm_small_kernel(
   mlxq_vmcnt<0>();
   __builtin_amdgcn_sched_barrier(0);
 
-  // ---- reduction over the eight K slices, in wave order.
+  // ---- reduction over the K slices, in wave order.
 #pragma unroll
   for (int sub = 0; sub < 4; ++sub)
 #pragma unroll
@@ -329,10 +328,22 @@ static int launch_small(const void* x, int64_t M, int64_t K, const uint32_t* wq,
   if (kind >= 2 && epi.act_table == nullptr) return set_error(MLXQ_EINVAL, "qmm: activation table missing");
   // bf16 scales with whole blocks of 8 groups are staged in LDS (16-byte aligned row blocks).
   const bool szs = std::is_same<SB, uint16_t>::value && (K / GS) % 8 == 0;
-#define MLXQ_SL(E, Z)                                                                                 \
-  hipLaunchKernelGGL((qmm_small_kernel<SB, BITS, GS, E, Z>), dim3((unsigned)tiles), dim3(kWaves * 64), \
+  // Waves per tile.  Eight (144 KB of LDS, one workgroup per CU) while every tile has a CU of its own;
+  // past that the surplus tiles were a second round, so four (72 KB, two workgroups per CU): both
+  // tiles' loads, reductions and epilogues overlap.  Same-process A/B, 8 -> 4 waves, Q4 g64 unless
+  // stated: 333 x 3072 x 4096 (384 tiles) 27.8 -> 24.0 us, 256 x 3072 x 4608 (288) 26.7 -> 22.6,
+  // 320 x 4096 x 4096 Q8 (320) 40.0 -> 35.6, 200 x 2048 x 8192 g32 (512) 22.7 -> 19.7, 300 x 2880 x
+  // 5000 (395) 31.6 -> 29.5; with a tile per CU eight stay ahead (each walks half the K steps).
+  const bool four = tiles > device_cu_count();
+#define MLXQ_SLW(E, Z, W)                                                                             \
+  hipLaunchKernelGGL((qmm_small_kernel<SB, BITS, GS, E, Z, W>), dim3((unsigned)tiles), dim3(W * 64),  \
                      0, st, (const uint16_t*)x, M, K, wq, (const SB*)s, (const SB*)b, N,               \
                      (uint16_t*)y, epi)
+#define MLXQ_SL(E, Z)               \
+  do {                              \
+    if (four) MLXQ_SLW(E, Z, 4);    \
+    else MLXQ_SLW(E, Z, 8);         \
+  } while (0)
   if constexpr (std::is_same<SB, uint16_t>::value) {
     if (szs) {
       switch (kind) {
@@ -351,6 +362,7 @@ static int launch_small(const void* x, int64_t M, int64_t K, const uint32_t* wq,
     default: MLXQ_SL(3, false); break;
   }
 #undef MLXQ_SL
+#undef MLXQ_SLW
   return check_launch("qmm_small");
 }
 
