@@ -1,4 +1,4 @@
-// qmm_f32_strip.hip — the large-M quantized GEMM in f32 (y[M,N] = x[M,K] . W^T, K % 64 == 0) for the
+// qmm_f32_strip.h — the large-M quantized GEMM in f32 (y[M,N] = x[M,K] . W^T, K % 64 == 0) for the
 // operand mixes MLX computes in f32: fp16 or f32 activations, and bf16 ones against f32 scales.
 //
 // Since
@@ -15,7 +15,9 @@
 // and is 1.4e-7 in this form, as with two FMAs per output and group.
 //
 // Workgroup: 8 waves, tile BM (128 or 64) x 256, K advanced 64 per step; wave w owns columns
-// [32 w, 32 w + 32) of all BM rows.  What bounds it is the LDS port: a wave reads 1 KB of activations
+// [32 w, 32 w + 32) of all BM rows.  Small grids (strip_shape) take KS = 2 or 4 K-groups of 8 / KS
+// waves instead: each group walks its own share of K, with its own activation ring, over the same
+// 256 / KS columns, and the partial sums meet in LDS at the end.  What bounds it is the LDS port: a wave reads 1 KB of activations
 // per MFMA (32 cycles of one SIMD's matrix core; four SIMDs against 128 bytes per cycle).  Hence the
 // weights never pass through LDS: a lane loads its own column's packed words two steps ahead and
 // converts them straight into its MFMA operand, each code once per workgroup, and with the codes
@@ -28,11 +30,13 @@
 // Same-process A/B against the kernel it replaces (128 x 256 tiles of 64 x 64 per wave, codes and
 // split activations through LDS, fp16 split into two bf16 passes; LoRA in a launch of its own):
 // [4096, 1280] fp16 x Q4 [10240, 1280]^T with bias 281 -> 154 us; [77, 1280] fp16 x Q8 [5120, 1280]^T
-// with bias and GELU 50.5 -> 21.0; [4608, 3072] f32 x Q4 [12288, 3072]^T with bias, rank-32 LoRA and
+// with bias and GELU 50.5 -> 8.7 (21.0 without K-groups); [4608, 3072] f32 x Q4 [12288, 3072]^T with bias, rank-32 LoRA and
 // GELU 1043 -> 795.
 //
 // All buffer resources start at the tile's own first row, so 32-bit offsets reach any operand, and
 // rows past M or N read as zero.
+#pragma once
+
 #include <type_traits>
 
 #include "mlxq_common.h"
@@ -41,7 +45,6 @@ namespace mlxq {
 
 namespace {
 
-constexpr int kStripBN = 256;
 constexpr int kStripGroupM = 8;  // M-tiles per group of the tile order
 constexpr int kStripFlags = 0x00020000;  // raw buffer resource word 3 for gfx9-family loads
 
@@ -129,7 +132,7 @@ __device__ __forceinline__ float add_f16(uint32_t w, float sum) {
 }  // namespace
 
 // XT: activation storage (float, _Float16, or uint16_t bf16 bits); SB: scale/bias storage.
-template <typename XT, typename SB, int BITS, int GS, int BM>
+template <typename XT, typename SB, int BITS, int GS, int BM, int KS>
 __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict__ x, int64_t M, int64_t K,
                                                             const uint32_t* __restrict__ wq,
                                                             const SB* __restrict__ scales,
@@ -146,44 +149,59 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   constexpr int SPB = GPB * GS / 64;          // K steps per table
   constexpr int SPP = SPB / 8;                // K steps per pair of groups
   constexpr int STAGES = XF32 ? 3 : 4;        // activation ring
-  constexpr int A_LD = BM / 64;               // 8-value chunks per thread (f32), or direct-to-LDS rounds
+  constexpr int NS = 8 / KS;                  // waves (32-column strips) per K-group
+  constexpr int BN = 32 * NS;
+  constexpr int A_ROWS = 8 * NS;              // rows one round of a K-group's loads covers
+  constexpr int A_LD = BM / A_ROWS;           // 8-value chunks per thread (f32), or direct-to-LDS rounds
+  static_assert(A_LD >= 1, "tile too low for the K-group");
   constexpr int NW = GS == 32 ? 2 : BITS / 4; // weight loads per lane per step (8 or 16 bytes)
-  constexpr int OFF_X = STAGES * STAGE;       // [group % 8][BM rows] f32 sums
-  constexpr int OFF_S = OFF_X + 8 * BM * 4;
+  constexpr int OFF_X = STAGES * STAGE;       // per K-group: its ring, then [group % 8][BM rows] f32 sums
+  constexpr int REGION = OFF_X + 8 * BM * 4;
+  constexpr int OFF_S = KS * REGION;
   constexpr int SW = 32 * GPB * (int)sizeof(SB);  // per wave: [half][32 columns][8 groups] scales, then biases
-  __shared__ __attribute__((aligned(16))) unsigned char lds[OFF_S + 8 * 2 * SW];
-  auto stage_at = [&](int t) { return lds + (XF32 ? t % 3 : t & 3) * STAGE; };
+  constexpr int PARTS = KS > 1 ? 8 * TM * 4096 : 0;  // the partial sums, over everything else
+  __shared__ __attribute__((aligned(16))) unsigned char lds_all[OFF_S + 8 * 2 * SW > PARTS ? OFF_S + 8 * 2 * SW : PARTS];
 
-  const int tid = threadIdx.x, lane = tid & 63, r32 = lane & 31, half = lane >> 5;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + kStripBN - 1) / kStripBN;
+  const int lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
+  const int wave_all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int kg = wave_all / NS, wave = wave_all % NS, tid = threadIdx.x % (64 * NS);  // K-group; within it
+  unsigned char* const lds = lds_all + kg * REGION;
+  auto stage_at = [&](int t) { return lds + (XF32 ? t % 3 : t & 3) * STAGE; };
+  const int64_t tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
   int64_t tm, tn;
   strip_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
-  const int64_t bm0 = tm * BM, bn0 = tn * kStripBN;
-  const int rows_m = (int)(M - bm0 < BM ? M - bm0 : BM), rows_n = (int)(N - bn0 < kStripBN ? N - bn0 : kStripBN);
+  const int64_t bm0 = tm * BM, bn0 = tn * BN;
+  const int rows_m = (int)(M - bm0 < BM ? M - bm0 : BM), rows_n = (int)(N - bn0 < BN ? N - bn0 : BN);
   const uint32_t kwords = (uint32_t)(K * BITS / 32);
-  const int groups = (int)(K / GS), T = (int)(K / 64);
+  const int groups_all = (int)(K / GS);
+  // This K-group's steps [t0, t0 + T), whole groups; every group runs T_run steps, the ones past its own
+  // on repeated operands with zero scales.
+  constexpr int UNIT = GS == 128 ? 2 : 1;  // steps
+  const int units = (int)(K / (64 * UNIT));
+  const int t0 = UNIT * (kg * units / KS), T = UNIT * ((kg + 1) * units / KS) - t0;
+  const int T_run = UNIT * ((units + KS - 1) / KS);
+  const int groups = T * 64 / GS, g_base = t0 * 64 / GS;
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<XT*>(x + bm0 * K), (short)0, (int)(uint32_t)(rows_m * K * (int64_t)sizeof(XT)), kStripFlags);
   const __amdgpu_buffer_rsrc_t rw = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint32_t*>(wq + bn0 * kwords), (short)0, (int)(uint32_t)(rows_n * (int64_t)kwords * 4), kStripFlags);
   const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<SB*>(scales + bn0 * groups), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups * (int64_t)sizeof(SB)), kStripFlags);
+      const_cast<SB*>(scales + bn0 * groups_all), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups_all * (int64_t)sizeof(SB)), kStripFlags);
   const __amdgpu_buffer_rsrc_t rz = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<SB*>(biases + bn0 * groups), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups * (int64_t)sizeof(SB)), kStripFlags);
+      const_cast<SB*>(biases + bn0 * groups_all), (short)0, (int)(uint32_t)(rows_n * (int64_t)groups_all * (int64_t)sizeof(SB)), kStripFlags);
 
   // ---- activations.  16-byte chunk c (8 values) of row r sits at chunk c ^ swz_f(r) of its row.
-  // fp16 / bf16: round i of wave w fills rows 64 i + 8 w .. + 7, lane L the chunk that belongs at
-  // position L & 7 of row 64 i + 8 w + (L >> 3).  f32: thread t loads chunk t & 7 (32 bytes) of rows
-  // t / 8 + 64 i.
+  // fp16 / bf16: round i of wave w fills rows A_ROWS i + 8 w .. + 7, lane L the chunk that belongs at
+  // position L & 7 of row A_ROWS i + 8 w + (L >> 3).  f32: thread t loads chunk t & 7 (32 bytes) of
+  // rows t / 8 + A_ROWS i.
   uint32_t x_off[A_LD];
 #pragma unroll
   for (int i = 0; i < A_LD; ++i) {
     if constexpr (XF32) {
-      x_off[i] = (uint32_t)(((tid >> 3) + 64 * i) * K * 4 + (tid & 7) * 32);
+      x_off[i] = (uint32_t)(((tid >> 3) + A_ROWS * i) * K * 4 + t0 * 256 + (tid & 7) * 32);
     } else {
-      const int r = 64 * i + 8 * wave + (lane >> 3);
-      x_off[i] = (uint32_t)((r * K + ((lane & 7) ^ swz_f(r)) * 8) * 2);
+      const int r = A_ROWS * i + 8 * wave + (lane >> 3);
+      x_off[i] = (uint32_t)((r * K + t0 * 64 + ((lane & 7) ^ swz_f(r)) * 8) * 2);
     }
   }
   auto dma_x = [&](int t) {  // !XF32
@@ -192,7 +210,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     const uint32_t tc = (uint32_t)(t < T ? t : T - 1);
 #pragma unroll
     for (int i = 0; i < A_LD; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(base + (64 * i + 8 * wave) * 128),
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(base + (A_ROWS * i + 8 * wave) * 128),
                                                16, x_off[i] + tc * 128u, 0, 0, 0);
 #else
     (void)t;
@@ -208,7 +226,8 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
         xr[i][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, x_off[i] + tc * 256u + 16u * q, 0, 0));
   };
   float* const xtab = reinterpret_cast<float*>(lds + OFF_X);
-  float xrun[XF32 ? A_LD : 1];  // GS 128: a row's sum over its group's first step
+  constexpr int XPASS = BM / NS > 16 ? BM / NS / 16 : 1;
+  float xrun[XF32 ? A_LD : XPASS];  // GS 128: a row's sum over its group's first step
   // X of group g for tile row `row`; the lanes that share a row write the same value.
   auto put_x = [&](int row, int g, float v) { xtab[(g & 7) * BM + row] = v; };
   // f32: split step t's registers into its stage and leave the group sums.  POS: t's position in its
@@ -217,7 +236,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     unsigned char* const base = stage_at(t);
 #pragma unroll
     for (int i = 0; i < A_LD; ++i) {
-      const int row = (tid >> 3) + 64 * i, c = tid & 7;
+      const int row = (tid >> 3) + A_ROWS * i, c = tid & 7;
       u32x4 hi, lo;
       float sum = 0.0f;
 #pragma unroll
@@ -247,10 +266,13 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
       }
     }
   };
-  // fp16 / bf16: the group sums of step t from its landed stage, BM / 8 rows per wave, four lanes a row
-  // (two chunks each).
+  // fp16 / bf16: the group sums of step t from its landed stage, BM / NS rows per wave, four lanes a
+  // row (two chunks each), 16 rows at a time.
   auto sum_x = [&](int t, auto POS) {
-    const int row = wave * (BM / 8) + ((lane >> 2) & (BM / 8 - 1)), q = lane & 3;
+    constexpr int RW = BM / NS;
+#pragma unroll
+    for (int ps = 0; ps < XPASS; ++ps) {
+    const int row = wave * RW + 16 * ps + ((lane >> 2) & (RW < 16 ? RW - 1 : 15)), q = lane & 3;
     const unsigned char* const base = stage_at(t) + row * 128;
     float part[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -275,8 +297,9 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     } else {
       sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4e, 0xf, 0xf, true));
       if constexpr (GS == 64) put_x(row, t, sum);
-      else if constexpr (decltype(POS)::value == 0) xrun[0] = sum;
-      else put_x(row, t >> 1, xrun[0] + sum);
+      else if constexpr (decltype(POS)::value == 0) xrun[ps] = sum;
+      else put_x(row, t >> 1, xrun[ps] + sum);
+    }
     }
   };
 
@@ -284,7 +307,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   // chunk 4 h + kk of k (group 64 and 128), or 4 (kk >> 1) + 2 h + (kk & 1) (group 32, so that MFMAs 0, 1
   // and 2, 3 stay inside one group): its packed words are contiguous, one or two loads.
   const uint32_t ncol = (uint32_t)(32 * wave + r32);
-  const uint32_t w_off = (ncol * kwords + (uint32_t)half * (GS == 32 ? BITS / 2 : BITS)) * 4u;
+  const uint32_t w_off = (ncol * kwords + (uint32_t)t0 * (2 * BITS) + (uint32_t)half * (GS == 32 ? BITS / 2 : BITS)) * 4u;
   auto chunk_of = [&](int kk) { return GS == 32 ? 4 * (kk >> 1) + 2 * half + (kk & 1) : 4 * half + kk; };
   uint32_t wr[2][BITS], wc[BITS];
   auto load_w = [&](int t, auto SLOT) {
@@ -312,12 +335,13 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   };
 
   // ---- scales and biases, 16 groups at a time: lane (h, r32) loads groups 16 b + 8 h .. + 7 of its
-  // column into the wave's LDS tables, from which each group's scale and bias are read back.  Groups past the last are zero.
+  // column into the wave's LDS tables, from which each group's scale and bias are read back.  Groups
+  // past the last are zero.
   struct Batch { uint32_t s[SBF ? 8 : 4], z[SBF ? 8 : 4]; };
   auto load_batch = [&](int b, Batch& d) {
     const int g0 = 16 * b + 8 * half;
-    const uint32_t at = (ncol * (uint32_t)groups + (uint32_t)g0) * (uint32_t)sizeof(SB);
-    if (16 * b + 16 <= groups && (SBF || (groups & 1) == 0)) {  // whole and dword-aligned
+    const uint32_t first = ncol * (uint32_t)groups_all + (uint32_t)(g_base + g0), at = first * (uint32_t)sizeof(SB);
+    if (16 * b + 16 <= groups && (SBF || ((groups_all | g_base) & 1) == 0)) {  // whole and dword-aligned
 #pragma unroll
       for (int q = 0; q < (SBF ? 2 : 1); ++q) {
         const u32x4 s = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, at + 16u * q, 0, 0));
@@ -332,7 +356,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
       uint32_t s[8], z[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint32_t idx = g0 + e < groups ? ncol * (uint32_t)groups + (uint32_t)(g0 + e) : 0xffffffffu / (uint32_t)sizeof(SB);
+        const uint32_t idx = g0 + e < groups ? first + (uint32_t)e : 0xffffffffu / (uint32_t)sizeof(SB);
         s[e] = load_sb_bits<SB>(rs, idx);  // past the resource: zero
         z[e] = load_sb_bits<SB>(rz, idx);
       }
@@ -343,7 +367,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
       }
     }
   };
-  unsigned char* const stab = lds + OFF_S + wave * 2 * SW;
+  unsigned char* const stab = lds_all + OFF_S + wave_all * 2 * SW;
   auto put_tables = [&](const Batch& d) {
     unsigned char* const p = stab + half * (SW / 2) + r32 * (8 * (int)sizeof(SB));
 #pragma unroll
@@ -496,21 +520,35 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   read_a(0, lds, 0);
   cf[0] = codes8<BITS, F16>(wc, 0);
   int t = 0;
-  for (; t + 1 < T; t += 2) {
+  for (; t + 1 < T_run; t += 2) {
     step(t, I0{});
     step(t + 1, I1{});
   }
-  if (t < T) step(t, I0{});
+  if (t < T_run) step(t, I0{});
   // The last pair's bias term when its second group does not exist, and the last group's fold.
-  if (T % SPP != 0) bias_pair((T - 1) / SPP);
+  if (T_run % SPP != 0) bias_pair((T_run - 1) / SPP);
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int v = 0; v < 16; ++v) yv[i][v] = fmaf(s_prev, acc[i][v], yv[i][v]);
-  mlxq_vmcnt<0>();  // no direct-to-LDS load outlives the workgroup
+  mlxq_vmcnt<0>();  // no direct-to-LDS load outlives the loop
 
-  // ---- epilogue: lane holds column n and rows m = 32 i + 8 (v >> 2) + 4 half + (v & 3): y + bias in
-  // f32, the LoRA residual (xa . lbt^T on the f32 matrix cores) times its scale, the activation.
+  // ---- K-groups: every wave leaves its partial sums in LDS (over the rings and tables, which all waves
+  // are past), and takes 1 / KS of its strip's 4-row pieces (i, q) to add up, in K-group order, and finish.
+  constexpr int MINE = TM * 4 / KS;
+  auto part = reinterpret_cast<f32x4 (*)[TM * 4][64]>(lds_all);
+  if constexpr (KS > 1) {
+    strip_barrier();
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int q = 0; q < 4; ++q)
+        part[wave_all][4 * i + q][lane] = f32x4{yv[i][4 * q], yv[i][4 * q + 1], yv[i][4 * q + 2], yv[i][4 * q + 3]};
+    strip_barrier();
+  }
+
+  // ---- epilogue: lane holds column n and rows m = 32 i + 8 q + 4 half + e: y + bias in f32, the LoRA
+  // residual (xa . lbt^T on the f32 matrix cores) times its scale, the activation.
   const bool n_ok = (int)ncol < rows_n;
   const int64_t n = bn0 + (n_ok ? (int)ncol : 0);
   const float bv = epi.bias == nullptr ? -0.0f
@@ -521,11 +559,8 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   auto finish = [&](auto ACT) {
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-      f32x16 o;
-#pragma unroll
-      for (int v = 0; v < 16; ++v) o[v] = yv[i][v] + bv;
+      f32x16 r = {};
       if (epi.R > 0) {
-        f32x16 r = {};
         const int mr = 32 * i + r32 < rows_m ? 32 * i + r32 : rows_m - 1;
         for (int k = 0; k < epi.R; k += 16) {
           const f32x4* const xp = reinterpret_cast<const f32x4*>(epi.xa + (bm0 + mr) * epi.R + k + 8 * half);
@@ -537,17 +572,28 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
             r = __builtin_amdgcn_mfma_f32_32x32x2f32(x1[e], l1[e], r, 0, 0, 0);
           }
         }
-#pragma unroll
-        for (int v = 0; v < 16; ++v) o[v] += r[v] * epi.lora_scale;
       }
 #pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        float ov = o[v];
-        if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_EXACT) ov = gelu_erf(ov);
-        else if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_TANH) ov = gelu_tanh<false>(ov);
-        const int row = 32 * i + 8 * (v >> 2) + 4 * half + (v & 3);
-        const uint32_t at = n_ok ? (uint32_t)(row * N + n) * 4u : 0xfffffffcu;  // rows past M fall past the resource
-        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ov), ry, at, 0, 0);
+      for (int q = 0; q < 4; ++q) {
+        if (KS > 1 && (4 * i + q) / MINE != kg) continue;  // wave-uniform
+        f32x4 o;
+        if constexpr (KS > 1) {
+          o = part[wave][4 * i + q][lane];
+#pragma unroll
+          for (int k = 1; k < KS; ++k) o += part[k * NS + wave][4 * i + q][lane];
+        } else {
+          o = f32x4{yv[i][4 * q], yv[i][4 * q + 1], yv[i][4 * q + 2], yv[i][4 * q + 3]};
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float ov = o[e] + bv;
+          if (epi.R > 0) ov += r[4 * q + e] * epi.lora_scale;
+          if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_EXACT) ov = gelu_erf(ov);
+          else if constexpr (decltype(ACT)::value == MLXQ_ACT_GELU_TANH) ov = gelu_tanh<false>(ov);
+          const int row = 32 * i + 8 * q + 4 * half + e;
+          const uint32_t at = n_ok ? (uint32_t)(row * N + n) * 4u : 0xfffffffcu;  // rows past M fall past the resource
+          __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(ov), ry, at, 0, 0);
+        }
       }
     }
   };
@@ -556,45 +602,81 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   else finish(std::integral_constant<int, MLXQ_ACT_NONE>{});
 }
 
-template <typename XT, typename SB, int BITS, int GS, int BM>
+template <typename XT, typename SB, int BITS, int GS, int BM, int KS>
 static int launch_strip(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                         int64_t N, void* y, const F32Epilogue& epi, hipStream_t st) {
-  const int64_t tiles = ((M + BM - 1) / BM) * ((N + kStripBN - 1) / kStripBN);
+  constexpr int BN = 256 / KS;
+  const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "qmm_f32: problem too large");
-  hipLaunchKernelGGL((qmm_f32_strip_kernel<XT, SB, BITS, GS, BM>), dim3((unsigned)tiles), dim3(512), 0, st, (const XT*)x,
-                     M, K, wq, (const SB*)s, (const SB*)b, N, (float*)y, epi);
+  hipLaunchKernelGGL((qmm_f32_strip_kernel<XT, SB, BITS, GS, BM, KS>), dim3((unsigned)tiles), dim3(512), 0, st,
+                     (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N, (float*)y, epi);
   return check_launch("qmm_f32");
+}
+
+// Tile height and K-groups: 0: 128 rows; 1: 64 rows; 2: 64 rows in 2 K-groups; 3: 32 rows in 4.
+// One workgroup runs per CU, so a shape costs its rounds of tiles times its chain of K steps: the
+// shape with the least rounds * (steps * t + 5 us), with t, the measured time of a step (us), 0.95 /
+// 0.63 / 0.71 / 0.63 for one pass and 1.7 / 0.95 / 1.2 / 1.25 for two.  Measured, us for shapes 0..3
+// (Q4 g64 unless stated): fp16 77 x 1280 x 5120 Q8 26.4 / 19.1 / 13.9 / 9.3, 77 x 5120 x 1280 81.7 /
+// 55.4 / 33.8 / 17.1, 256 x 1280 x 5120 25.9 / 18.3 / 13.9 / 21.9, 512 x 3072 x 3072 52.7 / 36.1 / 25.1 /
+// 39.8, 2048 x 1280 x 1280 26.7 / 19.1 / 25.4 / 35.1, 1024 x 1280 x 10240 54.0 / 54.9 / 64.3 / 132;
+// f32 20 x 3072 x 12288 82.8 / 47.5 / 33.6 / 19.9, 256 x 3072 x 3072 86.4 / 51.6 / 34.8 / 38.0,
+// 512 x 3072 x 12288 90.1 / 108 / 115 / 213, 1024 x 3072 x 3072 88.3 / 53.4 / 71.3 / 107.
+inline int strip_shape(int64_t M, int64_t K, int64_t N, int gs, bool two_pass) {
+  static constexpr int kRows[4] = {128, 64, 64, 32}, kGroups[4] = {1, 1, 2, 4};
+  static constexpr int kStep[2][4] = {{95, 63, 71, 63}, {170, 95, 120, 125}};  // 10 ns
+  const int64_t cus = device_cu_count(), steps = K / 64;
+  int best = 0;
+  int64_t best_cost = 0;
+  for (int i = 0; i < 4; ++i) {
+    const int64_t bn = 256 / kGroups[i];
+    if (i > 1 && steps / (gs == 128 ? 2 : 1) < kGroups[i]) continue;  // every K-group needs a step
+    const int64_t tiles = ((M + kRows[i] - 1) / kRows[i]) * ((N + bn - 1) / bn);
+    const int64_t cost = (tiles + cus - 1) / cus * ((steps + kGroups[i] - 1) / kGroups[i] * kStep[two_pass][i] + 500);
+    if (i == 0 || cost < best_cost) {
+      best = i;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
+template <typename XT, typename SB, int BITS, int GS>
+static int strip_tile(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                      void* y, const F32Epilogue& epi, hipStream_t st) {
+  switch (strip_shape(M, K, N, GS, std::is_same<XT, float>::value)) {
+    case 0: return launch_strip<XT, SB, BITS, GS, 128, 1>(x, M, K, wq, s, b, N, y, epi, st);
+    case 1: return launch_strip<XT, SB, BITS, GS, 64, 1>(x, M, K, wq, s, b, N, y, epi, st);
+    case 2: return launch_strip<XT, SB, BITS, GS, 64, 2>(x, M, K, wq, s, b, N, y, epi, st);
+    default: return launch_strip<XT, SB, BITS, GS, 32, 4>(x, M, K, wq, s, b, N, y, epi, st);
+  }
 }
 
 template <typename XT, typename SB>
 static int strip_bits_gs(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                          int64_t N, int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st) {
-  const bool big = ((M + 127) / 128) * ((N + kStripBN - 1) / kStripBN) >= device_cu_count() * 3 / 4;
-#define MLXQ_ST(B, G)                                                                             \
-  if (bits == B && gs == G)                                                                       \
-    return big ? launch_strip<XT, SB, B, G, 128>(x, M, K, wq, s, b, N, y, epi, st)                \
-               : launch_strip<XT, SB, B, G, 64>(x, M, K, wq, s, b, N, y, epi, st);
+#define MLXQ_ST(B, G) \
+  if (bits == B && gs == G) return strip_tile<XT, SB, B, G>(x, M, K, wq, s, b, N, y, epi, st);
   MLXQ_ST(4, 32) MLXQ_ST(4, 64) MLXQ_ST(4, 128) MLXQ_ST(8, 32) MLXQ_ST(8, 64) MLXQ_ST(8, 128)
 #undef MLXQ_ST
   return set_error(MLXQ_EINVAL, "qmm_f32: unsupported bits=%d group_size=%d", bits, gs);
 }
 
-// Whether a tile's rows fit 32-bit byte offsets (operands of any number of rows do).
-bool qmm_f32_strip_fits(int64_t K, int64_t N) { return K % 64 == 0 && K < (1LL << 22) && N < (1LL << 22); }
-
-int run_qmm_f32_strip(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
-                      const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, const F32Epilogue& epi,
-                      hipStream_t st) {
-  if (M == 0 || N == 0) return MLXQ_OK;
-  if (x_dtype == MLXQ_FLOAT32) {
-    if (sb_dtype == MLXQ_BFLOAT16) return strip_bits_gs<float, uint16_t>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
-    return strip_bits_gs<float, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
+// One operand mix per translation unit (qmm_f32_strip_*.hip), so that they compile side by side.
+#define MLXQ_STRIP_ENTRY(NAME, XT, SB)                                                                          \
+  int NAME(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,    \
+           int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st) {                                 \
+    return strip_bits_gs<XT, SB>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);                                   \
   }
-  if (x_dtype == MLXQ_FLOAT16) {
-    if (sb_dtype == MLXQ_BFLOAT16) return strip_bits_gs<_Float16, uint16_t>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
-    return strip_bits_gs<_Float16, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
-  }
-  return strip_bits_gs<uint16_t, float>(x, M, K, wq, s, b, N, gs, bits, y, epi, st);
-}
+int run_strip_f32_bf16(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                       int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st);
+int run_strip_f32_f32(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                      int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st);
+int run_strip_f16_bf16(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                       int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st);
+int run_strip_f16_f32(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                      int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st);
+int run_strip_bf16_f32(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
+                       int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st);
 
 }  // namespace mlxq

@@ -63,7 +63,12 @@ def _check(mlxq, x, pack, gs, bits, what, **kw):
     (9, 1, 64, 64, 4), (33, 31, 128, 128, 8), (64, 257, 192, 64, 8), (65, 256, 64, 32, 4),
     (31, 255, 1024, 64, 4), (127, 33, 1088, 64, 8), (129, 300, 960, 64, 4), (20, 513, 2048, 128, 4),
     (40, 64, 2176, 128, 8), (63, 97, 512, 32, 8), (17, 130, 576, 32, 4), (12, 40, 448, 32, 8),
-    (30, 70, 2304, 64, 4), (4224, 2100, 320, 64, 4), (6200, 1030, 384, 128, 8), (3000, 2600, 128, 32, 4),
+    (30, 70, 2304, 64, 4),
+    # K-groups: as many steps as groups, one more, uneven shares, an odd first group (scale rows that
+    # start mid-word), 64-row tiles in two groups, and grids that fill the CUs
+    (33, 63, 256, 64, 4), (32, 65, 320, 64, 8), (40, 200, 448, 64, 4), (9, 4096, 1152, 128, 4), (77, 5120, 1280, 64, 8),
+    (256, 3000, 704, 64, 4), (250, 2100, 832, 32, 8), (512, 2048, 1536, 128, 8),
+    (4224, 2100, 320, 64, 4), (6200, 1030, 384, 128, 8), (3000, 2600, 128, 32, 4),
 ])
 def test_strip_edges(mlxq, xdt, sb, M, N, K, gs, bits):
     banner("strip", xdt, sb, M, N, K, gs, bits)
