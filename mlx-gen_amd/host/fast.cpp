@@ -11,6 +11,8 @@
 
 #include <ATen/ATen.h>
 
+#include <vector>
+
 #include "../../include/mlxq.h"
 
 namespace {
@@ -249,11 +251,96 @@ PyObject* embedding(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// dequantize(wq, scales, biases, group_size, bits)
+PyObject* dequantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    long v[2];
+    Pack p;
+    if (n != 5 || !ints(a + 3, 2, v) || (v[1] != 4 && v[1] != 8)) return nullptr;
+    const at::Tensor* wq = plain(a[0], 16);
+    if (!wq || wq->dim() != 2) return nullptr;
+    const int64_t K = wq->size(1) * 32 / v[1];
+    if (!get_pack(a[0], a[1], a[2], K, v[0], v[1], p)) return nullptr;
+    bool ok;
+    void* st = stream_of(p.wq, ok);
+    if (!ok) return nullptr;
+    at::Tensor out = at::empty({p.N, K}, p.s.options());
+    if (unlocked([&] {
+          return mlxq_dequantize((const uint32_t*)p.wq.data_ptr(), p.s.data_ptr(), p.b.data_ptr(), p.dt, p.N, K,
+                                 (int)v[0], (int)v[1], out.data_ptr(), st);
+        }) != MLXQ_OK)
+      return nullptr;
+    return THPVariable_Wrap(std::move(out));
+  });
+}
+
+// quantize_batched(weights, group_size, bits): a list of equal 2-D weights -> a list of (wq, scales,
+// biases), the scales and biases of each two views of one allocation, the biases 256 to 511 bytes past
+// the scales' end.
+PyObject* quantize_batched(PyObject*, PyObject* const* a, Py_ssize_t n) {
+  return guarded([&]() -> PyObject* {
+    long v[2];
+    if (n != 3 || !PyList_CheckExact(a[0]) || !ints(a + 1, 2, v)) return nullptr;
+    const Py_ssize_t count = PyList_GET_SIZE(a[0]);
+    const long gs = v[0], bits = v[1];
+    if (count < 1 || (bits != 4 && bits != 8) || (gs != 32 && gs != 64 && gs != 128)) return nullptr;
+    std::vector<at::Tensor> w;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      const at::Tensor* t = plain(PyList_GET_ITEM(a[0], i), 16);
+      if (!t || t->dim() != 2 || t->numel() == 0) return nullptr;
+      if (i && (t->sizes() != w[0].sizes() || t->scalar_type() != w[0].scalar_type() || t->device() != w[0].device()))
+        return nullptr;
+      w.push_back(*t);
+    }
+    const int64_t N = w[0].size(0), K = w[0].size(1), G = K / gs;
+    const int dt = code_of(w[0].scalar_type());
+    if ((dt != MLXQ_BFLOAT16 && dt != MLXQ_FLOAT32) || K % gs != 0) return nullptr;
+    bool ok;
+    void* st = stream_of(w[0], ok);
+    if (!ok) return nullptr;
+    const int64_t esz = dt == MLXQ_FLOAT32 ? 4 : 2, off = (N * G * esz + 511) / 256 * 256 / esz;
+    std::vector<at::Tensor> q, s, b;
+    std::vector<const void*> wp;
+    std::vector<uint32_t*> qp;
+    std::vector<void*> sp, bp;
+    for (Py_ssize_t i = 0; i < count; ++i) {
+      q.push_back(at::empty({N, K * bits / 32}, w[0].options().dtype(at::kInt)));
+      at::Tensor sb = at::empty({off + N * G}, w[0].options());
+      s.push_back(sb.as_strided({N, G}, {G, 1}, 0));
+      b.push_back(sb.as_strided({N, G}, {G, 1}, off));
+      wp.push_back(w[i].data_ptr());
+      qp.push_back((uint32_t*)q[i].data_ptr());
+      sp.push_back(s[i].data_ptr());
+      bp.push_back(b[i].data_ptr());
+    }
+    if (unlocked([&] {
+          return mlxq_quantize_batched(wp.data(), (int)count, dt, N, K, (int)gs, (int)bits, qp.data(), sp.data(),
+                                       bp.data(), st);
+        }) != MLXQ_OK)
+      return nullptr;
+    PyObject* out = PyList_New(count);
+    for (Py_ssize_t i = 0; out && i < count; ++i) {
+      PyObject* t = PyTuple_New(3);
+      if (!t) {
+        Py_CLEAR(out);
+        break;
+      }
+      PyTuple_SET_ITEM(t, 0, THPVariable_Wrap(q[i]));
+      PyTuple_SET_ITEM(t, 1, THPVariable_Wrap(s[i]));
+      PyTuple_SET_ITEM(t, 2, THPVariable_Wrap(b[i]));
+      PyList_SET_ITEM(out, i, t);
+    }
+    return out;
+  });
+}
+
 PyMethodDef kMethods[] = {
     {"quantized_matmul", (PyCFunction)(void*)quantized_matmul, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, nullptr},
     {"swiglu", (PyCFunction)(void*)swiglu, METH_FASTCALL, nullptr},
     {"embedding", (PyCFunction)(void*)embedding, METH_FASTCALL, nullptr},
+    {"dequantize", (PyCFunction)(void*)dequantize, METH_FASTCALL, nullptr},
+    {"quantize_batched", (PyCFunction)(void*)quantize_batched, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -162,6 +162,10 @@ def quantize(w: torch.Tensor, group_size: int = DEFAULT_GROUP_SIZE, bits: int = 
 def quantize_batched(ws, group_size: int = DEFAULT_GROUP_SIZE, bits: int = 4):
     """quantize() over a list of weights of one shape and dtype, in launches of up to 16 weights
     (mlxq_quantize_batched): the same (wq, scales, biases) triples as one quantize() per weight."""
+    if type(ws) is list:
+        packs = _lib.fast().quantize_batched(ws, group_size, bits)
+        if packs is not None:
+            return packs
     ws = [w.contiguous() for w in ws]
     if not ws:
         return []
@@ -189,6 +193,9 @@ def _k_of(wq: torch.Tensor, bits: int) -> int:
 
 
 def dequantize(wq, scales, biases, group_size: int = DEFAULT_GROUP_SIZE, bits: int = 4):
+    out = _lib.fast().dequantize(wq, scales, biases, group_size, bits)
+    if out is not None:
+        return out
     if bits not in (4, 8):
         _bad("dequantize", f"bits must be 4 or 8 (got {bits})")
     wq, scales, biases = _pack3(wq, scales, biases)

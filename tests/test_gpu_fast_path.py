@@ -23,6 +23,8 @@ def test_host_tensors_take_the_general_path(mlxq):
     assert f.linear(x, wq, s, s, 64, 4, None, None, None, 1.0, 0) is None
     assert f.swiglu(x, (wq, s, s), [wq, s, s], 64, 4) is None
     assert f.embedding(torch.zeros(3, dtype=torch.int32), wq, s, s, 64, 4, 1) is None
+    assert f.dequantize(wq, s, s, 64, 4) is None and f.quantize_batched([x, x], 64, 4) is None
+    assert f.quantize_batched((x,), 64, 4) is None and f.quantize_batched([], 64, 4) is None
     assert f.linear(None, 3, "a", s, 64, 4, None, None, None, 1.0, 0) is None
     assert f.quantized_matmul(x) is None
     with pytest.raises(ValueError):
@@ -90,3 +92,24 @@ def test_fast_swiglu_embedding_and_prepared_operands(mlxq):
         mlxq.linear(x, *gate, 64, 4, activation=9)
     with pytest.raises(mlxq.MlxqError):
         mlxq.quantized_matmul(x, *gate, False, 64, 4)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("N,K,gs,bits,count", [(5, 192, 64, 4, 1), (33, 128, 128, 8, 3), (7, 96, 32, 4, 17)])
+def test_fast_quantize_dequantize(mlxq, dt, N, K, gs, bits, count):
+    ws = [(torch.randn((N, K), device="cuda") * 0.02).to(dt) for _ in range(count)]
+    got = mlxq.quantize_batched(ws, gs, bits)
+    want = mlxq.quantize_batched(tuple(ws), gs, bits)  # a tuple: the general path
+    assert type(got) is list and all(type(t) is tuple for t in got)
+    for g, w in zip(got, want):
+        for a, b in zip(g, w):
+            assert a.dtype == b.dtype and a.shape == b.shape and a.stride() == b.stride() and torch.equal(a, b)
+        assert g[2].data_ptr() - g[1].data_ptr() == w[2].data_ptr() - w[1].data_ptr()
+    d = mlxq.dequantize(*got[0], gs, bits)
+    strided = got[0][1].t().contiguous().t()  # needs preparation: the general path
+    assert d.dtype == dt and torch.equal(d, mlxq.dequantize(got[0][0], strided, got[0][2], gs, bits))
+    with pytest.raises(mlxq.MlxqError):
+        mlxq.dequantize(got[0][0], got[0][1][:, :0], got[0][2], gs, bits)
+    with pytest.raises(mlxq.MlxqError):
+        mlxq.quantize_batched(ws, 48, bits)
