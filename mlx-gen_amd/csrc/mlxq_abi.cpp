@@ -617,6 +617,14 @@ int mlxq_linear(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t
     }
     return run_qmm_f32(x, x_dtype, M, K, wq, scales, biases, sb_dtype, N, group_size, bits, y, st, fe);
   }
+  // A bf16 decode product takes a bf16 bias and activation in its own store.
+  if (epilogue && p.d0_bf16 && p.out_bf16 && M <= 8 && !p.lora &&
+      qmv_mfma_applicable(x_dtype, sb_dtype, M, K, N, group_size, bits)) {
+    const uint16_t* table = nullptr;
+    if (p.act != MLXQ_ACT_NONE && !(table = act_table_ptr(fused_act_of(p.act), st))) return MLXQ_EDEVICE;
+    return run_qmv_mfma(x, M, K, wq, scales, biases, N, group_size, bits, y, st,
+                        p.bias ? (const uint16_t*)ep->bias : nullptr, table);
+  }
   // The product in D0, straight into y when y has that dtype; a bf16 product whose result
   // promotes to f32 goes through the workspace (the elementwise epilogue widens it into y).
   void* y0 = p.promoted() ? (char*)workspace + p.y0 : y;

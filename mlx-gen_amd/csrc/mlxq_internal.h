@@ -85,8 +85,11 @@ int run_qmm_wide(const void* x, int64_t M, int64_t K, const uint32_t* wq, const 
                  int sb_dtype, int64_t N, int gs, int bits, void* y, const QmmEpilogue& epi,
                  hipStream_t st, const QmmBatch& batch = QmmBatch{});
 bool qmv_mfma_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_t N, int gs, int bits);
+// bias [N] (bf16) and act_table (a FusedAct's bf16 table), null when absent, are applied to the rounded
+// product, one rounding per op.
 int run_qmv_mfma(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
-                 int64_t N, int gs, int bits, void* y, hipStream_t st);
+                 int64_t N, int gs, int bits, void* y, hipStream_t st, const uint16_t* bias = nullptr,
+                 const uint16_t* act_table = nullptr);
 bool swiglu_qmv_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_t F, int gs, int bits);
 int run_swiglu_qmv(const void* x, int64_t M, int64_t K, const uint32_t* wq_g, const void* s_g,
                    const void* b_g, const uint32_t* wq_u, const void* s_u, const void* b_u, int64_t F,
