@@ -14,8 +14,8 @@
 // groups per bf16 MFMA (X in three bf16 terms), 1.7e-7 with four, 1.6e-7 with two after both folds,
 // and is 1.4e-7 in this form, as with two FMAs per output and group.
 //
-// Workgroup: 8 waves, tile BM (128 or 64) x 256, K advanced 64 per step; wave w owns columns
-// [32 w, 32 w + 32) of all BM rows.  Small grids (strip_shape) take KS = 2 or 4 K-groups of 8 / KS
+// Workgroup: 8 waves, tile BM (128 or 64) x 256 TN, K advanced 64 per step; wave w owns TN strips of 32
+// columns, all BM rows of them.  Small grids (strip_shape) take KS = 2 or 4 K-groups of 8 / KS
 // waves instead: each group walks its own share of K, with its own activation ring, over the same
 // 256 / KS columns, and the partial sums meet in LDS at the end.  What bounds it is the LDS port: a wave reads 1 KB of activations
 // per MFMA (32 cycles of one SIMD's matrix core; four SIMDs against 128 bytes per cycle).  Hence the
@@ -132,7 +132,7 @@ __device__ __forceinline__ float add_f16(uint32_t w, float sum) {
 }  // namespace
 
 // XT: activation storage (float, _Float16, or uint16_t bf16 bits); SB: scale/bias storage.
-template <typename XT, typename SB, int BITS, int GS, int BM, int KS>
+template <typename XT, typename SB, int BITS, int GS, int BM, int KS, int TN>
 __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict__ x, int64_t M, int64_t K,
                                                             const uint32_t* __restrict__ wq,
                                                             const SB* __restrict__ scales,
@@ -149,8 +149,9 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   constexpr int SPB = GPB * GS / 64;          // K steps per table
   constexpr int SPP = SPB / 8;                // K steps per pair of groups
   constexpr int STAGES = XF32 ? 3 : 4;        // activation ring
-  constexpr int NS = 8 / KS;                  // waves (32-column strips) per K-group
-  constexpr int BN = 32 * NS;
+  constexpr int NS = 8 / KS;                  // waves per K-group, TN 32-column strips each
+  constexpr int BN = 32 * TN * NS;
+  static_assert(KS == 1 || TN == 1, "K-groups add up one strip per wave");
   constexpr int A_ROWS = 8 * NS;              // rows one round of a K-group's loads covers
   constexpr int A_LD = BM / A_ROWS;           // 8-value chunks per thread (f32), or direct-to-LDS rounds
   static_assert(A_LD >= 1, "tile too low for the K-group");
@@ -160,7 +161,8 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   constexpr int OFF_S = KS * REGION;
   constexpr int SW = 32 * GPB * (int)sizeof(SB);  // per wave: [half][32 columns][8 groups] scales, then biases
   constexpr int PARTS = KS > 1 ? 8 * TM * 4096 : 0;  // the partial sums, over everything else
-  __shared__ __attribute__((aligned(16))) unsigned char lds_all[OFF_S + 8 * 2 * SW > PARTS ? OFF_S + 8 * 2 * SW : PARTS];
+  constexpr int TABLES = 8 * TN * 2 * SW;
+  __shared__ __attribute__((aligned(16))) unsigned char lds_all[OFF_S + TABLES > PARTS ? OFF_S + TABLES : PARTS];
 
   const int lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
   const int wave_all = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -306,41 +308,47 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   // ---- weights: column n = 32 w + r32 of the tile.  Lane half h covers, for MFMA kk of a step, 16-byte
   // chunk 4 h + kk of k (group 64 and 128), or 4 (kk >> 1) + 2 h + (kk & 1) (group 32, so that MFMAs 0, 1
   // and 2, 3 stay inside one group): its packed words are contiguous, one or two loads.
-  const uint32_t ncol = (uint32_t)(32 * wave + r32);
-  const uint32_t w_off = (ncol * kwords + (uint32_t)t0 * (2 * BITS) + (uint32_t)half * (GS == 32 ? BITS / 2 : BITS)) * 4u;
+  uint32_t ncol[TN], w_off[TN];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    ncol[j] = (uint32_t)(32 * (TN * wave + j) + r32);
+    w_off[j] = (ncol[j] * kwords + (uint32_t)t0 * (2 * BITS) + (uint32_t)half * (GS == 32 ? BITS / 2 : BITS)) * 4u;
+  }
   auto chunk_of = [&](int kk) { return GS == 32 ? 4 * (kk >> 1) + 2 * half + (kk & 1) : 4 * half + kk; };
-  uint32_t wr[2][BITS], wc[BITS];
+  uint32_t wr[2][TN][BITS], wc[TN][BITS];
   auto load_w = [&](int t, auto SLOT) {
     constexpr int sl = decltype(SLOT)::value;
-    const uint32_t at = w_off + (uint32_t)(t < T ? t : T - 1) * (8u * BITS);
     constexpr int EACH = BITS / NW;  // words per load
 #pragma unroll
-    for (int q = 0; q < NW; ++q) {
-      const uint32_t o = at + (GS == 32 ? 4u * BITS * q : 16u * q);
+    for (int jq = 0; jq < TN * NW; ++jq) {
+      const int j = jq / NW, q = jq % NW;
+      const uint32_t o = w_off[j] + (uint32_t)(t < T ? t : T - 1) * (8u * BITS) + (GS == 32 ? 4u * BITS * q : 16u * q);
       if constexpr (EACH == 2) {
         const u32x2 v = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rw, o, 0, 0));
 #pragma unroll
-        for (int e = 0; e < 2; ++e) wr[sl][2 * q + e] = v[e];
+        for (int e = 0; e < 2; ++e) wr[sl][j][2 * q + e] = v[e];
       } else {
         const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw, o, 0, 0));
 #pragma unroll
-        for (int e = 0; e < 4; ++e) wr[sl][4 * q + e] = v[e];
+        for (int e = 0; e < 4; ++e) wr[sl][j][4 * q + e] = v[e];
       }
     }
   };
   auto take_w = [&](auto SLOT) {
     constexpr int sl = decltype(SLOT)::value;
 #pragma unroll
-    for (int e = 0; e < BITS; ++e) wc[e] = take(wr[sl][e]);
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int e = 0; e < BITS; ++e) wc[j][e] = take(wr[sl][j][e]);
   };
 
   // ---- scales and biases, 16 groups at a time: lane (h, r32) loads groups 16 b + 8 h .. + 7 of its
   // column into the wave's LDS tables, from which each group's scale and bias are read back.  Groups
   // past the last are zero.
   struct Batch { uint32_t s[SBF ? 8 : 4], z[SBF ? 8 : 4]; };
-  auto load_batch = [&](int b, Batch& d) {
+  auto load_batch = [&](int b, int j, Batch& d) {
     const int g0 = 16 * b + 8 * half;
-    const uint32_t first = ncol * (uint32_t)groups_all + (uint32_t)(g_base + g0), at = first * (uint32_t)sizeof(SB);
+    const uint32_t first = ncol[j] * (uint32_t)groups_all + (uint32_t)(g_base + g0), at = first * (uint32_t)sizeof(SB);
     if (16 * b + 16 <= groups && (SBF || ((groups_all | g_base) & 1) == 0)) {  // whole and dword-aligned
 #pragma unroll
       for (int q = 0; q < (SBF ? 2 : 1); ++q) {
@@ -367,42 +375,50 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
       }
     }
   };
-  unsigned char* const stab = lds_all + OFF_S + wave_all * 2 * SW;
-  auto put_tables = [&](const Batch& d) {
-    unsigned char* const p = stab + half * (SW / 2) + r32 * (8 * (int)sizeof(SB));
+  unsigned char* const stab = lds_all + OFF_S + wave_all * TN * 2 * SW;  // [strip][scales, biases]
+  auto put_tables = [&](int j, const Batch& d) {
+    unsigned char* const p = stab + j * 2 * SW + half * (SW / 2) + r32 * (8 * (int)sizeof(SB));
 #pragma unroll
     for (int q = 0; q < (SBF ? 2 : 1); ++q) {
       *reinterpret_cast<u32x4*>(p + 16 * q) = u32x4{d.s[4 * q], d.s[4 * q + 1], d.s[4 * q + 2], d.s[4 * q + 3]};
       *reinterpret_cast<u32x4*>(p + SW + 16 * q) = u32x4{d.z[4 * q], d.z[4 * q + 1], d.z[4 * q + 2], d.z[4 * q + 3]};
     }
   };
-  auto scale_of = [&](int g) {
-    return SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + ((g >> 3) & 1) * (SW / 2)) + r32 * 8, g & 7);
+  auto scale_of = [&](int j, int g) {
+    return SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + j * 2 * SW + ((g >> 3) & 1) * (SW / 2)) + r32 * 8, g & 7);
   };
 
-  f32x16 acc[TM], yv[TM];
+  f32x16 acc[TM][TN], yv[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      acc[i][v] = 0.0f;
-      yv[i][v] = 0.0f;
-    }
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        acc[i][j][v] = 0.0f;
+        yv[i][j][v] = 0.0f;
+      }
   // y += b . X over the groups 2 p and 2 p + 1; this half's operands are those of group 2 p + half.
   auto bias_pair = [&](int p) {
     const int g = 2 * p + half;
-    const float z = SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + SW + ((p >> 2) & 1) * (SW / 2)) + r32 * 8, 2 * (p & 3) + half);
+    float z[TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+      z[j] = SBLoad<SB>::ld(reinterpret_cast<const SB*>(stab + j * 2 * SW + SW + ((p >> 2) & 1) * (SW / 2)) + r32 * 8,
+                            2 * (p & 3) + half);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
       const float xg = xtab[(g & 7) * BM + 32 * i + r32];
-      yv[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(g < groups ? xg : 0.0f, z, yv[i], 0, 0, 0);
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+        yv[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(g < groups ? xg : 0.0f, z[j], yv[i][j], 0, 0, 0);
     }
   };
 
   // ---- the loop.  Sub-step u = kk * P + part of a step multiplies fragments of one activation part
   // by the codes of MFMA kk; its fragments were read one sub-step earlier.
   constexpr int NSUB = 4 * P;
-  u32x4 af[2][TM], cf[2];
+  u32x4 af[2][TM], cf[2][TN];
   int a_off[4];
 #pragma unroll
   for (int kk = 0; kk < 4; ++kk) a_off[kk] = r32 * 128 + ((chunk_of(kk) ^ swz_f(r32)) << 4);
@@ -411,7 +427,11 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     for (int i = 0; i < TM; ++i)
       af[slot][i] = *reinterpret_cast<const u32x4*>(base + (u % P) * PART + i * 4096 + a_off[u / P]);
   };
-  float s_prev = 0.0f, s_next[2] = {0.0f, 0.0f};
+  auto convert = [&](int slot, int kk) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) cf[slot][j] = codes8<BITS, F16>(wc[j], kk);
+  };
+  float s_prev[TN] = {}, s_next[2][TN] = {};
   auto mfma = [&](const u32x4& a, const u32x4& c, const f32x16& d) {
     if constexpr (F16)
       return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, c), d, 0, 0, 0);
@@ -424,41 +444,53 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     constexpr int u = decltype(U)::value, kk = u / P;
     constexpr bool start = u % P == 0 && (GS == 32 ? kk % 2 == 0 : GS == 64 ? kk == 0 : kk == 0 && decltype(POS)::value == 0);
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
       if constexpr (start) {
 #pragma unroll
-        for (int v = 0; v < 16; ++v) yv[i][v] = fmaf(s_prev, acc[i][v], yv[i][v]);
+        for (int v = 0; v < 16; ++v) yv[i][j][v] = fmaf(s_prev[j], acc[i][j][v], yv[i][j][v]);
         // Pinned here (else the folds sink to where y is next read), and vector and matrix instructions
         // stay on their side, so a block's old sums die before its new ones are born.
-        asm volatile("" : "+v"(yv[i]));
+        asm volatile("" : "+v"(yv[i][j]));
         __builtin_amdgcn_sched_barrier(0x4 | 0x10 | 0x80);
-        acc[i] = mfma(af[u & 1][i], cf[kk & 1], f32x16{});
+        acc[i][j] = mfma(af[u & 1][i], cf[kk & 1][j], f32x16{});
       } else {
-        acc[i] = mfma(af[u & 1][i], cf[kk & 1], acc[i]);
+        acc[i][j] = mfma(af[u & 1][i], cf[kk & 1][j], acc[i][j]);
       }
     }
-    if constexpr (start) s_prev = s_next[GS == 32 ? kk / 2 : 0];
+    if constexpr (start) {
+#pragma unroll
+      for (int j = 0; j < TN; ++j) s_prev[j] = s_next[GS == 32 ? kk / 2 : 0][j];
+    }
   };
   using I0 = std::integral_constant<int, 0>;
   using I1 = std::integral_constant<int, 1>;
-  Batch nb;
+  Batch nb[TN];
+  auto load_batches = [&](int b) {
+#pragma unroll
+    for (int j = 0; j < TN; ++j) load_batch(b, j, nb[j]);
+  };
   // Step t: before its middle barrier the first half of its sub-steps, and (f32) the staging of step
   // t + 1; after it the loads of later steps, the rest, and the first fragments of step t + 1.
   auto step = [&](int t, auto PAR) __attribute__((always_inline)) {
     using NPAR = std::integral_constant<int, 1 - decltype(PAR)::value>;
     const unsigned char* const As = stage_at(t);
     const unsigned char* const An = stage_at(t + 1);
-    if constexpr (GS == 32) {
-      s_next[0] = scale_of(2 * t);
-      s_next[1] = scale_of(2 * t + 1);
-    } else if constexpr (GS == 64 || decltype(PAR)::value == 0) {
-      s_next[0] = scale_of(GS == 64 ? t : t >> 1);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+      if constexpr (GS == 32) {
+        s_next[0][j] = scale_of(j, 2 * t);
+        s_next[1][j] = scale_of(j, 2 * t + 1);
+      } else if constexpr (GS == 64 || decltype(PAR)::value == 0) {
+        s_next[0][j] = scale_of(j, GS == 64 ? t : t >> 1);
+      }
     }
     if constexpr (XF32) stage_x(t + 1, NPAR{});
     auto half1 = [&](auto U) {
       constexpr int u = decltype(U)::value;
       read_a((u + 1) & 1, As, u + 1);
-      if constexpr ((u + 1) % P == 0) cf[((u + 1) / P) & 1] = codes8<BITS, F16>(wc, (u + 1) / P);
+      if constexpr ((u + 1) % P == 0) convert(((u + 1) / P) & 1, (u + 1) / P);
       sub(U, PAR);
     };
     half1(std::integral_constant<int, 0>{});
@@ -470,7 +502,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     // x(t + 1) was issued in step t - 2, whatever its order against w(t + 1); x(t + 2) and w(t + 2) in
     // step t - 1.
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (!XF32) mlxq_vmcnt<NW + A_LD>();
+    if constexpr (!XF32) mlxq_vmcnt<TN * NW + A_LD>();
     strip_barrier();
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (XF32) load_x(t + 2);
@@ -482,7 +514,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     take_w(NPAR{});
     load_w(t + 3, NPAR{});
     read_a(0, An, 0);
-    cf[0] = codes8<BITS, F16>(wc, 0);
+    convert(0, 0);
     sub(std::integral_constant<int, NSUB - 1>{}, PAR);
     __builtin_amdgcn_sched_barrier(0);
     // A pair of groups ends with this step: their X sums were left during the step before, so all are
@@ -490,35 +522,37 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     if (SPP == 1 || decltype(PAR)::value == 1) {
       if ((t + 1) % SPP == 0) bias_pair(t / SPP);
       if ((t + 1) % SPB == 0) {
-        put_tables(nb);
-        load_batch((t + 1) / SPB + 1, nb);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) put_tables(j, nb[j]);
+        load_batches((t + 1) / SPB + 1);
       }
     }
   };
 
   // ---- prologue: batch 0's scales, x and w of the first steps (issued x(0) w(0) x(1) w(1) x(2) w(2)).
-  load_batch(0, nb);
+  load_batches(0);
   if constexpr (XF32) load_x(0);
   else dma_x(0);
   load_w(0, I0{});
   if constexpr (!XF32) dma_x(1);
   load_w(1, I1{});
   if constexpr (!XF32) dma_x(2);
-  put_tables(nb);
+#pragma unroll
+  for (int j = 0; j < TN; ++j) put_tables(j, nb[j]);
   if constexpr (XF32) {
     stage_x(0, I0{});
     load_x(1);
   }
   take_w(I0{});
-  load_batch(1, nb);
+  load_batches(1);
   load_w(2, I0{});
   __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!XF32) mlxq_vmcnt<NW + 2 * A_LD>();  // x(0) is older than w(1), x(1), x(2) and w(2)
+  if constexpr (!XF32) mlxq_vmcnt<TN * NW + 2 * A_LD>();  // x(0) is older than w(1), x(1), x(2) and w(2)
   strip_barrier();
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (!XF32) sum_x(0, I0{});
   read_a(0, lds, 0);
-  cf[0] = codes8<BITS, F16>(wc, 0);
+  convert(0, 0);
   int t = 0;
   for (; t + 1 < T_run; t += 2) {
     step(t, I0{});
@@ -530,7 +564,9 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
-    for (int v = 0; v < 16; ++v) yv[i][v] = fmaf(s_prev, acc[i][v], yv[i][v]);
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) yv[i][j][v] = fmaf(s_prev[j], acc[i][j][v], yv[i][j][v]);
   mlxq_vmcnt<0>();  // no direct-to-LDS load outlives the loop
 
   // ---- K-groups: every wave leaves its partial sums in LDS (over the rings and tables, which all waves
@@ -543,22 +579,24 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     for (int i = 0; i < TM; ++i)
 #pragma unroll
       for (int q = 0; q < 4; ++q)
-        part[wave_all][4 * i + q][lane] = f32x4{yv[i][4 * q], yv[i][4 * q + 1], yv[i][4 * q + 2], yv[i][4 * q + 3]};
+        part[wave_all][4 * i + q][lane] = f32x4{yv[i][0][4 * q], yv[i][0][4 * q + 1], yv[i][0][4 * q + 2], yv[i][0][4 * q + 3]};
     strip_barrier();
   }
 
   // ---- epilogue: lane holds column n and rows m = 32 i + 8 q + 4 half + e: y + bias in f32, the LoRA
   // residual (xa . lbt^T on the f32 matrix cores) times its scale, the activation.
-  const bool n_ok = (int)ncol < rows_n;
-  const int64_t n = bn0 + (n_ok ? (int)ncol : 0);
-  const float bv = epi.bias == nullptr ? -0.0f
-                   : epi.bias_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(epi.bias)[n])
-                                   : static_cast<const float*>(epi.bias)[n];
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(
       y + bm0 * N, (short)0, (int)(uint32_t)(rows_m * N * 4), kStripFlags);
+  // (All blocks' residuals at once, in the registers of acc, made the loop itself spill: 785 -> 953 us.)
   auto finish = [&](auto ACT) {
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int ji = 0; ji < TN * TM; ++ji) {
+      const int j = ji / TM, i = ji % TM;
+      const bool n_ok = (int)ncol[j] < rows_n;
+      const int64_t n = bn0 + (n_ok ? (int)ncol[j] : 0);
+      const float bv = epi.bias == nullptr ? -0.0f
+                       : epi.bias_bf16 ? bf16_bits_to_f32(static_cast<const uint16_t*>(epi.bias)[n])
+                                       : static_cast<const float*>(epi.bias)[n];
       f32x16 r = {};
       if (epi.R > 0) {
         const int mr = 32 * i + r32 < rows_m ? 32 * i + r32 : rows_m - 1;
@@ -582,7 +620,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
 #pragma unroll
           for (int k = 1; k < KS; ++k) o += part[k * NS + wave][4 * i + q][lane];
         } else {
-          o = f32x4{yv[i][4 * q], yv[i][4 * q + 1], yv[i][4 * q + 2], yv[i][4 * q + 3]};
+          o = f32x4{yv[i][j][4 * q], yv[i][j][4 * q + 1], yv[i][j][4 * q + 2], yv[i][j][4 * q + 3]};
         }
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
@@ -602,13 +640,13 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   else finish(std::integral_constant<int, MLXQ_ACT_NONE>{});
 }
 
-template <typename XT, typename SB, int BITS, int GS, int BM, int KS>
+template <typename XT, typename SB, int BITS, int GS, int BM, int KS, int TN = 1>
 static int launch_strip(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                         int64_t N, void* y, const F32Epilogue& epi, hipStream_t st) {
-  constexpr int BN = 256 / KS;
+  constexpr int BN = 256 / KS * TN;
   const int64_t tiles = ((M + BM - 1) / BM) * ((N + BN - 1) / BN);
   if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "qmm_f32: problem too large");
-  hipLaunchKernelGGL((qmm_f32_strip_kernel<XT, SB, BITS, GS, BM, KS>), dim3((unsigned)tiles), dim3(512), 0, st,
+  hipLaunchKernelGGL((qmm_f32_strip_kernel<XT, SB, BITS, GS, BM, KS, TN>), dim3((unsigned)tiles), dim3(512), 0, st,
                      (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N, (float*)y, epi);
   return check_launch("qmm_f32");
 }
@@ -645,7 +683,18 @@ template <typename XT, typename SB, int BITS, int GS>
 static int strip_tile(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b, int64_t N,
                       void* y, const F32Epilogue& epi, hipStream_t st) {
   switch (strip_shape(M, K, N, GS, std::is_same<XT, float>::value)) {
-    case 0: return launch_strip<XT, SB, BITS, GS, 128, 1>(x, M, K, wq, s, b, N, y, epi, st);
+    case 0:
+      // f32 activations, Q4, more than a round and a half of tiles: 64 x 512 instead of 128 x 256, two
+      // strips per wave.  Both activation parts are then read from LDS for two strips' MFMAs instead of
+      // one (half the LDS reads), for twice the code conversions.  Same-process A/B, 128 x 256 ->
+      // 64 x 512: 4608 x 3072 x 12288 694 -> 648 us, 4608 x 12288 x 3072 748 -> 713, 4608 x 3072 x 3072
+      // g128 175 -> 164; 1024 x 3072 x 12288 (1.5 rounds) 171 -> 174.  Q8 needs twice the weight
+      // registers and spills (4608 x 3072 x 9216 597 -> 630); fp16's one pass has no second use.
+      if constexpr (std::is_same<XT, float>::value && BITS == 4) {
+        if (((M + 63) / 64) * ((N + 511) / 512) * 2 > device_cu_count() * 3)
+          return launch_strip<XT, SB, BITS, GS, 64, 1, 2>(x, M, K, wq, s, b, N, y, epi, st);
+      }
+      return launch_strip<XT, SB, BITS, GS, 128, 1>(x, M, K, wq, s, b, N, y, epi, st);
     case 1: return launch_strip<XT, SB, BITS, GS, 64, 1>(x, M, K, wq, s, b, N, y, epi, st);
     case 2: return launch_strip<XT, SB, BITS, GS, 64, 2>(x, M, K, wq, s, b, N, y, epi, st);
     default: return launch_strip<XT, SB, BITS, GS, 32, 4>(x, M, K, wq, s, b, N, y, epi, st);

@@ -68,7 +68,7 @@ def _check(mlxq, x, pack, gs, bits, what, **kw):
     # start mid-word), 64-row tiles in two groups, and grids that fill the CUs
     (33, 63, 256, 64, 4), (32, 65, 320, 64, 8), (40, 200, 448, 64, 4), (9, 4096, 1152, 128, 4), (77, 5120, 1280, 64, 8),
     (256, 3000, 704, 64, 4), (250, 2100, 832, 32, 8), (512, 2048, 1536, 128, 8),
-    (4224, 2100, 320, 64, 4), (6200, 1030, 384, 128, 8), (3000, 2600, 128, 32, 4),
+    (4224, 2100, 320, 64, 4), (5000, 2600, 576, 64, 4), (6100, 2050, 2176, 128, 4), (4100, 3100, 192, 32, 4), (6200, 1030, 384, 128, 8), (3000, 2600, 128, 32, 4),
 ])
 def test_strip_edges(mlxq, xdt, sb, M, N, K, gs, bits):
     banner("strip", xdt, sb, M, N, K, gs, bits)
