@@ -523,10 +523,13 @@ int mlxq_qmm_experts(const void* x, int x_dtype, int x_per_expert, int64_t E, in
   bat.y = M * N;
   bat.bias = N;
   hipStream_t st = (hipStream_t)stream;
+  const bool aligned = (M * N * yb) % 16 == 0 && (bat.sb * sbb) % 4 == 0;  // every expert's y and scales slices
   // All experts in one launch of the wide GEMM (grid.y = expert) when it applies: per-expert
   // problems of an encoder batch are a few dozen tiles each, too few to fill 256 CUs alone.
   const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256);
-  if (d0_bf16 && M > 8 && K % 64 == 0 && E * tiles >= 128 && E <= 65535 &&
+  const bool small = d0_bf16 && M > 8 && M <= 64 && K % 64 == 0 && K >= 512 && E <= 65535 && aligned &&
+                     qmm_small_fits(M, K, N, group_size, bits, sbb);
+  if (!small && d0_bf16 && M > 8 && K % 64 == 0 && E * tiles >= 128 && E <= 65535 &&
       qmm_wide_fits(M, K, N, group_size, bits, sbb)) {
     const QmmEpilogue qe = {(const uint16_t*)bias, nullptr, nullptr, 0, 1.0f, kFusedActNone, nullptr};
     return run_qmm_wide(x, M, K, wq, scales, biases, sb_dtype, N, group_size, bits, y, qe, st, bat);
@@ -534,12 +537,20 @@ int mlxq_qmm_experts(const void* x, int x_dtype, int x_per_expert, int64_t E, in
   // Otherwise expert by expert through the single-matrix paths (same rounding points; no
   // workspace: without LoRA nothing is staged and the result never promotes past D0).  Each
   // expert's slices must meet mlxq_linear's alignment: y 16 bytes, scales and biases 4 bytes.
-  if (E > 1 && ((M * N * yb) % 16 != 0 || (bat.sb * sbb) % 4 != 0))
+  if (E > 1 && !aligned)
     return set_error(MLXQ_EUNSUPPORTED,
                      "qmm_experts: expert by expert, each expert's y slice (M*N = %lld elements of %d "
                      "bytes) must be a multiple of 16 bytes and its scales/biases slice (N*K/group_size "
                      "= %lld of %d bytes) a multiple of 4 bytes; run such packs one expert at a time "
                      "on aligned copies", (long long)(M * N), yb, (long long)bat.sb, sbb);
+  // In bf16 those paths take every expert in one launch too: the GEMV, and up to 64 rows the K-split
+  // GEMM, whose 64-row tile dequantizes each weight once.
+  if (small) {
+    const QmmEpilogue qe = {(const uint16_t*)bias, nullptr, nullptr, 0, 1.0f, kFusedActNone, nullptr};
+    return run_qmm_small(x, M, K, wq, scales, biases, sb_dtype, N, group_size, bits, y, qe, st, bat);
+  }
+  if (d0_bf16 && M <= 8 && E <= 65535 && qmv_mfma_applicable(x_dtype, sb_dtype, M, K, N, group_size, bits))
+    return run_qmv_mfma(x, M, K, wq, scales, biases, N, group_size, bits, y, st, (const uint16_t*)bias, nullptr, bat);
   for (int64_t e = 0; e < E; ++e) {
     mlxq_epilogue ep = {};
     ep.bias = bias ? (const char*)bias + e * bat.bias * bb : nullptr;

@@ -80,7 +80,7 @@ bool qmm_wide_sb_reach(const void* scales, const void* biases, int64_t bytes, in
 bool qmm_small_fits(int64_t M, int64_t K, int64_t N, int gs, int bits, int sb_bytes);
 int run_qmm_small(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                   const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y,
-                  const QmmEpilogue& epi, hipStream_t st);
+                  const QmmEpilogue& epi, hipStream_t st, const QmmBatch& bat = QmmBatch{});
 int run_qmm_wide(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                  int sb_dtype, int64_t N, int gs, int bits, void* y, const QmmEpilogue& epi,
                  hipStream_t st, const QmmBatch& batch = QmmBatch{});
@@ -89,7 +89,7 @@ bool qmv_mfma_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_
 // product, one rounding per op.
 int run_qmv_mfma(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                  int64_t N, int gs, int bits, void* y, hipStream_t st, const uint16_t* bias = nullptr,
-                 const uint16_t* act_table = nullptr);
+                 const uint16_t* act_table = nullptr, const QmmBatch& bat = QmmBatch{});
 bool swiglu_qmv_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_t F, int gs, int bits);
 int run_swiglu_qmv(const void* x, int64_t M, int64_t K, const uint32_t* wq_g, const void* s_g,
                    const void* b_g, const uint32_t* wq_u, const void* s_u, const void* b_u, int64_t F,

@@ -42,7 +42,17 @@ template <typename SB, int BITS, int GS, int EPI, bool SZS, int kWaves>
 __global__ __launch_bounds__(kWaves * 64, 1) void qmm_small_kernel(
     const uint16_t* __restrict__ x, int64_t M, int64_t K, const uint32_t* __restrict__ wq,
     const SB* __restrict__ scales, const SB* __restrict__ biases, int64_t N,
-    uint16_t* __restrict__ y, QmmEpilogue epi) {
+    uint16_t* __restrict__ y, QmmEpilogue epi, QmmBatch bat) {
+  // Stacked launch: grid.y selects the matrix (expert); one matrix has all strides zero.
+  if (gridDim.y > 1) {
+    const int64_t e = blockIdx.y;
+    x += e * bat.x;
+    wq += e * bat.w;
+    scales += e * bat.sb;
+    biases += e * bat.sb;
+    y += e * bat.y;
+    if (epi.bias) epi.bias += e * bat.bias;
+  }
   constexpr bool FUSED = EPI != 0;
   constexpr int ACT = FUSED ? EPI - 1 : kFusedActNone;
   constexpr int WPL = BITS;  // packed words per lane per sub-tile per K step
@@ -320,7 +330,8 @@ __global__ __launch_bounds__(kWaves * 64, 1) void qmm_small_kernel(
 
 template <typename SB, int BITS, int GS>
 static int launch_small(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
-                        const void* b, int64_t N, void* y, const QmmEpilogue& epi, hipStream_t st) {
+                        const void* b, int64_t N, void* y, const QmmEpilogue& epi, hipStream_t st,
+                        const QmmBatch& bat) {
   const int64_t tiles = ((M + kTile - 1) / kTile) * ((N + kTile - 1) / kTile);
   const bool fused = epi.bias || epi.rank16 || epi.act != kFusedActNone;
   const int kind = fused ? 1 + epi.act : 0;
@@ -334,11 +345,11 @@ static int launch_small(const void* x, int64_t M, int64_t K, const uint32_t* wq,
   // stated: 333 x 3072 x 4096 (384 tiles) 27.8 -> 24.0 us, 256 x 3072 x 4608 (288) 26.7 -> 22.6,
   // 320 x 4096 x 4096 Q8 (320) 40.0 -> 35.6, 200 x 2048 x 8192 g32 (512) 22.7 -> 19.7, 300 x 2880 x
   // 5000 (395) 31.6 -> 29.5; with a tile per CU eight stay ahead (each walks half the K steps).
-  const bool four = tiles > device_cu_count();
+  const bool four = tiles * bat.count > device_cu_count();
 #define MLXQ_SLW(E, Z, W)                                                                             \
-  hipLaunchKernelGGL((qmm_small_kernel<SB, BITS, GS, E, Z, W>), dim3((unsigned)tiles), dim3(W * 64),  \
+  hipLaunchKernelGGL((qmm_small_kernel<SB, BITS, GS, E, Z, W>), dim3((unsigned)tiles, (unsigned)bat.count), dim3(W * 64), \
                      0, st, (const uint16_t*)x, M, K, wq, (const SB*)s, (const SB*)b, N,               \
-                     (uint16_t*)y, epi)
+                     (uint16_t*)y, epi, bat)
 #define MLXQ_SL(E, Z)               \
   do {                              \
     if (four) MLXQ_SLW(E, Z, 4);    \
@@ -376,10 +387,10 @@ bool qmm_small_fits(int64_t M, int64_t K, int64_t N, int gs, int bits, int sb_by
 
 int run_qmm_small(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                   const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y,
-                  const QmmEpilogue& epi, hipStream_t st) {
+                  const QmmEpilogue& epi, hipStream_t st, const QmmBatch& bat) {
   if (M == 0 || N == 0) return MLXQ_OK;
 #define MLXQ_SM(SB, B, G) \
-  if (bits == B && gs == G) return launch_small<SB, B, G>(x, M, K, wq, s, b, N, y, epi, st);
+  if (bits == B && gs == G) return launch_small<SB, B, G>(x, M, K, wq, s, b, N, y, epi, st, bat);
   if (sb_dtype == MLXQ_BFLOAT16) {
     MLXQ_SM(uint16_t, 4, 32) MLXQ_SM(uint16_t, 4, 64) MLXQ_SM(uint16_t, 4, 128)
     MLXQ_SM(uint16_t, 8, 32) MLXQ_SM(uint16_t, 8, 64) MLXQ_SM(uint16_t, 8, 128)

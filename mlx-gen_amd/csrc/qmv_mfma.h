@@ -156,8 +156,8 @@ __host__ __device__ constexpr int qmv_wave_lds(int bits, int gs, int steps, int 
 // sums are zero, whatever codes the weight loads find past the row's end) and so do the scales
 // and biases of groups past the row's end.
 // Contract of every kernel built from it (checked on the host by qmv_plan):
-// 1 <= M <= MR, K % (512/BITS) == 0, K % group == 0, bf16 scales and biases, the row's
-// K*BITS/512 load steps covered by the waves of one matrix (T each, the last wave's range may end
+// 1 <= M <= MR, K % group == 0, bf16 scales and biases, the row's
+// load steps (ceil(K*BITS/512)) covered by the waves of one matrix (T each, the last wave's range may end
 // past K), dynamic LDS of at least the operands and the partial sums (QmvPlan::lds, qmv_multi_lds), every
 // buffer < 2 GiB.
 template <int BITS, int GS, int STEPS, int MR, int T>
@@ -435,8 +435,18 @@ __global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
     const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
     const uint32_t* __restrict__ wq2, const uint16_t* __restrict__ scales2,
     const uint16_t* __restrict__ biases2, int N, int rows, uint16_t* __restrict__ y,
-    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table) {
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table, QmmBatch bat) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+  // Stacked launch: grid.y selects the matrix (expert); one matrix has all strides zero.
+  if (gridDim.y > 1) {
+    const int64_t e = blockIdx.y;
+    x += e * bat.x;
+    wq += e * bat.w;
+    scales += e * bat.sb;
+    biases += e * bat.sb;
+    y += e * bat.y;
+    if (bias) bias += e * bat.bias;
+  }
   const int NT = blockDim.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -544,6 +554,11 @@ constexpr bool qmv_multi_built(int bits, int gs, int steps, int mr, int nmat, in
 // workgroup fills a CU on its own (128 registers per wave).  12 against 8: the down GEMV
 // (K = 8192) 6.10 -> 5.84 us, gate (K = 3072) 5.40 -> 5.28 us, SwiGLU unchanged; 16 was no better.
 //
+// A row whose bytes are no multiple of 64 (K = 2880 in Q4: 22.5 load steps) ends inside its last load
+// step; the codes past its end are the next row's and fold to zero like those of a padded step.
+// Such rows had run on the VALU kernel: [4, 2880] x Q4 g64 [2880, 2880]^T 11.2 -> 4.2 us, [6, 736] x Q8
+// g32 [711, 736]^T 11.2 -> 3.7.
+//
 // When no count divides the row's load steps within those limits (K = 11008: 86 steps of Q4),
 // the waves take ceil(steps / waves) each and the last one's range ends past K (cost as above,
 // then the fewest padded steps); failing that, each wave takes two rounds of its load registers
@@ -553,7 +568,7 @@ constexpr bool qmv_multi_built(int bits, int gs, int steps, int mr, int nmat, in
 // stream the weights M times and lose to it).
 inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, QmvPlan& p) {
   const int64_t cpl = 512 / bits;
-  const int64_t LS = K / cpl;
+  const int64_t LS = (K + cpl - 1) / cpl;
   const int mr = M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8));
   for (int pass = 0; pass < 3; ++pass) {  // exact; ragged; ragged with two rounds
     const int ring = pass == 2 ? 2 : 1;
@@ -586,8 +601,7 @@ inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, QmvP
 inline bool qmv_plan(int64_t M, int64_t K, int gs, int bits, int nmat, QmvPlan& p) {
   if (M < 1 || M > 8 || (bits != 4 && bits != 8)) return false;
   if (gs != 32 && gs != 64 && gs != 128) return false;
-  const int64_t cpl = 512 / bits;
-  if (K <= 0 || K % cpl != 0 || K % gs != 0) return false;
+  if (K <= 0 || K % gs != 0) return false;
   if (qmv_plan_rows(M, K, gs, bits, nmat, p)) return true;
   for (int rows : {4, 2})  // launches of fewer rows
     if (M > rows && qmv_plan_rows(rows, K, gs, bits, nmat, p)) return true;
@@ -605,6 +619,7 @@ struct QmvArgs {
   void* y;
   const uint16_t* bias = nullptr;       // one matrix: the bf16 epilogue (gemv_finish)
   const uint16_t* act_table = nullptr;
+  QmmBatch bat;                         // one matrix: several of the same shape (grid.y)
 };
 
 // Rows per workgroup of one tile: 16 for SwiGLU; for one matrix, of 16, 12 and 8 the count whose
@@ -644,8 +659,8 @@ inline int qmv_multi_rows(const QmvArgs& a, const QmvPlan& p) {
   int64_t per_cu = kMaxWaves / p.waves;
   if (kMaxLds / lds < per_cu) per_cu = kMaxLds / lds;
   const int64_t wgs = device_cu_count() * (per_cu > 0 ? per_cu : 1);
-  const int64_t rows = (a.N + wgs - 1) / wgs;
-  return rows >= 32 ? (int)rows : 0;
+  const int64_t rows = (a.N * a.bat.count + wgs - 1) / wgs;
+  return rows >= 32 ? (int)(rows < a.N ? rows : a.N) : 0;
 }
 
 template <int BITS, int GS, int STEPS, int MR, int NMAT, int RING, bool MULTI>
@@ -661,10 +676,10 @@ static int launch_qmv_mfma(const QmvArgs& a, const QmvPlan& p, int rows, hipStre
       return set_error(MLXQ_EDEVICE, "qmv: hipFuncSetAttribute failed");
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL((qmv_mfma_kernel<BITS, GS, STEPS, MR, NMAT, RING, MULTI>), dim3((unsigned)((a.N + rows - 1) / rows)),
+  hipLaunchKernelGGL((qmv_mfma_kernel<BITS, GS, STEPS, MR, NMAT, RING, MULTI>), dim3((unsigned)((a.N + rows - 1) / rows), (unsigned)a.bat.count),
                      dim3(p.waves * 64), MULTI ? qmv_multi_lds(p) : p.lds, st, (const uint16_t*)a.x, (int)a.M, (int)a.K, a.wq,
                      (const uint16_t*)a.s, (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2,
-                     (const uint16_t*)a.b2, (int)a.N, rows, (uint16_t*)a.y, a.bias, a.act_table);
+                     (const uint16_t*)a.b2, (int)a.N, rows, (uint16_t*)a.y, a.bias, a.act_table, a.bat);
   return check_launch(NMAT == 2 ? "swiglu_qmv" : "qmv_mfma");
 }
 

@@ -64,7 +64,17 @@ __global__ __launch_bounds__(1024) void qmv_row_kernel(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint32_t* __restrict__ wq2,
     const uint16_t* __restrict__ scales2, const uint16_t* __restrict__ biases2, int K, int N,
-    uint16_t* __restrict__ y, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table) {
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table, QmmBatch bat) {
+  // Stacked launch: grid.y selects the matrix (expert); one matrix has all strides zero.
+  if (gridDim.y > 1) {
+    const int64_t e = blockIdx.y;
+    x += e * bat.x;
+    wq += e * bat.w;
+    scales += e * bat.sb;
+    biases += e * bat.sb;
+    y += e * bat.y;
+    if (bias) bias += e * bat.bias;
+  }
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int C = 16 * LS;                  // 64-code columns per row, padded to whole loads
   constexpr int G = G64 ? C : C / 2;          // groups per padded row (table entries)
@@ -321,10 +331,10 @@ static int launch_qmv_row(const QmvArgs& a, hipStream_t st) {
   }
   const int wpb = qmv_row_wpb(a.N, NMAT);
   const int lds = qmv_row_lds(LS, G64, NMAT, wpb);
-  hipLaunchKernelGGL((qmv_row_kernel<G64, LS, NMAT, VALU>), dim3((unsigned)((a.N + wpb - 1) / wpb)),
+  hipLaunchKernelGGL((qmv_row_kernel<G64, LS, NMAT, VALU>), dim3((unsigned)((a.N + wpb - 1) / wpb), (unsigned)a.bat.count),
                      dim3(wpb * 64), lds, st, (const uint16_t*)a.x, a.wq, (const uint16_t*)a.s,
                      (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2, (const uint16_t*)a.b2, (int)a.K,
-                     (int)a.N, (uint16_t*)a.y, a.bias, a.act_table);
+                     (int)a.N, (uint16_t*)a.y, a.bias, a.act_table, a.bat);
   return check_launch(NMAT == 2 ? "swiglu_qmv_row" : VALU ? "qmv_row_valu" : "qmv_row");
 }
 
@@ -354,8 +364,9 @@ bool qmv_mfma_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_
 }
 
 int run_qmv_mfma(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
-                 int64_t N, int gs, int bits, void* y, hipStream_t st, const uint16_t* bias, const uint16_t* act_table) {
-  const QmvArgs a = {x, M, K, N, wq, s, b, nullptr, nullptr, nullptr, y, bias, act_table};
+                 int64_t N, int gs, int bits, void* y, hipStream_t st, const uint16_t* bias, const uint16_t* act_table,
+                 const QmmBatch& bat) {
+  const QmvArgs a = {x, M, K, N, wq, s, b, nullptr, nullptr, nullptr, y, bias, act_table, bat};
   if (qmv_row_fits(M, K, gs, bits, 1)) return qmv_row<1>(a, gs, st);
   QmvPlan p;
   if (!qmv_plan(M, K, gs, bits, 1, p))
@@ -364,7 +375,7 @@ int run_qmv_mfma(const void* x, int64_t M, int64_t K, const uint32_t* wq, const 
   for (int64_t m0 = 0; m0 < M; m0 += p.rows) {  // launches of p.rows activation rows
     const int64_t rows = M - m0 < p.rows ? M - m0 : p.rows;
     const int rc = run_qmv_mfma(static_cast<const uint16_t*>(x) + m0 * K, rows, K, wq, s, b, N, gs, bits,
-                                static_cast<uint16_t*>(y) + m0 * N, st, bias, act_table);
+                                static_cast<uint16_t*>(y) + m0 * N, st, bias, act_table, bat);
     if (rc != MLXQ_OK) return rc;
   }
   return MLXQ_OK;
@@ -388,6 +399,8 @@ int run_qmv_row_valu(const void* x, int64_t K, const uint32_t* wq, const void* s
 
 bool swiglu_qmv_applicable(int x_dtype, int sb_dtype, int64_t M, int64_t K, int64_t F, int gs, int bits) {
   if (x_dtype != MLXQ_BFLOAT16 || sb_dtype != MLXQ_BFLOAT16 || !buffers_fit(M, K, F)) return false;
+  if (bits != 4 && bits != 8) return false;
+  if (K % (512 / bits) != 0) return false;  // the fused form's stated condition
   QmvPlan p;
   return qmv_row_fits(M, K, gs, bits, 2) || qmv_plan(M, K, gs, bits, 2, p);
 }

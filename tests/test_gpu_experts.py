@@ -121,3 +121,28 @@ def test_experts_empty_and_mismatch(mlxq):
     with pytest.raises(mlxq.MlxqError, match="lead with E"):
         mlxq.qmm_experts(to_gpu(bf16_normal(rng, (3, 4, 128))), wq_to_gpu(wq), to_gpu(s), to_gpu(b),
                          64, 4, per_expert=True)
+
+
+@pytest.mark.parametrize("per_expert", [False, True])
+@pytest.mark.parametrize("E,M,N,K,gs,bits", [
+    (3, 1, 72, 1152, 64, 4), (5, 1, 40, 192, 32, 8), (4, 3, 88, 384, 128, 4), (7, 8, 1000, 512, 64, 8),
+    (33, 4, 600, 1024, 64, 4), (6, 7, 64, 11008, 64, 4), (3, 9, 72, 512, 64, 4), (5, 64, 136, 640, 32, 8),
+    (9, 33, 1032, 2880, 64, 4),
+])
+def test_experts_one_launch_small_batches(mlxq, per_expert, E, M, N, K, gs, bits):
+    """Up to 8 rows (GEMV) and up to 64 (K-split GEMM) in one launch over grid.y: every expert bit for
+    bit its own linear with that bias, in one-row, one-tile, several-tile and split-row forms."""
+    banner("experts small batches", per_expert, E, M, N, K, gs, bits)
+    g = torch.Generator(device="cuda").manual_seed(E + M)
+    wq = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), generator=g, device="cuda", dtype=torch.int32)
+    mk = lambda shape, std: (torch.randn(shape, generator=g, device="cuda") * std).to(torch.bfloat16)  # noqa: E731
+    s, b, bias = mk((E, N, K // gs), 0.01), mk((E, N, K // gs), 0.05), mk((E, N), 0.5)
+    x = mk((E, M, K) if per_expert else (M, K), 1.0)
+    y = mlxq.qmm_experts(x, wq, s, b, gs, bits, bias=bias, per_expert=per_expert)
+    plain = mlxq.qmm_experts(x, wq, s, b, gs, bits, per_expert=per_expert)
+    for e in range(E):
+        xe = x[e] if per_expert else x
+        one = [t[e].contiguous() for t in (wq, s, b)]
+        if M <= 8 or K >= 512 and (M + 127) // 128 * ((N + 127) // 128) < 136:
+            assert torch.equal(y[e], mlxq.linear(xe, *one, gs, bits, bias=bias[e].contiguous()))
+            assert torch.equal(plain[e], mlxq.linear(xe, *one, gs, bits))
