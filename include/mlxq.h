@@ -150,7 +150,7 @@ int mlxq_qmv(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* w
 
 /* A GEMV on the VALU only (no matrix cores); any x / scales dtype; 1 <= M <= 8; y in
  * promote(x_dtype, sb_dtype).  The VALU GEMV with exact f32 dequant (the kernel quantized_matmul
- * uses for f32 operands and group size 32), except at M = 1 with bf16 x and scales, Q4, group
+ * uses for f32 operands), except at M = 1 with bf16 x and scales, Q4, group
  * 64/128 and K <= 8192, where it is the M = 1 matrix-core kernel's loads and fold with VALU dot
  * products.  Forced here so it can be measured against the matrix-core GEMV on bf16 decode
  * shapes. */
@@ -231,11 +231,12 @@ int mlxq_linear_noalloc(const void* x, int x_dtype, int64_t M, int64_t K, const 
  * f32 bias over a bf16 product would need a promoted second pass and returns MLXQ_EUNSUPPORTED.
  * x is [M, K] shared by every expert when x_per_expert == 0 (the gate_up projection of
  * gpt_oss.rs:702), else [E, M, K] (the down projection of :714).  Each expert's result equals the
- * single-matrix mlxq_linear with that bias.  bf16 x and scales with M > 8, K a multiple of 64 and at
- * least 128 GEMM tiles over all experts run every expert in one launch; otherwise the experts run
- * one after another through mlxq_linear, which needs each expert's slices aligned: M*N elements of
- * y a multiple of 16 bytes and N*K/group_size scales (biases) a multiple of 4 bytes, else
- * MLXQ_EUNSUPPORTED (the Python and C++ hosts then run those experts on aligned copies).
+ * single-matrix mlxq_linear with that bias.  bf16 x and scales run every expert in one launch with
+ * M <= 8 (the GEMV's shapes), with M <= 64, K a multiple of 64 and K >= 512, and with K a multiple of
+ * 64 and at least 128 GEMM tiles over all experts; otherwise the experts run one after another
+ * through mlxq_linear.  All but the last of these need each expert's slices aligned: M*N elements of
+ * y a multiple of 16 bytes and N*K/group_size scales (biases) a multiple of 4 bytes; shapes that none
+ * then takes return MLXQ_EUNSUPPORTED (the Python and C++ hosts run those experts on aligned copies).
  */
 int mlxq_qmm_experts(const void* x, int x_dtype, int x_per_expert, int64_t E, int64_t M, int64_t K,
                      const uint32_t* wq, const void* scales, const void* biases, int sb_dtype,

@@ -7,8 +7,8 @@
 // When M x N gives few tiles, a tile kernel leaves most CUs idle and each workgroup walks all of
 // K one latency-bound step after another.  Here a workgroup of 8 waves (4 when the
 // tiles outnumber the CUs) owns a 64x64 output tile and the waves split K: wave w of W takes K steps
-// [w*KT/W, (w+1)*KT/W), so a tile has W independent load chains of KT/W steps instead of one of KT.  Each wave moves its activation
-// rows global -> LDS with direct-to-LDS loads one step ahead (a private 2-stage ring, 8 rows x
+// [w*KT/W, (w+1)*KT/W), so a tile has W independent load chains of KT/W steps instead of one of KT.
+// Each wave moves its activation rows global -> LDS with direct-to-LDS loads one step ahead (a private 2-stage ring, 8 rows x
 // 128 bytes per load, i.e. whole cache lines) and reads MFMA fragments back with ds_read_b128;
 // its weight fragments go straight into registers two steps ahead.  The partial tiles meet
 // in LDS (over the rings) and are added in wave order (deterministic); waves 0-3 then finish one
