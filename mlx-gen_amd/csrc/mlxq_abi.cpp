@@ -615,7 +615,7 @@ int mlxq_linear(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t
   // An f32 product at GEMM size fuses the bias, an f32 LoRA residual and the activation (all in
   // f32); a bf16 residual (bf16 x and factors against f32 scales) and the shapes of the three-pass
   // kernel need the elementwise epilogue.
-  if (!p.d0_bf16 && M > 8 && (!p.lora || (!p.dr_bf16 && qmm_f32_strip_fits(K, N)))) {
+  if (!p.d0_bf16 && M > 8 && (!p.lora || (!p.dr_bf16 && qmm_f32_strip_fits(x_dtype, K, N, group_size)))) {
     F32Epilogue fe;
     fe.bias = p.bias ? ep->bias : nullptr;
     fe.bias_bf16 = p.bias && ep->bias_dtype == MLXQ_BFLOAT16;

@@ -122,7 +122,7 @@ struct F32Epilogue {
 int run_qmm_f32(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                 const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, hipStream_t st,
                 const F32Epilogue& epi = F32Epilogue{});
-bool qmm_f32_strip_fits(int64_t K, int64_t N);
+bool qmm_f32_strip_fits(int x_dtype, int64_t K, int64_t N, int gs);
 int run_qmm_f32_strip(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                       const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, const F32Epilogue& epi,
                       hipStream_t st);

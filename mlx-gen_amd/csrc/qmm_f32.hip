@@ -16,9 +16,10 @@
 // bf16 product.  With bf16 activations (f32 scales) x_lo is zero and the third pass is skipped;
 // fp16 activations split exactly (x_hi + x_lo == x).
 // Weights are dequantized exactly as fma(code, scale, bias) in f32 (scale and bias widened
-// exactly from bf16), then split.  This kernel serves K % 64 == 32 (group size 32), widths past the
-// factored kernel's reach and the LoKr dense product; everything else takes the factored kernel
-// (qmm_f32_strip.hip: the codes themselves as exact operands, one pass for fp16 x, two for f32 x).
+// exactly from bf16), then split.  This kernel serves f32 x at group size 32, K % 64 == 32 (group
+// size 32 too), widths past the factored kernel's reach and the LoKr dense product; everything else
+// takes the factored kernel (qmm_f32_strip.h: the codes themselves as exact operands, one pass for
+// 16-bit x, two for f32 x).
 //
 // Structure: a workgroup of 8 waves (2 x 4, 64 x 64 each) per 128 x 256 output tile (the LoKr
 // dense product: 4 waves, 2 x 2, per 128 x 128 tile), K advanced BK = 32 at a time through a
@@ -472,7 +473,7 @@ int run_qmm_f32(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t
                 const F32Epilogue& epi) {
   if (x_dtype == MLXQ_BFLOAT16 && sb_dtype == MLXQ_BFLOAT16)
     return set_error(MLXQ_EINVAL, "qmm_f32: bf16 operands take the bf16 GEMM");
-  if (qmm_f32_strip_fits(K, N))
+  if (qmm_f32_strip_fits(x_dtype, K, N, gs))
     return run_qmm_f32_strip(x, x_dtype, M, K, wq, s, b, sb_dtype, N, gs, bits, y, epi, st);
   if (epi.R > 0) return set_error(MLXQ_EINVAL, "qmm_f32: the three-pass kernel fuses no LoRA residual");
   if (x_dtype == MLXQ_FLOAT32) {

@@ -704,8 +704,9 @@ static int strip_tile(const void* x, int64_t M, int64_t K, const uint32_t* wq, c
 template <typename XT, typename SB>
 static int strip_bits_gs(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
                          int64_t N, int gs, int bits, void* y, const F32Epilogue& epi, hipStream_t st) {
-#define MLXQ_ST(B, G) \
-  if (bits == B && gs == G) return strip_tile<XT, SB, B, G>(x, M, K, wq, s, b, N, y, epi, st);
+#define MLXQ_ST(B, G)                                          \
+  if constexpr (!(std::is_same<XT, float>::value && G == 32)) \
+    if (bits == B && gs == G) return strip_tile<XT, SB, B, G>(x, M, K, wq, s, b, N, y, epi, st);
   MLXQ_ST(4, 32) MLXQ_ST(4, 64) MLXQ_ST(4, 128) MLXQ_ST(8, 32) MLXQ_ST(8, 64) MLXQ_ST(8, 128)
 #undef MLXQ_ST
   return set_error(MLXQ_EINVAL, "qmm_f32: unsupported bits=%d group_size=%d", bits, gs);
