@@ -47,6 +47,8 @@ namespace {
 
 constexpr int kStripGroupM = 8;  // M-tiles per group of the tile order
 constexpr int kStripFlags = 0x00020000;  // raw buffer resource word 3 for gfx9-family loads
+// Added to an activation offset (below 2^31: 128 rows of less than 2^24 bytes), past the tile's rows: zero.
+constexpr uint32_t kStripPast = 0x80000000u;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
@@ -177,7 +179,8 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   const uint32_t kwords = (uint32_t)(K * BITS / 32);
   const int groups_all = (int)(K / GS);
   // This K-group's steps [t0, t0 + T), whole groups; every group runs T_run steps, the ones past its own
-  // on repeated operands with zero scales.
+  // on zero activations with zero scales (with the last step's activations, an infinity among them would
+  // fold as 0 * inf).
   constexpr int UNIT = GS == 128 ? 2 : 1;  // steps
   const int units = (int)(K / (64 * UNIT));
   const int t0 = UNIT * (kg * units / KS), T = UNIT * ((kg + 1) * units / KS) - t0;
@@ -209,23 +212,23 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
   auto dma_x = [&](int t) {  // !XF32
 #if defined(__HIP_DEVICE_COMPILE__)
     unsigned char* const base = stage_at(t);
-    const uint32_t tc = (uint32_t)(t < T ? t : T - 1);
+    const uint32_t at = t < T ? (uint32_t)t * 128u : kStripPast;
 #pragma unroll
     for (int i = 0; i < A_LD; ++i)
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (__attribute__((address_space(3))) void*)(base + (A_ROWS * i + 8 * wave) * 128),
-                                               16, x_off[i] + tc * 128u, 0, 0, 0);
+                                               16, x_off[i] + at, 0, 0, 0);
 #else
     (void)t;
 #endif
   };
   u32x4 xr[XF32 ? A_LD : 1][2];
   auto load_x = [&](int t) {  // XF32
-    const uint32_t tc = (uint32_t)(t < T ? t : T - 1);
+    const uint32_t at = t < T ? (uint32_t)t * 256u : kStripPast;
 #pragma unroll
     for (int i = 0; i < A_LD; ++i)
 #pragma unroll
       for (int q = 0; q < 2; ++q)
-        xr[i][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, x_off[i] + tc * 256u + 16u * q, 0, 0));
+        xr[i][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, x_off[i] + at + 16u * q, 0, 0));
   };
   float* const xtab = reinterpret_cast<float*>(lds + OFF_X);
   constexpr int XPASS = BM / NS > 16 ? BM / NS / 16 : 1;

@@ -124,3 +124,26 @@ def test_strip_bias_lora_act(mlxq, xdt, fdt, act, rank, M, N):
     rel = ((got.double() - p).norm() / p.norm()).item()
     print(f"    rel {rel:.2e}", flush=True)
     assert rel < 2e-6
+
+
+@pytest.mark.parametrize("xdt", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K,gs,bits", [(33, 65, 320, 64, 4), (40, 200, 448, 64, 8), (20, 64, 704, 64, 4), (40, 70, 832, 32, 4),
+                                           (9, 4096, 1152, 128, 4), (250, 2100, 832, 32, 8)])
+def test_strip_infinity_in_uneven_k_groups(mlxq, xdt, M, N, K, gs, bits):
+    """K shared unevenly among a workgroup's K-groups: an infinity anywhere in a row of positive activations
+    against positive codes, scales and biases gives infinities, not the NaN of a step that a shorter share
+    runs besides."""
+    banner("strip infinity", xdt, M, N, K, gs, bits)
+    rng = np.random.default_rng(K)
+    _, wq, s, b = _pack(rng, N, K, gs, bits, "f32")
+    wq, s, b = wq | (0x11111111 if bits == 4 else 0x01010101), s.abs() + 0.5, b.abs() + 0.25
+    x = torch.from_numpy(rng.uniform(0.5, 1.5, (M, K)).astype(np.float32)).to("cuda").to(DT[xdt])
+    clean = mlxq.linear(x, wq, s, b, gs, bits)
+    for i, k in enumerate(range(0, K, 16)):
+        row = i % M
+        x2 = x.clone()
+        x2[row, k] = float("inf")
+        y = mlxq.linear(x2, wq, s, b, gs, bits)
+        assert bool((y[row] == float("inf")).all()), k
+        y[row] = clean[row]
+        assert torch.equal(y, clean), k
