@@ -79,18 +79,14 @@ at::Tensor result(const at::Tensor& x, int64_t N, int dt) {
   return at::empty(shape, x.options().dtype(type_of(dt)));
 }
 
-// The raw current stream of a device: torch's own query, looked up once.
+// torch's query of a device's raw current stream, looked up when the module is loaded: a lookup on first
+// use under a static's guard could yield the interpreter lock to a thread that then waits for the guard.
+PyObject* g_stream_query = nullptr;
+
 void* stream_of(const at::Tensor& t, bool& ok) {
-  static PyObject* const query = [] {
-    PyObject* m = PyImport_ImportModule("torch._C");
-    PyObject* f = m ? PyObject_GetAttrString(m, "_cuda_getCurrentRawStream") : nullptr;
-    Py_XDECREF(m);
-    return f;
-  }();
   ok = false;
-  if (!query) return nullptr;
   PyObject* index = PyLong_FromLong(t.get_device());
-  PyObject* r = index ? PyObject_CallOneArg(query, index) : nullptr;
+  PyObject* r = index ? PyObject_CallOneArg(g_stream_query, index) : nullptr;
   Py_XDECREF(index);
   if (!r) return nullptr;
   void* st = PyLong_AsVoidPtr(r);
@@ -348,4 +344,9 @@ PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, kMethods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fast(void) { return PyModule_Create(&kModule); }
+PyMODINIT_FUNC PyInit__fast(void) {
+  PyObject* c = PyImport_ImportModule("torch._C");
+  Py_XSETREF(g_stream_query, c ? PyObject_GetAttrString(c, "_cuda_getCurrentRawStream") : nullptr);
+  Py_XDECREF(c);
+  return g_stream_query ? PyModule_Create(&kModule) : nullptr;
+}

@@ -1,6 +1,10 @@
 """The operators' native call path (mlxq._fast) against their general path, which a caller-given
 workspace or output forces: the same bits for operands that need no preparation, and the general
 path's handling (copies, errors) for those that do."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -113,3 +117,15 @@ def test_fast_quantize_dequantize(mlxq, dt, N, K, gs, bits, count):
         mlxq.dequantize(got[0][0], got[0][1][:, :0], got[0][2], gs, bits)
     with pytest.raises(mlxq.MlxqError):
         mlxq.quantize_batched(ws, 48, bits)
+
+
+def test_stream_query_is_looked_up_at_import():
+    """No GPU needed: the module takes torch's stream query when it is loaded (a first call of several
+    threads at once must not import), so it does not load without one."""
+    code = ("import torch, sys; sys.path.insert(0, {!r}); import mlxq; q = torch._C._cuda_getCurrentRawStream\n"
+            "del torch._C._cuda_getCurrentRawStream\n"
+            "try:\n    import mlxq._fast; print('loaded')\n"
+            "except (ImportError, AttributeError):\n    torch._C._cuda_getCurrentRawStream = q; import mlxq._fast; print('ok')\n")
+    pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mlx-gen_amd")
+    r = subprocess.run([sys.executable, "-c", code.format(pkg)], capture_output=True, text=True, timeout=110)
+    assert r.stdout.strip() == "ok", r.stdout + r.stderr
