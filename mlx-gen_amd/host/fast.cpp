@@ -4,9 +4,10 @@
 // dtype checks, one ctypes conversion per argument and the stream object came to ~14 us a call,
 // against 5-7 us of kernel.  Each function here takes the call whose operands need no preparation
 // (GPU tensors of the expected ranks, shapes and dtypes, contiguous and aligned), allocates the
-// result and calls the C ABI; for anything else, and for every status but MLXQ_OK, it returns None
-// and the caller's general path prepares the operands or reports the error.  Nothing is kept from
-// one call to the next.
+// result and calls the C ABI; for anything else, and for a call that the library refuses, it returns
+// None and the caller's general path prepares the operands or reports the error.  A device error is
+// raised from here: the launch that failed is not made a second time.  Nothing is kept from one call to
+// the next.
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <ATen/ATen.h>
@@ -95,12 +96,25 @@ void* stream_of(const at::Tensor& t, bool& ok) {
   return st;
 }
 
-// Calls the library without the interpreter lock, as ctypes does.
+// MlxqError, given by the Python side when it loads the module.
+PyObject* g_error = nullptr;
+
+// A status that no second attempt may hide, raised as MlxqError(status, message).
+struct DeviceError {
+  int rc;
+};
+
+void refuse(int rc) {
+  if (rc != MLXQ_OK && rc != MLXQ_EINVAL && rc != MLXQ_EUNSUPPORTED) throw DeviceError{rc};
+}
+
+// Calls the library without the interpreter lock, as ctypes does; its last error is this thread's.
 template <typename F>
 int unlocked(F&& call) {
   PyThreadState* save = PyEval_SaveThread();
   const int rc = call();
   PyEval_RestoreThread(save);
+  refuse(rc);
   return rc;
 }
 
@@ -109,6 +123,15 @@ template <typename F>
 PyObject* guarded(F&& f) {
   try {
     if (PyObject* r = f()) return r;
+  } catch (const DeviceError& e) {
+    if (g_error) {
+      PyErr_Clear();
+      if (PyObject* v = PyObject_CallFunction(g_error, "is", e.rc, mlxq_last_error())) {
+        PyErr_SetObject(g_error, v);
+        Py_DECREF(v);
+      }
+      return nullptr;
+    }
   } catch (...) {
   }
   PyErr_Clear();
@@ -330,7 +353,15 @@ PyObject* quantize_batched(PyObject*, PyObject* const* a, Py_ssize_t n) {
   });
 }
 
+// set_error_type(MlxqError)
+PyObject* set_error_type(PyObject*, PyObject* type) {
+  Py_INCREF(type);
+  Py_XSETREF(g_error, type);
+  Py_RETURN_NONE;
+}
+
 PyMethodDef kMethods[] = {
+    {"set_error_type", (PyCFunction)set_error_type, METH_O, nullptr},
     {"quantized_matmul", (PyCFunction)(void*)quantized_matmul, METH_FASTCALL, nullptr},
     {"linear", (PyCFunction)(void*)linear, METH_FASTCALL, nullptr},
     {"swiglu", (PyCFunction)(void*)swiglu, METH_FASTCALL, nullptr},

@@ -142,7 +142,8 @@ _fast = None
 
 def fast():
     """The native call path of the operators (_fast.so, host/fast.cpp): each function returns None for
-    a call whose operands need preparation or that failed, and the caller takes its general path."""
+    a call whose operands need preparation or that is refused, and the caller takes its general path; a
+    device error is raised as MlxqError."""
     global _fast
     if _fast is None:
         load()
@@ -151,6 +152,7 @@ def fast():
         except ImportError as e:
             raise ImportError(f"mlxq._fast is missing or does not load ({e}): build it with "
                               "`make -C mlx-gen_amd/csrc` (or __graft_entry__.build())") from e
+        module.set_error_type(MlxqError)
         _fast = module
     return _fast
 

@@ -1,6 +1,7 @@
 """The operators' native call path (mlxq._fast) against their general path, which a caller-given
 workspace or output forces: the same bits for operands that need no preparation, and the general
 path's handling (copies, errors) for those that do."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -129,3 +130,31 @@ def test_stream_query_is_looked_up_at_import():
     pkg = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "mlx-gen_amd")
     r = subprocess.run([sys.executable, "-c", code.format(pkg)], capture_output=True, text=True, timeout=110)
     assert r.stdout.strip() == "ok", r.stdout + r.stderr
+
+
+@pytest.mark.gpu
+def test_device_error_is_raised_once(mlxq):
+    """A launch check that finds an error (here one that a refused hipSetDevice left recorded on this
+    thread) raises MLXQ_EDEVICE with the library's message, as the general path does, and is not tried again."""
+    path = next(line.split()[-1] for line in open("/proc/self/maps") if "libamdhip64" in line)
+    hip = ctypes.CDLL(path)
+    p = _pack(40, 128, 64, 4, torch.bfloat16)
+    x = torch.ones((2, 128), device="cuda", dtype=torch.bfloat16)
+    ids = torch.zeros(3, device="cuda", dtype=torch.int32)
+    w = [torch.ones((8, 128), device="cuda")]
+    out = torch.empty((2, 40), device="cuda", dtype=torch.bfloat16)
+    calls = [lambda: mlxq.quantized_matmul(x, *p, out=out),  # the general path
+             lambda: mlxq.quantized_matmul(x, *p), lambda: mlxq.linear(x, *p), lambda: mlxq.swiglu(x, p, p),
+             lambda: mlxq.embedding(ids, *p), lambda: mlxq.dequantize(*p), lambda: mlxq.quantize_batched(w)]
+    for call in calls:
+        call()
+        torch.cuda.synchronize()
+        assert hip.hipSetDevice(9999) != 0
+        try:
+            with pytest.raises(mlxq.MlxqError, match="launch failed") as e:
+                call()
+        finally:
+            hip.hipGetLastError()
+        assert e.value.status == 3
+        call()
+    torch.cuda.synchronize()
