@@ -29,11 +29,13 @@ int code_of(at::ScalarType t) {
 
 at::ScalarType type_of(int code) { return code == MLXQ_BFLOAT16 ? at::kBFloat16 : at::kFloat; }
 
-// A plain GPU tensor in row-major order whose data starts at a multiple of `align` bytes.
+// A plain GPU tensor in row-major order whose data starts at a multiple of `align` bytes (a nested tensor
+// calls itself strided and contiguous too, and is for the general path to refuse).
 const at::Tensor* plain(PyObject* o, size_t align) {
   if (!THPVariable_CheckExact(o)) return nullptr;
   const at::Tensor& t = THPVariable_Unpack(o);
-  if (!t.is_cuda() || t.layout() != at::kStrided || !t.is_contiguous() || t.is_conj() || t.is_neg()) return nullptr;
+  if (!t.is_cuda() || t.layout() != at::kStrided || t.is_nested()) return nullptr;
+  if (!t.is_contiguous() || t.is_conj() || t.is_neg()) return nullptr;
   if (reinterpret_cast<uintptr_t>(t.data_ptr()) % align != 0) return nullptr;
   return &t;
 }

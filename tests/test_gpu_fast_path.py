@@ -158,3 +158,13 @@ def test_device_error_is_raised_once(mlxq):
         assert e.value.status == 3
         call()
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+def test_nested_tensors_stay_refused(mlxq):
+    p = _pack(32, 64, 64, 4, torch.bfloat16)
+    row = torch.ones(64, device="cuda", dtype=torch.bfloat16)
+    x = torch.nested.nested_tensor([row, row, row])
+    for call in (lambda: mlxq.linear(x, *p), lambda: mlxq.quantized_matmul(x, *p), lambda: mlxq.swiglu(x, p, p)):
+        with pytest.raises(RuntimeError, match="Nested"):
+            call()
