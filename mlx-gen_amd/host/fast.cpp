@@ -12,6 +12,8 @@
 
 #include <ATen/ATen.h>
 
+#include <string.h>
+
 #include <vector>
 
 #include "../../include/mlxq.h"
@@ -375,9 +377,22 @@ PyMethodDef kMethods[] = {
 
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_fast", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};
 
+// Built against one torch's headers: another one's objects may be laid out differently.
+bool built_for_this_torch() {
+  PyObject* torch = PyImport_ImportModule("torch");
+  PyObject* v = torch ? PyObject_GetAttrString(torch, "__version__") : nullptr;
+  const char* text = v ? PyUnicode_AsUTF8(v) : nullptr;
+  const bool same = text && strcmp(text, MLXQ_TORCH_VERSION) == 0;
+  if (text && !same) PyErr_Format(PyExc_ImportError, "mlxq._fast is built for torch %s, not %s", MLXQ_TORCH_VERSION, text);
+  Py_XDECREF(v);
+  Py_XDECREF(torch);
+  return same;
+}
+
 }  // namespace
 
 PyMODINIT_FUNC PyInit__fast(void) {
+  if (!built_for_this_torch()) return nullptr;
   PyObject* c = PyImport_ImportModule("torch._C");
   Py_XSETREF(g_stream_query, c ? PyObject_GetAttrString(c, "_cuda_getCurrentRawStream") : nullptr);
   Py_XDECREF(c);
