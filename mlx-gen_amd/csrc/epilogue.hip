@@ -426,16 +426,42 @@ __global__ void linear_epilogue_kernel(LinearEpilogueArgs a) {
 // for each, had taken 5.7 ms for [4608, 12288] f32 at R = 32, where y's 453 MB take 92 us.  The
 // activation rows are the MFMA's A side, so a lane holds 16 rows m of one column; its two columns
 // are neighbours (n = 2 (lane & 31) + j), so a wave's access to a row of y is 64 contiguous
-// elements.
-template <typename YI, typename YO, bool DRB>
+// elements.  A lane reads its part of y before anything is stored: y_out may be y_in, so reads left
+// among the stores waited for memory one after another.
+// SPLIT waves share a block, each making its products again and finishing 16 / SPLIT of a lane's rows:
+// a small grid is bound by one wave's chain of activations and stores (lora_epilogue_split).
+template <typename YI, typename YO, bool DRB, int SPLIT>
 __global__ __launch_bounds__(256) void lora_epilogue_kernel(LinearEpilogueArgs a, int64_t tiles_n) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r32 = lane & 31, half = lane >> 5;
-  const int64_t m0 = (int64_t)(blockIdx.x / tiles_n) * 32;
-  const int64_t n0 = (int64_t)(blockIdx.x % tiles_n) * 256 + wave * 64;
+  constexpr int RPW = 16 / SPLIT;  // rows of a lane that this wave finishes: v0 .. v0 + RPW - 1
+  const int lane = threadIdx.x & 63, r32 = lane & 31, half = lane >> 5;
+  const int64_t w = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int v0 = (int)(w % SPLIT) * RPW;
+  const int64_t m0 = w / SPLIT / tiles_n * 32, n0 = w / SPLIT % tiles_n * 64;
+  if (m0 >= a.M) return;  // waves past the last block
   const int64_t mr = m0 + r32 < a.M ? m0 + r32 : a.M - 1;  // rows and columns past the ends repeat
   int64_t nr[2];                                           // the last one and are never stored
 #pragma unroll
   for (int j = 0; j < 2; ++j) nr[j] = n0 + 2 * r32 + j < a.N ? n0 + 2 * r32 + j : a.N - 1;
+  const int64_t n = n0 + 2 * r32;
+  const YI* const yi = static_cast<const YI*>(a.y_in);
+  YO* const yo = static_cast<YO*>(a.y_out);
+  struct alignas(2 * sizeof(YI)) VI { YI v[2]; };
+  struct alignas(2 * sizeof(YO)) VO { YO v[2]; };
+  // Pairs need an even N (a row's start aligned to two elements); both pointers are.
+  const bool pairs = a.N % 2 == 0 && reinterpret_cast<uintptr_t>(a.y_in) % sizeof(VI) == 0 &&
+                     reinterpret_cast<uintptr_t>(a.y_out) % sizeof(VO) == 0;
+  auto row = [&](int v) { return m0 + 8 * ((v0 + v) >> 2) + 4 * half + ((v0 + v) & 3); };
+  VI in[RPW];
+  if (pairs) {
+#pragma unroll
+    for (int v = 0; v < RPW; ++v)
+      in[v] = *reinterpret_cast<const VI*>(yi + (row(v) < a.M ? row(v) : a.M - 1) * a.N + (n < a.N ? n : a.N - 2));
+  } else {
+#pragma unroll
+    for (int v = 0; v < RPW; ++v)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) in[v].v[j] = yi[(row(v) < a.M ? row(v) : a.M - 1) * a.N + nr[j]];
+  }
   f32x16 r[2] = {f32x16{}, f32x16{}};
   for (int k = 0; k < a.R; k += 16) {
     if constexpr (DRB) {
@@ -460,33 +486,40 @@ __global__ __launch_bounds__(256) void lora_epilogue_kernel(LinearEpilogueArgs a
       }
     }
   }
-  const int64_t n = n0 + 2 * r32;
   if (n >= a.N) return;
-  const YI* const yi = static_cast<const YI*>(a.y_in);
-  YO* const yo = static_cast<YO*>(a.y_out);
-  struct alignas(2 * sizeof(YI)) VI { YI v[2]; };
-  struct alignas(2 * sizeof(YO)) VO { YO v[2]; };
-  // Pairs need an even N (a row's start aligned to two elements); both pointers are.
-  const bool pairs = a.N % 2 == 0 && reinterpret_cast<uintptr_t>(a.y_in) % sizeof(VI) == 0 &&
-                     reinterpret_cast<uintptr_t>(a.y_out) % sizeof(VO) == 0;
+  float rv[2][RPW];
 #pragma unroll
-  for (int v = 0; v < 16; ++v) {
-    const int64_t m = m0 + 8 * (v >> 2) + 4 * half + (v & 3);
-    if (m >= a.M) continue;
-    const int64_t t = m * a.N + n;
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int v = 0; v < RPW; ++v) {
+      rv[j][v] = r[j][v];
+#pragma unroll
+      for (int s = 1; s < SPLIT; ++s) rv[j][v] = v0 == s * RPW ? r[j][s * RPW + v] : rv[j][v];
+    }
+#pragma unroll
+  for (int v = 0; v < RPW; ++v) {
+    if (row(v) >= a.M) continue;
+    const int64_t t = row(v) * a.N + n;
     if (pairs) {
-      const VI in = *reinterpret_cast<const VI*>(yi + t);
       VO out;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) Act<YO>::st(out.v, j, epilogue_finish(a, Act<YI>::ld(in.v, j), n + j, true, r[j][v]));
+      for (int j = 0; j < 2; ++j) Act<YO>::st(out.v, j, epilogue_finish(a, Act<YI>::ld(in[v].v, j), n + j, true, rv[j][v]));
       *reinterpret_cast<VO*>(yo + t) = out;
     } else {
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        if (n + j < a.N) Act<YO>::st(yo, t + j, epilogue_finish(a, Act<YI>::ld(yi, t + j), n + j, true, r[j][v]));
+        if (n + j < a.N) Act<YO>::st(yo, t + j, epilogue_finish(a, Act<YI>::ld(in[v].v, j), n + j, true, rv[j][v]));
     }
   }
 }
+
+// Waves per 32 x 64 block.  Same-process times in us for 1 / 4 / 16 (whole calls; one thread per output in
+// brackets): 36 blocks, [66, 1024] rank 1 with GELU 20.9 / - / - [16.2]; 16 blocks, [28, 640] rank 8
+// 10.7 / 6.9 / 5.7 [8.5]; 64 blocks, [11, 832] rank 16 17.2 / 15.6 / 14.0 [16.7]; 124 blocks, [98, 1216]
+// rank 1 with GELU 26.5 / 20.5 / 19.2 [24.5]; 101 blocks, [5, 704] rank 256 30.9 / 29.3 / 40.2; 365 blocks,
+// [140, 1792] rank 64 39.1 / 31.0 / 34.5; 560 blocks, [233, 832] rank 256 63.0 / 65.7 / 96.5; 814 blocks, rank
+// 256 61.6 / 91.4 / 188.
+static int lora_epilogue_split(int64_t tiles) { return tiles <= 64 ? 16 : tiles <= 512 ? 4 : 1; }
 
 int run_linear_epilogue(const LinearEpilogueArgs& a, hipStream_t st) {
   const int64_t total = a.M * a.N;
@@ -498,18 +531,26 @@ int run_linear_epilogue(const LinearEpilogueArgs& a, hipStream_t st) {
     return set_error(MLXQ_EINVAL, "linear epilogue: activation table missing");
   const dim3 b(256);
   if (a.R > 0) {
-    const int64_t tiles_n = (a.N + 255) / 256, tiles = (a.M + 31) / 32 * tiles_n;
-    const dim3 g((unsigned)tiles);
-#define MLXQ_LE(YI, YO)                                                                             \
-  do {                                                                                              \
-    if (a.dr_bf16) hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, true>), g, b, 0, st, a, tiles_n); \
-    else hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, false>), g, b, 0, st, a, tiles_n);        \
+    const int64_t tiles_n = (a.N + 63) / 64, tiles = (a.M + 31) / 32 * tiles_n;
+    const int split = lora_epilogue_split(tiles);
+    const dim3 g((unsigned)((tiles * split + 3) / 4));
+#define MLXQ_LES(YI, YO, S)                                                                             \
+  do {                                                                                                  \
+    if (a.dr_bf16) hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, true, S>), g, b, 0, st, a, tiles_n); \
+    else hipLaunchKernelGGL((lora_epilogue_kernel<YI, YO, false, S>), g, b, 0, st, a, tiles_n);         \
+  } while (0)
+#define MLXQ_LE(YI, YO)                     \
+  do {                                      \
+    if (split == 1) MLXQ_LES(YI, YO, 1);    \
+    else if (split == 4) MLXQ_LES(YI, YO, 4); \
+    else MLXQ_LES(YI, YO, 16);              \
   } while (0)
     if (a.y_in_bf16 && a.y_out_bf16) MLXQ_LE(uint16_t, uint16_t);
     else if (a.y_in_bf16) MLXQ_LE(uint16_t, float);
     else if (a.y_out_bf16) MLXQ_LE(float, uint16_t);
     else MLXQ_LE(float, float);
 #undef MLXQ_LE
+#undef MLXQ_LES
     return check_launch("linear_epilogue");
   }
   const dim3 g((unsigned)blocks);

@@ -60,3 +60,28 @@ def test_lora_residual_f32_infinity(mlxq):
     assert torch.isinf(out[4]).all()
     keep = [i for i in range(33) if i != 4]
     assert (out[keep] == 64 * 17).all()
+
+
+@pytest.mark.parametrize("xdt,fdt,ydt", [("bf16", "bf16", "bf16"), ("bf16", "bf16", "f32"), ("f32", "bf16", "f32"), ("f16", "f32", "bf16"),
+                                         ("bf16", "f32", "bf16")])
+@pytest.mark.parametrize("N,rank", [(640, 8), (333, 17), (64, 32), (1, 1), (2050, 64)])
+def test_lora_epilogue_grid_forms(mlxq, xdt, fdt, ydt, N, rank):
+    """One, four or sixteen waves per 32 x 64 block (over 512 blocks, up to 512, up to 64): the same bits,
+    with paired columns and (odd N, a y that starts at an odd element) single ones."""
+    banner("lora epilogue forms", xdt, fdt, ydt, N, rank)
+    g = torch.Generator(device="cuda").manual_seed(N + rank)
+    mk = lambda shape, dt: torch.randn(shape, generator=g, device="cuda").to(DT[dt])  # noqa: E731
+    blocks_n = (N + 63) // 64
+    M = 32 * (512 // blocks_n + 1) - 5
+    x, a, b, y = mk((M, 96), xdt), mk((96, rank), fdt), mk((rank, N), fdt), mk((M, N), ydt)
+    big = mlxq.lora_residual(x, y.clone(), a, b, 0.75)
+    xs, fs = x.double(), mlxq.promote(DT[xdt], DT[fdt])
+    r = (xs @ a.double()).to(fs).double() @ b.double()
+    want = y.double() + (r.to(fs).double() * 0.75).to(fs).double()
+    tol = 2.0 ** -6 if "bf16" in (str(fs)[-4:], ydt) or fs == torch.bfloat16 else 1e-5
+    assert ((big.double() - want).norm() / want.norm()).item() < tol
+    for m0, rows in ((0, 32 * max(1, 512 // blocks_n)), (32, 32 * max(1, 64 // blocks_n) - 3), (M - 5, 5)):
+        shifted = torch.empty(rows * N + 1, device="cuda", dtype=DT[ydt])
+        for ys in (y[m0:m0 + rows].clone(), shifted[1:].view(rows, N).copy_(y[m0:m0 + rows])):
+            got = mlxq.lora_residual(x[m0:m0 + rows], ys, a, b, 0.75)
+            assert torch.equal(got, big[m0:m0 + rows]), (m0, rows)
