@@ -457,7 +457,11 @@ __global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
   const int n_end = N - n_begin < rows ? N : n_begin + rows;
   using Tile = GemvTile<BITS, GS, STEPS, MR, STEPS * RING>;
   Tile t(lane, wave_all, wave_all - mat * W, M, K, N, lds);
-  // Partial sums [wave][row m < MR][17]: over the operands, or (MULTI) in two buffers past them.
+  // Partial sums [wave][row m][17]: over the operands, all 16 rows, or (MULTI) in two buffers past them, the
+  // rows below MR.  One tile stores every row, unconditionally: with only the lanes of rows below MR storing,
+  // the compiler tracked the fold for those lanes and took up to 11 more registers (64 -> 68 for Q4 group 32,
+  // two steps, two rows), one workgroup per CU instead of two: [2, 1792] SwiGLU 6784 5.7 -> 6.4 us.
+  constexpr int RR = MULTI ? MR : 16;
   float* const red0 = reinterpret_cast<float*>(lds + (MULTI ? (NT >> 6) * (M * Tile::XW + 16 * Tile::PW * 4) : 0));
   const int red_buf = (NT >> 6) * MR * 17;
   const int sb_total = (int)(((uint32_t)N * (uint32_t)t.G * 2u + 3u) & ~3u);  // whole dwords
@@ -494,13 +498,13 @@ __global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
     } else {
       t.template fold<false>(yacc, 0);
     }
-    // Split-K reduction: row 4 q + e of the tile's column c16 (rows past MR are never read).
+    // Split-K reduction: row 4 q + e of the tile's column c16 (rows past M are never read).
     float* const red = red0 + buf * red_buf;
     const int c16 = lane & 15, q = lane >> 4;
     if constexpr (!MULTI) __syncthreads();
-    if (4 * q < MR) {
+    if (!MULTI || 4 * q < MR) {
 #pragma unroll
-      for (int e = 0; e < Tile::E; ++e) red[(wave_all * MR + 4 * q + e) * 17 + c16] = yacc[e];
+      for (int e = 0; e < Tile::E; ++e) red[(wave_all * RR + 4 * q + e) * 17 + c16] = yacc[e];
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
@@ -509,10 +513,10 @@ __global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
     for (int idx = tid; idx < 16 * M; idx += NT) {  // a one-wave workgroup has 64 < 16*M threads
       const int m = idx >> 4, nl = idx & 15;
       float v = 0.0f;
-      for (int w = 0; w < W; ++w) v += red[(w * MR + m) * 17 + nl];
+      for (int w = 0; w < W; ++w) v += red[(w * RR + m) * 17 + nl];
       if constexpr (NMAT == 2) {
         float u = 0.0f;
-        for (int w = 0; w < W; ++w) u += red[((W + w) * MR + m) * 17 + nl];
+        for (int w = 0; w < W; ++w) u += red[((W + w) * RR + m) * 17 + nl];
         // each op rounded to bf16 as the reference's separate ops are (qwen3.rs:178-181)
         if (nl < nr) y[m * N + n0 + nl] = f32_to_bf16_bits(silu_bf16(round_bf16(v)) * round_bf16(u));
       } else {
@@ -582,7 +586,7 @@ inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, QmvP
       const int64_t waves = nmat * wpm;
       if (waves > kMaxWaves) continue;
       const int64_t operands = waves * (int64_t)qmv_wave_lds(bits, gs, (int)t, (int)M);
-      const int64_t red = waves * mr * 17 * 4;  // one buffer of partial sums
+      const int64_t red = waves * 16 * 17 * 4;  // one tile's partial sums
       const int64_t lds = operands > red ? operands : red;
       if (lds > kMaxLds) continue;
       const int64_t cost = waves > 12 ? waves - 12 : 12 - waves;

@@ -1,0 +1,65 @@
+"""Registers of the built kernels, read from the library's own code objects: the decode GEMV's speed rests
+on how many of its workgroups a CU holds (512 registers per lane of a SIMD, handed out in eights)."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+LIB = os.path.join(ROOT, "mlx-gen_amd", "mlxq", "libmlxq_hip.so")
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """name -> (VGPRs, spilled VGPRs) of every kernel built here."""
+    if not os.path.exists(os.path.join(LLVM, "llvm-readelf")):
+        pytest.skip("no LLVM tools")
+    d = tmp_path_factory.mktemp("co")
+    subprocess.run([f"{LLVM}/llvm-objcopy", "--dump-section", f".hip_fatbin={d}/fat", LIB, f"{d}/copy.so"], check=True)
+    data = open(d / "fat", "rb").read()
+    out = {}
+    for m in re.finditer(rb"__CLANG_OFFLOAD_BUNDLE__", data):
+        p = m.start()
+        count, q = struct.unpack("<Q", data[p + 24:p + 32])[0], p + 32
+        for _ in range(count):
+            off, size, n = struct.unpack("<QQQ", data[q:q + 24])
+            name, q = data[q + 24:q + 24 + n], q + 24 + n
+            if b"gfx950" not in name or size == 0:
+                continue
+            (d / "co").write_bytes(data[p + off:p + off + size])
+            notes = subprocess.run([f"{LLVM}/llvm-readelf", "--notes", d / "co"], capture_output=True, text=True, check=True).stdout
+            for k in notes.split("- .agpr_count:")[1:]:
+                num = lambda f: int(re.search(rf"\.{f}:\s+(\d+)", k).group(1))  # noqa: E731
+                out[re.search(r"\.symbol:\s+(\S+)\.kd", k).group(1)] = num("vgpr_count"), num("vgpr_spill_count")
+    names = subprocess.run(["c++filt"], input="\n".join(out), capture_output=True, text=True, check=True).stdout.split("\n")
+    return dict(zip(names, out.values()))
+
+
+def _gemv(kernels):
+    """(bits, gs, steps, rows, matrices, rounds, several tiles) -> (VGPRs, spills)."""
+    found = {}
+    for name, v in kernels.items():
+        m = re.search(r"qmv_mfma_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (true|false)>", name)
+        if m:
+            found[tuple(int(t) for t in m.groups()[:6]) + (m.group(7) == "true",)] = v
+    assert len(found) > 200
+    return found
+
+
+# The forms whose one-tile kernel has at most 64 registers, so that two 16-wave workgroups share a CU: most
+# load steps per (bits, group size), and where fewer rows are the condition, (steps, most rows).
+TWO_PER_CU = {(8, 32): [(3, 8), (4, 2)], (8, 64): [(4, 8), (6, 2)], (8, 128): [(4, 8), (6, 2)],
+              (4, 32): [(1, 8)], (4, 64): [(2, 8), (3, 2)], (4, 128): [(4, 8)]}
+
+
+def test_one_tile_gemv_keeps_two_workgroups_per_cu(kernels):
+    seen = 0
+    for (bits, gs, steps, rows, nmat, ring, multi), (vgpr, _) in _gemv(kernels).items():
+        two = any(steps <= st and rows <= r for st, r in TWO_PER_CU[bits, gs]) or (bits, gs, steps, rows) == (4, 32, 2, 2)
+        if two and ring == 1 and not multi:
+            seen += 1
+            assert vgpr <= 64, (bits, gs, steps, rows, nmat, vgpr)
+    assert seen > 100
