@@ -430,23 +430,13 @@ __device__ __forceinline__ uint16_t gemv_finish(float v, int n, const uint16_t* 
 // anew for them (M = 5, K = 4096: 80 KB of activations per 64 KB of weights).  The decode MLP 4096 /
 // 11008 at M = 5: 30.3 -> 20.7 us, with the down projection's five rows in one launch instead of two.
 template <int BITS, int GS, int STEPS, int MR, int NMAT, int RING, bool MULTI>
-__global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
+__device__ __forceinline__ void qmv_mfma_body(
     const uint16_t* __restrict__ x, int M, int K, const uint32_t* __restrict__ wq,
     const uint16_t* __restrict__ scales, const uint16_t* __restrict__ biases,
     const uint32_t* __restrict__ wq2, const uint16_t* __restrict__ scales2,
     const uint16_t* __restrict__ biases2, int N, int rows, uint16_t* __restrict__ y,
-    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table, QmmBatch bat) {
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  // Stacked launch: grid.y selects the matrix (expert); one matrix has all strides zero.
-  if (gridDim.y > 1) {
-    const int64_t e = blockIdx.y;
-    x += e * bat.x;
-    wq += e * bat.w;
-    scales += e * bat.sb;
-    biases += e * bat.sb;
-    y += e * bat.y;
-    if (bias) bias += e * bat.bias;
-  }
   const int NT = blockDim.x;
   const int tid = threadIdx.x;
   const int lane = tid & 63;
@@ -526,6 +516,37 @@ __global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
     n0 = nn;
     buf ^= 1;
   } while (MULTI && n0 < n_end);
+}
+
+// Arguments come first in the order they are needed: 14 dwords of them are preloaded into registers, and
+// each further one that a workgroup's first loads wait for costs it a scalar load from memory.  With one
+// signature for both forms and the epilogue's operands besides, short launches took 0.1 us longer (2-3 %),
+// [2, 1664] x Q8 g128 [31437, 1664]^T 12.4 -> 13.3.
+template <int BITS, int GS, int STEPS, int MR, int RING, bool MULTI>
+__global__ __launch_bounds__(kMaxWaves * 64) void qmv_mfma_kernel(
+    const uint16_t* __restrict__ x, int M, int K, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, int N, int rows, uint16_t* __restrict__ y,
+    const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table, QmmBatch bat) {
+  // Stacked launch: the workgroup's y index selects the matrix (expert).
+  if (const int64_t e = blockIdx.y; e > 0) {
+    x += e * bat.x;
+    wq += e * bat.w;
+    scales += e * bat.sb;
+    biases += e * bat.sb;
+    y += e * bat.y;
+    if (bias) bias += e * bat.bias;
+  }
+  qmv_mfma_body<BITS, GS, STEPS, MR, 1, RING, MULTI>(x, M, K, wq, scales, biases, nullptr, nullptr, nullptr, N, rows, y,
+                                                     bias, act_table);
+}
+
+template <int BITS, int GS, int STEPS, int MR, int RING, bool MULTI>
+__global__ __launch_bounds__(kMaxWaves * 64) void swiglu_mfma_kernel(
+    const uint16_t* __restrict__ x, int M, int K, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, const uint32_t* __restrict__ wq2, const uint16_t* __restrict__ scales2,
+    const uint16_t* __restrict__ biases2, int N, int rows, uint16_t* __restrict__ y) {
+  qmv_mfma_body<BITS, GS, STEPS, MR, 2, RING, MULTI>(x, M, K, wq, scales, biases, wq2, scales2, biases2, N, rows, y,
+                                                     nullptr, nullptr);
 }
 
 struct QmvPlan {
@@ -672,18 +693,26 @@ static int launch_qmv_mfma(const QmvArgs& a, const QmvPlan& p, int rows, hipStre
   // The dynamic-LDS limit is raised once per device (any thread may get here first; setting it
   // twice is harmless).
   static std::atomic<bool> attr_set[64];
+  const void* kernel;
+  if constexpr (NMAT == 1) kernel = reinterpret_cast<const void*>(&qmv_mfma_kernel<BITS, GS, STEPS, MR, RING, MULTI>);
+  else kernel = reinterpret_cast<const void*>(&swiglu_mfma_kernel<BITS, GS, STEPS, MR, RING, MULTI>);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return set_error(MLXQ_EDEVICE, "qmv: no current device");
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmv_mfma_kernel<BITS, GS, STEPS, MR, NMAT, RING, MULTI>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds) != hipSuccess)
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds) != hipSuccess)
       return set_error(MLXQ_EDEVICE, "qmv: hipFuncSetAttribute failed");
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
-  hipLaunchKernelGGL((qmv_mfma_kernel<BITS, GS, STEPS, MR, NMAT, RING, MULTI>), dim3((unsigned)((a.N + rows - 1) / rows), (unsigned)a.bat.count),
-                     dim3(p.waves * 64), MULTI ? qmv_multi_lds(p) : p.lds, st, (const uint16_t*)a.x, (int)a.M, (int)a.K, a.wq,
-                     (const uint16_t*)a.s, (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2,
-                     (const uint16_t*)a.b2, (int)a.N, rows, (uint16_t*)a.y, a.bias, a.act_table, a.bat);
+  const dim3 grid((unsigned)((a.N + rows - 1) / rows), (unsigned)a.bat.count), block(p.waves * 64);
+  const unsigned lds = MULTI ? qmv_multi_lds(p) : p.lds;
+  if constexpr (NMAT == 1)
+    hipLaunchKernelGGL((qmv_mfma_kernel<BITS, GS, STEPS, MR, RING, MULTI>), grid, block, lds, st, (const uint16_t*)a.x,
+                       (int)a.M, (int)a.K, a.wq, (const uint16_t*)a.s, (const uint16_t*)a.b, (int)a.N, rows,
+                       (uint16_t*)a.y, a.bias, a.act_table, a.bat);
+  else
+    hipLaunchKernelGGL((swiglu_mfma_kernel<BITS, GS, STEPS, MR, RING, MULTI>), grid, block, lds, st, (const uint16_t*)a.x,
+                       (int)a.M, (int)a.K, a.wq, (const uint16_t*)a.s, (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2,
+                       (const uint16_t*)a.b2, (int)a.N, rows, (uint16_t*)a.y);
   return check_launch(NMAT == 2 ? "swiglu_qmv" : "qmv_mfma");
 }
 

@@ -59,22 +59,12 @@ __device__ __forceinline__ float dpp_f32(float v) {
 // the dot product of its 16 codes with their activations by v_dot2_f32_bf16, two products per
 // instruction with f32 accumulation (y += s * dot, plus b * X once per column), and all 64 lanes' partial sums are added at the end.  It exists for the kernel-choice
 // A/B (mlxq_qmv_valu), not for quantized_matmul.
-template <bool G64, int LS, int NMAT, bool VALU = false>
-__global__ __launch_bounds__(1024) void qmv_row_kernel(
+template <bool G64, int LS, int NMAT, bool VALU>
+__device__ __forceinline__ void qmv_row_body(
     const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
     const uint16_t* __restrict__ biases, const uint32_t* __restrict__ wq2,
     const uint16_t* __restrict__ scales2, const uint16_t* __restrict__ biases2, int K, int N,
-    uint16_t* __restrict__ y, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table, QmmBatch bat) {
-  // Stacked launch: grid.y selects the matrix (expert); one matrix has all strides zero.
-  if (gridDim.y > 1) {
-    const int64_t e = blockIdx.y;
-    x += e * bat.x;
-    wq += e * bat.w;
-    scales += e * bat.sb;
-    biases += e * bat.sb;
-    y += e * bat.y;
-    if (bias) bias += e * bat.bias;
-  }
+    uint16_t* __restrict__ y, const uint16_t* __restrict__ bias, const uint16_t* __restrict__ act_table) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   constexpr int C = 16 * LS;                  // 64-code columns per row, padded to whole loads
   constexpr int G = G64 ? C : C / 2;          // groups per padded row (table entries)
@@ -280,6 +270,32 @@ __global__ __launch_bounds__(1024) void qmv_row_kernel(
   }
 }
 
+// Arguments in the order they are needed, a signature for each form, as the tile kernels have.
+template <bool G64, int LS, bool VALU>
+__global__ __launch_bounds__(1024) void qmv_row_kernel(
+    const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, int K, int N, uint16_t* __restrict__ y, const uint16_t* __restrict__ bias,
+    const uint16_t* __restrict__ act_table, QmmBatch bat) {
+  // Stacked launch: the workgroup's y index selects the matrix (expert).
+  if (const int64_t e = blockIdx.y; e > 0) {
+    x += e * bat.x;
+    wq += e * bat.w;
+    scales += e * bat.sb;
+    biases += e * bat.sb;
+    y += e * bat.y;
+    if (bias) bias += e * bat.bias;
+  }
+  qmv_row_body<G64, LS, 1, VALU>(x, wq, scales, biases, nullptr, nullptr, nullptr, K, N, y, bias, act_table);
+}
+
+template <bool G64, int LS>
+__global__ __launch_bounds__(1024) void swiglu_row_kernel(
+    const uint16_t* __restrict__ x, const uint32_t* __restrict__ wq, const uint16_t* __restrict__ scales,
+    const uint16_t* __restrict__ biases, const uint32_t* __restrict__ wq2, const uint16_t* __restrict__ scales2,
+    const uint16_t* __restrict__ biases2, int K, int N, uint16_t* __restrict__ y) {
+  qmv_row_body<G64, LS, 2, false>(x, wq, scales, biases, wq2, scales2, biases2, K, N, y, nullptr, nullptr);
+}
+
 template <int NMAT>
 static int qmv_kind(const QmvArgs& a, int gs, int bits, const QmvPlan& p, hipStream_t st) {
   if (bits == 8) {
@@ -321,20 +337,26 @@ template <bool G64, int LS, int NMAT, bool VALU = false>
 static int launch_qmv_row(const QmvArgs& a, hipStream_t st) {
   static_assert(qmv_row_lds(LS, G64, NMAT, 16) <= kMaxLds, "one-row workgroup exceeds the LDS");
   static std::atomic<bool> attr_set[64];
+  const void* kernel;
+  if constexpr (NMAT == 1) kernel = reinterpret_cast<const void*>(&qmv_row_kernel<G64, LS, VALU>);
+  else kernel = reinterpret_cast<const void*>(&swiglu_row_kernel<G64, LS>);
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return set_error(MLXQ_EDEVICE, "qmv: no current device");
   if (dev < 0 || dev >= 64 || !attr_set[dev].load(std::memory_order_acquire)) {
-    if (hipFuncSetAttribute(reinterpret_cast<const void*>(&qmv_row_kernel<G64, LS, NMAT, VALU>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds) != hipSuccess)
+    if (hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, kMaxLds) != hipSuccess)
       return set_error(MLXQ_EDEVICE, "qmv: hipFuncSetAttribute failed");
     if (dev >= 0 && dev < 64) attr_set[dev].store(true, std::memory_order_release);
   }
   const int wpb = qmv_row_wpb(a.N, NMAT);
   const int lds = qmv_row_lds(LS, G64, NMAT, wpb);
-  hipLaunchKernelGGL((qmv_row_kernel<G64, LS, NMAT, VALU>), dim3((unsigned)((a.N + wpb - 1) / wpb), (unsigned)a.bat.count),
-                     dim3(wpb * 64), lds, st, (const uint16_t*)a.x, a.wq, (const uint16_t*)a.s,
-                     (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2, (const uint16_t*)a.b2, (int)a.K,
-                     (int)a.N, (uint16_t*)a.y, a.bias, a.act_table, a.bat);
+  const dim3 grid((unsigned)((a.N + wpb - 1) / wpb), (unsigned)a.bat.count), block(wpb * 64);
+  if constexpr (NMAT == 1)
+    hipLaunchKernelGGL((qmv_row_kernel<G64, LS, VALU>), grid, block, lds, st, (const uint16_t*)a.x, a.wq, (const uint16_t*)a.s,
+                       (const uint16_t*)a.b, (int)a.K, (int)a.N, (uint16_t*)a.y, a.bias, a.act_table, a.bat);
+  else
+    hipLaunchKernelGGL((swiglu_row_kernel<G64, LS>), grid, block, lds, st, (const uint16_t*)a.x, a.wq, (const uint16_t*)a.s,
+                       (const uint16_t*)a.b, a.wq2, (const uint16_t*)a.s2, (const uint16_t*)a.b2, (int)a.K, (int)a.N,
+                       (uint16_t*)a.y);
   return check_launch(NMAT == 2 ? "swiglu_qmv_row" : VALU ? "qmv_row_valu" : "qmv_row");
 }
 

@@ -42,9 +42,10 @@ def _gemv(kernels):
     """(bits, gs, steps, rows, matrices, rounds, several tiles) -> (VGPRs, spills)."""
     found = {}
     for name, v in kernels.items():
-        m = re.search(r"qmv_mfma_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (\d+), (true|false)>", name)
+        m = re.search(r"(qmv|swiglu)_mfma_kernel<(\d+), (\d+), (\d+), (\d+), (\d+), (true|false)>", name)
         if m:
-            found[tuple(int(t) for t in m.groups()[:6]) + (m.group(7) == "true",)] = v
+            n = [int(t) for t in m.groups()[1:6]]
+            found[(*n[:4], 1 if m.group(1) == "qmv" else 2, n[4], m.group(7) == "true")] = v
     assert len(found) > 200
     return found
 
@@ -63,3 +64,29 @@ def test_one_tile_gemv_keeps_two_workgroups_per_cu(kernels):
             seen += 1
             assert vgpr <= 64, (bits, gs, steps, rows, nmat, vgpr)
     assert seen > 100
+
+
+# Pointers are two dwords, sizes one; the first 14 dwords of arguments are preloaded into registers.
+NEEDED_FIRST = {  # what a workgroup needs for its loads and its result, in this order
+    "qmv_mfma_kernel": ["x", "M", "K", "wq", "scales", "biases", "N", "rows", "y"],
+    "qmv_row_kernel": ["x", "wq", "scales", "biases", "K", "N", "y"],
+}
+
+
+def test_gemv_arguments_are_preloaded(kernels):
+    """A short launch waits for each argument that its first loads need and that is not in registers when
+    it starts: those come before the epilogue's and the stacked launch's, which SwiGLU does not have."""
+    seen = set()
+    for name in kernels:
+        m = re.search(r"mlxq::(qmv_mfma_kernel|qmv_row_kernel|swiglu_mfma_kernel|swiglu_row_kernel)<.*>\((.*)\)", name)
+        if not m:
+            continue
+        seen.add(m.group(1))
+        args = [t.strip() for t in m.group(2).split(",")]
+        first = NEEDED_FIRST.get(m.group(1))
+        if first is None:
+            assert len(args) == (12 if "mfma" in m.group(1) else 10) and "QmmBatch" not in m.group(2), name
+            continue
+        assert [t == "int" for t in args[:len(first)]] == [len(f) == 1 and f.isupper() or f == "rows" for f in first], name
+        assert sum(1 if t == "int" else 2 for t in args[:len(first)]) <= 14, name
+    assert len(seen) == 4
