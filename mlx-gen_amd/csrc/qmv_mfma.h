@@ -587,11 +587,14 @@ constexpr bool qmv_multi_built(int bits, int gs, int steps, int mr, int nmat, in
 // When no count divides the row's load steps within those limits (K = 11008: 86 steps of Q4),
 // the waves take ceil(steps / waves) each and the last one's range ends past K (cost as above,
 // then the fewest padded steps); failing that, each wave takes two rounds of its load registers
-// (ring 2: twice the K at the same registers).  A launch holds its activation rows whole in LDS
+// (ring 2: twice the K at the same registers).  one_batch: only plans whose lanes stage all their
+// activation chunks at once; a second batch waits for memory again before the wave's first product
+// (16 waves of 4 steps in one batch against 11 of 6 in two: [8, 7808] x Q4 g128 [880, 7808]^T 5.4 against
+// 6.4 us, SwiGLU [7, 3968] x [7936, 3968]^T 9.7 against 12.5), so the others are for what fits no such plan.  A launch holds its activation rows whole in LDS
 // (M x K x 2 bytes), so rows that fit no plan go out as launches of four, else two rows (M = 8,
 // K = 18944: four launches of two rows 46 us against 85 us on the VALU GEMV; single rows would
 // stream the weights M times and lose to it).
-inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, QmvPlan& p) {
+inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, bool one_batch, QmvPlan& p) {
   const int64_t cpl = 512 / bits;
   const int64_t LS = (K + cpl - 1) / cpl;
   const int mr = M <= 1 ? 1 : (M <= 2 ? 2 : (M <= 4 ? 4 : 8));
@@ -610,6 +613,7 @@ inline bool qmv_plan_rows(int64_t M, int64_t K, int gs, int bits, int nmat, QmvP
       const int64_t red = waves * 16 * 17 * 4;  // one tile's partial sums
       const int64_t lds = operands > red ? operands : red;
       if (lds > kMaxLds) continue;
+      if (one_batch && mr * ((t * cpl / 8 + 63) / 64) > kCopySlots) continue;
       const int64_t cost = waves > 12 ? waves - 12 : 12 - waves;
       const int64_t pad = wpm * t - LS;
       if (found && (cost > best_cost || (cost == best_cost && pad >= best_pad))) continue;
@@ -627,9 +631,10 @@ inline bool qmv_plan(int64_t M, int64_t K, int gs, int bits, int nmat, QmvPlan& 
   if (M < 1 || M > 8 || (bits != 4 && bits != 8)) return false;
   if (gs != 32 && gs != 64 && gs != 128) return false;
   if (K <= 0 || K % gs != 0) return false;
-  if (qmv_plan_rows(M, K, gs, bits, nmat, p)) return true;
+  for (bool one_batch : {true, false})
+    if (qmv_plan_rows(M, K, gs, bits, nmat, one_batch, p)) return true;
   for (int rows : {4, 2})  // launches of fewer rows
-    if (M > rows && qmv_plan_rows(rows, K, gs, bits, nmat, p)) return true;
+    if (M > rows && qmv_plan_rows(rows, K, gs, bits, nmat, false, p)) return true;
   return false;
 }
 
