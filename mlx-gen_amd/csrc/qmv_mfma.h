@@ -682,6 +682,14 @@ inline int qmv_multi_lds(const QmvPlan& p) { return p.operands + 2 * p.waves * p
 // 4096 x 11008 17.7 -> 14.6 us, M = 8, 3072 x 8192 11.9 -> 10.1, M = 4 10.1 -> 9.4, but M = 2 8.3 -> 9.0;
 // M = 8, 2560 x 9728 g128 11.0 -> 6.4; M = 1 Q8, 4096 x 14336 (16 waves) 17.7 -> 15.4, 3072 x 18432 (12
 // waves) 15.4 -> 15.6; 18-22 rows per workgroup 5-6 % slower (M = 4, 2048 x 5120 5.1 -> 5.4).
+// Few load steps per wave and tile need more rows: with little of the stream to run on through the
+// reductions, 33 to 47 rows are three rounds of tiles as one tile each makes, and the one-tile kernels of so
+// few steps are small enough (64 registers) for twice the waves on a CU.  One tile -> several at M < 3 and
+// one step: SwiGLU [1, 1024] x Q4 g32 [11136, 1024]^T (44 rows) 5.2 -> 6.0 us, [2, 1664] x [8196, 1664]^T (33)
+// 5.1 -> 5.5, but [2, 960] x Q8 [28817, 960]^T (113) 12.1 -> 9.8; two steps: SwiGLU [1, .] Q8 g32 (35) 5.9 -> 6.9,
+// [1, .] Q4 g32 (43) 8.2 -> 7.1; eight steps: (33) 19.4 -> 17.0.  From three rows on, one step: SwiGLU M = 3
+// (36) 5.9 -> 6.6, M = 5 (34) 6.5 -> 6.8, M = 8 (34) 7.8 -> 7.4; three or more workgroups to a CU (up to 5
+// waves) M = 3 (38) 4.5 -> 4.9, M = 4 (41) 5.3 -> 5.6, M = 8 (40) 7.9 -> 6.5; else M = 3 (37) 5.6 -> 4.6.
 inline int qmv_multi_rows(const QmvArgs& a, const QmvPlan& p) {
   if (a.M < 3 && p.waves <= 12) return 0;
   const int lds = qmv_multi_lds(p);
@@ -690,7 +698,11 @@ inline int qmv_multi_rows(const QmvArgs& a, const QmvPlan& p) {
   if (kMaxLds / lds < per_cu) per_cu = kMaxLds / lds;
   const int64_t wgs = device_cu_count() * (per_cu > 0 ? per_cu : 1);
   const int64_t rows = (a.N * a.bat.count + wgs - 1) / wgs;
-  return rows >= 32 ? (int)(rows < a.N ? rows : a.N) : 0;
+  const int steps = p.steps * p.ring;
+  int64_t least = 32;
+  if (a.M < 3) least = steps == 1 ? 48 : steps == 2 ? 40 : 32;
+  else if (steps == 1 && a.M < 6 && (a.wq2 != nullptr || per_cu >= 3)) least = 48;
+  return rows >= least ? (int)(rows < a.N ? rows : a.N) : 0;
 }
 
 template <int BITS, int GS, int STEPS, int MR, int NMAT, int RING, bool MULTI>

@@ -40,3 +40,16 @@ def test_long_rows_keep_one_launch(plans):
     """Rows that fit only with two batches still go out in one launch, rows past the LDS in launches of four."""
     five, eight = plans([(5, 11008, 4096, 64, 4, 1), (8, 14336, 4096, 64, 4, 1)])
     assert five[3] == 5 and five[4] == 16 and eight[3] == 4
+
+
+# Short chains per tile take more rows before a workgroup walks several tiles; longer ones keep 32.
+@pytest.mark.parametrize("M,K,N,gs,bits,nmat,several", [
+    (1, 1024, 11136, 32, 4, 2, False), (1, 1024, 12288, 32, 4, 2, True), (2, 1664, 8196, 64, 4, 1, False),
+    (2, 960, 28817, 64, 8, 1, True), (2, 2048, 8704, 32, 4, 2, False), (2, 2048, 10240, 32, 4, 2, True),
+    (3, 640, 28426, 128, 4, 1, False), (5, 1024, 8576, 128, 4, 2, False), (8, 1024, 8576, 128, 4, 2, True),
+    (3, 1280, 9373, 128, 4, 1, True), (5, 4096, 11008, 64, 4, 2, True), (1, 4096, 14336, 64, 8, 1, True),
+    (8, 2560, 9728, 128, 4, 1, True), (2, 3072, 8192, 64, 4, 2, False),
+])
+def test_several_tiles_where_they_pay(plans, M, K, N, gs, bits, nmat, several):
+    (waves, steps, ring, _, _, rows), = plans([(M, K, N, gs, bits, nmat)])
+    assert (rows > 0) == several, (waves, steps, ring, rows)
