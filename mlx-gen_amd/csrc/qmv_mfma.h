@@ -567,6 +567,7 @@ constexpr bool qmv_ring_built(int bits, int gs, int steps, int mr, int ring) {
 constexpr bool qmv_multi_built(int bits, int gs, int steps, int mr, int nmat, int ring) {
   if (bits == 4 && gs == 32) return ring == 1 && (steps == 1 || (steps == 2 && (nmat == 1 || mr <= 2)));
   if (bits == 4 && gs == 64) return ring == 1 ? steps <= 4 || nmat == 1 : steps == 4 && nmat == 1;
+  if (bits == 4 && gs == 128) return !(steps == 8 && ring == 2 && nmat == 2);
   return true;
 }
 

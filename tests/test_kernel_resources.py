@@ -90,3 +90,9 @@ def test_gemv_arguments_are_preloaded(kernels):
         assert [t == "int" for t in args[:len(first)]] == [len(f) == 1 and f.isupper() or f == "rows" for f in first], name
         assert sum(1 if t == "int" else 2 for t in args[:len(first)]) <= 14, name
     assert len(seen) == 4
+
+
+def test_gemv_does_not_spill(kernels):
+    """Spills double a short launch's time; every form that would spill is left out of the dispatch."""
+    assert not {k: v for k, v in _gemv(kernels).items() if v[1]}
+    assert not [n for n, v in kernels.items() if re.search("(qmv|swiglu)_row_kernel<", n) and v[1]]
