@@ -221,8 +221,13 @@ int run_qmv(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq
     return run_qmm_f32(x, x_dtype, M, K, wq, s, b, sb_dtype, N, gs, bits, y, st);
   }
   // bf16 operands take the matrix-core GEMV; f32 and fp16 activations, f32 scales and a K past its
-  // reach take the VALU kernel above (same exact-f32 dequant semantics).
-  if (qmv_mfma_applicable(x_dtype, sb_dtype, M, K, N, gs, bits))
+  // reach take the VALU kernel above (same exact-f32 dequant semantics).  So does one row against many
+  // weight rows in Q8 whose K ends inside a load step (32 past a multiple of 64): the matrix cores save
+  // least there, and the tile kernel's waves share K unevenly.  VALU against tile kernel, us: [1, 800] x
+  // [14530, 800]^T 5.0 / 5.7, [1, 1248] x [13234, .] 5.0 / 7.8, [1, 5472] x [17741, .] 20.4 / 23.1, but [1, 1120] x
+  // [7789, .] 3.8 / 3.4 and in Q4 [1, 1312] x [19180, .] 6.6 / 5.5.
+  const bool valu = M == 1 && bits == 8 && K % 64 != 0 && N >= 48 * device_cu_count();
+  if (!valu && qmv_mfma_applicable(x_dtype, sb_dtype, M, K, N, gs, bits))
     return run_qmv_mfma(x, M, K, wq, s, b, N, gs, bits, y, st);
   return run_qmv_valu(x, x_dtype, M, K, wq, s, b, sb_dtype, N, gs, bits, y, st);
 }

@@ -87,3 +87,19 @@ def test_swiglu_tiles(mlxq, M, K, F, gs, bits):
         f1 = min(F, f0 + 4096)
         part = mlxq.swiglu(x, tuple(t[f0:f1].contiguous() for t in g), tuple(t[f0:f1].contiguous() for t in u), gs, bits)
         assert torch.equal(h[:, f0:f1], part)
+
+
+@pytest.mark.parametrize("K,N,valu", [(800, 14530, True), (1248, 12288, True), (32, 12300, True), (1248, 12287, False), (1280, 14530, False)])
+def test_one_row_q8_ragged_k(mlxq, K, N, valu):
+    """One Q8 row whose K ends inside a load step runs on the VALU kernel from 48 weight rows per CU on
+    (256 CUs); either kernel is within half a bf16 ulp and the f32 sums of the exact product."""
+    banner("one row q8 ragged", K, N)
+    p = _pack(K, N, K, 32, 8)
+    x = torch.randn((1, K), device="cuda").to(torch.bfloat16)
+    y = mlxq.quantized_matmul(x, *p, True, 32, 8)
+    w, mag = _dense(p, 32, 8)
+    want = x.double() @ w.t().contiguous()
+    bound = (K + 64) * 2.0 ** -24 * (x.double().abs() @ mag.t().contiguous()) + 2.0 ** -8 * want.abs()
+    assert bool(((y.double() - want).abs() <= bound).all())
+    if valu:
+        assert torch.equal(y, mlxq.qmv_valu(x, *p, 32, 8))
