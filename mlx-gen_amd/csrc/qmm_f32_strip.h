@@ -47,7 +47,10 @@ namespace {
 
 constexpr int kStripGroupM = 8;  // M-tiles per group of the tile order
 constexpr int kStripFlags = 0x00020000;  // raw buffer resource word 3 for gfx9-family loads
-// Added to an activation offset (below 2^31: 128 rows of less than 2^24 bytes), past the tile's rows: zero.
+// Widths (K and N) below which the rows of a 64-row tile stay below 2^31 bytes, as do those of a 128-row
+// tile below half of it.
+constexpr int64_t kStripReach = 1LL << 23;
+// Added to an activation offset (below 2^31), past the tile's rows: zero.
 constexpr uint32_t kStripPast = 0x80000000u;
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
@@ -666,6 +669,7 @@ static int launch_strip(const void* x, int64_t M, int64_t K, const uint32_t* wq,
 inline int strip_shape(int64_t M, int64_t K, int64_t N, int gs, bool two_pass) {
   static constexpr int kRows[4] = {128, 64, 64, 32}, kGroups[4] = {1, 1, 2, 4};
   static constexpr int kStep[2][4] = {{95, 63, 71, 63}, {170, 95, 120, 125}};  // 10 ns
+  if (K >= kStripReach / 2 || N >= kStripReach / 2) return 1;  // 32-bit offsets within a tile
   const int64_t cus = device_cu_count(), steps = K / 64;
   int best = 0;
   int64_t best_cost = 0;

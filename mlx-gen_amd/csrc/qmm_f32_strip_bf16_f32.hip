@@ -14,7 +14,7 @@ MLXQ_STRIP_ENTRY(run_strip_bf16_f32, uint16_t, float)
 // |x| from 4e34.  It is the slower one ([65, 6144] x [12288, 6144]^T 227 us against 74).  fp16 and bf16
 // activations have exact products with the codes (1.4e-7 against 2.4e-6).
 bool qmm_f32_strip_fits(int x_dtype, int64_t K, int64_t N, int gs) {
-  return K % 64 == 0 && K < (1LL << 22) && N < (1LL << 22) && !(x_dtype == MLXQ_FLOAT32 && gs == 32);
+  return K % 64 == 0 && K < kStripReach && N < kStripReach && !(x_dtype == MLXQ_FLOAT32 && gs == 32);
 }
 
 int run_qmm_f32_strip(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,

@@ -147,3 +147,29 @@ def test_strip_infinity_in_uneven_k_groups(mlxq, xdt, M, N, K, gs, bits):
         assert bool((y[row] == float("inf")).all()), k
         y[row] = clean[row]
         assert torch.equal(y, clean), k
+
+
+@pytest.mark.parametrize("xdt,M,N,K", [("f16", 70, (1 << 22) + 40, 64), ("bf16", 9, (1 << 23) - 64, 64), ("f16", 66, 33, (1 << 22) + 64)])
+def test_strip_widest(mlxq, xdt, M, N, K):
+    """Widths past 2^22: products with the codes stay exact (2e-7 of the result, where weights split into
+    bf16 parts give 2e-6).  Some columns of the wide ones, from both ends and the middle.  A long K is summed
+    in f32 over K / 64 groups, whose two terms cancel (b = -7.5 s): 2^-24 times the root of their number and
+    the terms' size, about 8 times the sum's."""
+    banner("strip widest", xdt, M, N, K)
+    g = torch.Generator(device="cuda").manual_seed(K)
+    wq = torch.randint(-2 ** 31, 2 ** 31, (N, K // 8), generator=g, device="cuda", dtype=torch.int32)
+    s = torch.randn((N, K // 64), generator=g, device="cuda") * 0.01
+    b = s * -7.5
+    x = torch.randn((M, K), generator=g, device="cuda").to(DT[xdt])
+    y = mlxq.linear(x, wq, s, b, 64, 4)
+    pick = torch.arange(N, device="cuda") if N < 1000 else torch.cat([torch.arange(n, n + 300, device="cuda") for n in (0, N // 2, N - 300)])
+    want = torch.zeros((M, len(pick)), dtype=torch.float64, device="cuda")
+    shift = torch.arange(0, 32, 4, device="cuda", dtype=torch.int32)
+    for k in range(0, K, 1 << 20):
+        k1 = min(K, k + (1 << 20))
+        codes = ((wq[pick, k // 8:k1 // 8][..., None] >> shift) & 15).view(len(pick), -1).double()
+        w = codes * s[pick, k // 64:k1 // 64].double().repeat_interleave(64, 1) + b[pick, k // 64:k1 // 64].double().repeat_interleave(64, 1)
+        want += x[:, k:k1].double() @ w.t().contiguous()
+    rel = ((y[:, pick].double() - want).norm() / want.norm()).item()
+    print(f"    rel {rel:.2e}", flush=True)
+    assert rel < (5e-7 if K < 1000 else 8 * 2.0 ** -24 * (K / 64) ** 0.5)
