@@ -686,9 +686,12 @@ inline int qmv_multi_lds(const QmvPlan& p) { return p.operands + 2 * p.waves * p
 // Few load steps per wave and tile need more rows: with little of the stream to run on through the
 // reductions, 33 to 47 rows are three rounds of tiles as one tile each makes, and the one-tile kernels of so
 // few steps are small enough (64 registers) for twice the waves on a CU.  One tile -> several at M < 3 and
-// one step: SwiGLU [1, 1024] x Q4 g32 [11136, 1024]^T (44 rows) 5.2 -> 6.0 us, [2, 1664] x [8196, 1664]^T (33)
-// 5.1 -> 5.5, but [2, 960] x Q8 [28817, 960]^T (113) 12.1 -> 9.8; two steps: SwiGLU [1, .] Q8 g32 (35) 5.9 -> 6.9,
-// [1, .] Q4 g32 (43) 8.2 -> 7.1; eight steps: (33) 19.4 -> 17.0.  From three rows on, one step: SwiGLU M = 3
+// one step: SwiGLU [1, 1024] x Q4 g32 (44 rows) 5.2 -> 6.0 us, (52 rows) 6.0 -> 7.1, [2, 1664] x [8196, 1664]^T (33)
+// 5.1 -> 5.5, but [2, 960] x Q8 [28817, 960]^T (113) 12.1 -> 9.8; two: SwiGLU [1, .] Q8 g32 (35) 5.9 -> 6.9,
+// [2, 1024] Q8 (48) 6.9 -> 7.5; six and 16 waves: SwiGLU [2, 3072] x Q8 g128 [8064, 3072]^T (32) 9.8 -> 11.3, (50)
+// 15.9 -> 15.4, but six and 13 waves, whose one-tile form leaves the CU's other slots empty: [2, 9728] x g128
+// [10101, 9728]^T (40) 22.1 -> 13.4, or whose tiles are of 8 rows: [2, 3872] x Q8 g32 [9269, 3872]^T (37) 13.2 ->
+// 9.7; eight: (33) 19.4 -> 17.0.  From three rows on, one step: SwiGLU M = 3
 // (36) 5.9 -> 6.6, M = 5 (34) 6.5 -> 6.8, M = 8 (34) 7.8 -> 7.4; three or more workgroups to a CU (up to 5
 // waves) M = 3 (38) 4.5 -> 4.9, M = 4 (41) 5.3 -> 5.6, M = 8 (40) 7.9 -> 6.5; else M = 3 (37) 5.6 -> 4.6.
 inline int qmv_multi_rows(const QmvArgs& a, const QmvPlan& p) {
@@ -701,7 +704,10 @@ inline int qmv_multi_rows(const QmvArgs& a, const QmvPlan& p) {
   const int64_t rows = (a.N * a.bat.count + wgs - 1) / wgs;
   const int steps = p.steps * p.ring;
   int64_t least = 32;
-  if (a.M < 3) least = steps == 1 ? 48 : steps == 2 ? 40 : 32;
+  if (a.M < 3) {
+    if (steps <= 2) least = a.wq2 != nullptr ? 64 : steps == 1 ? 48 : 40;
+    else if (steps < 8 && p.waves == 16 && (a.wq2 != nullptr || qmv_tile_rows(a.N, 1) > 8)) least = 48;
+  }
   else if (steps == 1 && a.M < 6 && (a.wq2 != nullptr || per_cu >= 3)) least = 48;
   return rows >= least ? (int)(rows < a.N ? rows : a.N) : 0;
 }

@@ -44,8 +44,11 @@ def test_long_rows_keep_one_launch(plans):
 
 # Short chains per tile take more rows before a workgroup walks several tiles; longer ones keep 32.
 @pytest.mark.parametrize("M,K,N,gs,bits,nmat,several", [
-    (1, 1024, 11136, 32, 4, 2, False), (1, 1024, 12288, 32, 4, 2, True), (2, 1664, 8196, 64, 4, 1, False),
-    (2, 960, 28817, 64, 8, 1, True), (2, 2048, 8704, 32, 4, 2, False), (2, 2048, 10240, 32, 4, 2, True),
+    (1, 1024, 11136, 32, 4, 2, False), (1, 1024, 13184, 32, 4, 2, False), (1, 1024, 16384, 32, 4, 2, True),
+    (2, 1664, 8196, 64, 4, 1, False), (2, 960, 28817, 64, 8, 1, True), (2, 2048, 8704, 32, 4, 2, False),
+    (2, 3072, 8064, 128, 8, 2, False), (2, 9728, 10101, 128, 4, 1, True), (2, 6528, 12017, 64, 4, 1, True),
+    (2, 3872, 9269, 32, 8, 1, True), (2, 4000, 8762, 32, 8, 1, False),
+    (2, 3072, 12288, 128, 8, 2, True), (1, 3968, 10240, 128, 8, 2, True),
     (3, 640, 28426, 128, 4, 1, False), (5, 1024, 8576, 128, 4, 2, False), (8, 1024, 8576, 128, 4, 2, True),
     (3, 1280, 9373, 128, 4, 1, True), (5, 4096, 11008, 64, 4, 2, True), (1, 4096, 14336, 64, 8, 1, True),
     (8, 2560, 9728, 128, 4, 1, True), (2, 3072, 8192, 64, 4, 2, False),
