@@ -230,8 +230,10 @@ int mlxq_linear_noalloc(const void* x, int x_dtype, int64_t M, int64_t K, const 
  * or NULL, y [E, M, N].  The reference's stacked packs carry a bf16 bias (gpt_oss.rs:478-487); an
  * f32 bias over a bf16 product would need a promoted second pass and returns MLXQ_EUNSUPPORTED.
  * x is [M, K] shared by every expert when x_per_expert == 0 (the gate_up projection of
- * gpt_oss.rs:702), else [E, M, K] (the down projection of :714).  Each expert's result equals the
- * single-matrix mlxq_linear with that bias.  bf16 x and scales run every expert in one launch with
+ * gpt_oss.rs:702), else [E, M, K] (the down projection of :714).  Each expert's result is the
+ * single-matrix mlxq_linear's with that bias: the same products, rounded at the same points.  How the f32
+ * sums over K are split follows the whole launch, so with 9 rows or more (and one row of Q8 with a ragged
+ * K) an expert's last bf16 bit may depend on how many share the stack.  bf16 x and scales run every expert in one launch with
  * M <= 8 (the GEMV's shapes), with M <= 64, K a multiple of 64 and K >= 512, and with K a multiple of
  * 64 and at least 128 GEMM tiles over all experts; otherwise the experts run one after another
  * through mlxq_linear.  All but the last of these need each expert's slices aligned: M*N elements of

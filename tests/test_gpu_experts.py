@@ -131,7 +131,9 @@ def test_experts_empty_and_mismatch(mlxq):
 ])
 def test_experts_one_launch_small_batches(mlxq, per_expert, E, M, N, K, gs, bits):
     """Up to 8 rows (GEMV) and up to 64 (K-split GEMM) in one launch over grid.y: every expert bit for
-    bit its own linear with that bias, in one-row, one-tile, several-tile and split-row forms."""
+    bit its own linear with that bias, in one-row, one-tile, several-tile and split-row forms.  (The K-split
+    GEMM splits K by eight for up to 256 tiles over all experts, as for one; larger stacks are below.)"""
+    assert M <= 8 or E * ((M + 63) // 64) * ((N + 63) // 64) <= 256
     banner("experts small batches", per_expert, E, M, N, K, gs, bits)
     g = torch.Generator(device="cuda").manual_seed(E + M)
     wq = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), generator=g, device="cuda", dtype=torch.int32)
@@ -143,6 +145,39 @@ def test_experts_one_launch_small_batches(mlxq, per_expert, E, M, N, K, gs, bits
     for e in range(E):
         xe = x[e] if per_expert else x
         one = [t[e].contiguous() for t in (wq, s, b)]
-        if M <= 8 or K >= 512 and (M + 127) // 128 * ((N + 127) // 128) < 136:
-            assert torch.equal(y[e], mlxq.linear(xe, *one, gs, bits, bias=bias[e].contiguous()))
-            assert torch.equal(plain[e], mlxq.linear(xe, *one, gs, bits))
+        assert torch.equal(y[e], mlxq.linear(xe, *one, gs, bits, bias=bias[e].contiguous()))
+        assert torch.equal(plain[e], mlxq.linear(xe, *one, gs, bits))
+
+
+# More than 256 tiles of 64 x 64 over all experts (four waves per tile): one row past the GEMV's eight and a
+# full tile of rows, ragged columns, scales that are staged (groups in eights) and not, K that the four waves
+# share unevenly.  N * M a multiple of 8: the stack's slices are aligned.
+@pytest.mark.parametrize("per_expert", [False, True])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize("E,M,N,K,gs,bits", [
+    (32, 16, 1000, 2880, 64, 4), (9, 64, 2056, 1024, 128, 4), (300, 9, 40, 576, 64, 8), (17, 33, 1032, 832, 32, 4),
+    (33, 40, 520, 512, 32, 8), (5, 57, 3352, 704, 64, 4), (64, 24, 264, 1152, 128, 8),
+])
+def test_experts_more_than_256_tiles(mlxq, per_expert, bias, E, M, N, K, gs, bits):
+    """Against float64 over the weights dequantized to bf16, within the f32 sums, (K + 4) * 2^-24 of the
+    magnitudes, and one rounding to bf16 (2^-8 of the product), a bias one more, of the sum."""
+    banner("experts past 256 tiles", per_expert, bias, E, M, N, K, gs, bits)
+    assert E * ((N + 63) // 64) > 256 and M * N % 8 == 0
+    g = torch.Generator(device="cuda").manual_seed(E + M)
+    wq = torch.randint(-2 ** 31, 2 ** 31, (E, N, K * bits // 32), generator=g, device="cuda", dtype=torch.int32)
+    mk = lambda shape, std: (torch.randn(shape, generator=g, device="cuda") * std).to(torch.bfloat16)  # noqa: E731
+    s, z, b = mk((E, N, K // gs), 0.01), mk((E, N, K // gs), 0.05), mk((E, N), 0.5) if bias else None
+    x = mk((E, M, K) if per_expert else (M, K), 1.0)
+    y = mlxq.qmm_experts(x, wq, s, z, gs, bits, bias=b, per_expert=per_expert)
+    worst = 0.0
+    for e in range(E):
+        w = mlxq.dequantize(wq[e], s[e], z[e], gs, bits).double().t().contiguous()
+        xe = (x[e] if per_expert else x).double()
+        want = xe @ w
+        bound = (K + 4) * 2.0 ** -24 * (xe.abs() @ w.abs()) + 2.0 ** -8 * want.abs()
+        if bias:
+            want = want + b[e].double()
+            bound += 2.0 ** -8 * want.abs()
+        worst = max(worst, ((y[e].double() - want).abs() / bound).max().item())
+    print(f"    worst error / bound {worst:.3f}", flush=True)
+    assert worst <= 1
