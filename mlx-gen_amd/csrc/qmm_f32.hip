@@ -131,15 +131,15 @@ __device__ __forceinline__ void f32_tile_coords(int64_t bid, int64_t tiles_m, in
 // WAVES: 4 (2 x 2 waves of 64 x 64) or 8 (2 x 4 waves of 64 x 32, two per SIMD).  EPI: the f32
 // epilogue (dense bias in its own dtype, then the f32 activation) is applied before the store.
 // WT: uint32_t for packed codes (wq, scales, biases); uint16_t (bf16) or float for a dense [N, K]
-// weight matrix passed in wq's place (scales, biases, BITS and GS unused), the LoKr residual's
+// weight matrix passed in wq's place (scales, biases, BITS and gs_log2 unused), the LoKr residual's
 // x . delta^T.  A dense f32 matrix against bf16 activations is rounded to bf16 first (MLX casts
-// the delta to the activation dtype).
-template <typename XT, typename SB, int BITS, int GS, int WAVES, int BN, int BK, bool EPI,
-          typename WT = uint32_t>
+// the delta to the activation dtype).  gs_log2: the group size, at run time: a thread's codes of a step lie in
+// one group whatever it is, and only sizes past the factored kernel's reach bring 64 and 128 here.
+template <typename XT, typename SB, int BITS, int WAVES, int BN, int BK, bool EPI, typename WT = uint32_t>
 __global__ __launch_bounds__(WAVES * 64) void qmm_f32_kernel(const XT* __restrict__ x, int64_t M,
                                                          int64_t K, const uint32_t* __restrict__ wq,
                                                          const SB* __restrict__ scales,
-                                                         const SB* __restrict__ biases, int64_t N,
+                                                         const SB* __restrict__ biases, int64_t N, int gs_log2,
                                                          float* __restrict__ y, F32Epilogue epi) {
   constexpr bool XLO = XStore<XT>::LO;  // activations carry a low part
   constexpr bool DENSE = !std::is_same<WT, uint32_t>::value;
@@ -168,7 +168,7 @@ __global__ __launch_bounds__(WAVES * 64) void qmm_f32_kernel(const XT* __restric
   f32_tile_coords(blockIdx.x, tiles_m, tiles_n, tm, tn);
   const int64_t bm0 = tm * BM, bn0 = tn * BN;
   const int64_t kwords = K * BITS / 32;
-  const int64_t groups = K / GS;
+  const int64_t groups = K >> gs_log2;
   const int ksteps = (int)((K + BK - 1) / BK);
 
   // Staging registers, two slots (steps of even / odd parity): activation chunks (8 values each:
@@ -212,7 +212,7 @@ __global__ __launch_bounds__(WAVES * 64) void qmm_f32_kernel(const XT* __restric
           b_reg[sl][q + 1] = v[1];
         }
       }
-      const int64_t g = n * groups + kc / GS;
+      const int64_t g = n * groups + (kc >> gs_log2);
       s_reg[sl] = SBLoad<SB>::ld(scales, g);
       z_reg[sl] = SBLoad<SB>::ld(biases, g);
     }
@@ -433,9 +433,9 @@ __global__ __launch_bounds__(WAVES * 64) void qmm_f32_kernel(const XT* __restric
   f32_store_dispatch<EPI>(epi.act, store);
 }
 
-template <typename XT, typename SB, int BITS, int GS>
+template <typename XT, typename SB, int BITS>
 static int launch_qmm_f32(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
-                          const void* b, int64_t N, void* y, const F32Epilogue& epi, hipStream_t st) {
+                          const void* b, int64_t N, int gs, void* y, const F32Epilogue& epi, hipStream_t st) {
   // 8 waves (2 x 4 of 64 x 64) on 128 x 256 tiles with 32-deep K steps (96 KB of LDS, one
   // workgroup per CU).  With loads two steps ahead, same-box A/B on the FLUX shapes (f32 x, Q4
   // g64, up / down in ms): this form 1.103 / 1.346; 4 waves on 128 x 128 (two workgroups per CU)
@@ -446,13 +446,14 @@ static int launch_qmm_f32(const void* x, int64_t M, int64_t K, const uint32_t* w
   const int64_t tiles = ((M + kF32BM - 1) / kF32BM) * ((N + BN - 1) / BN);
   if (tiles == 0) return MLXQ_OK;
   if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "qmm_f32: problem too large");
+  const int gs_log2 = gs == 32 ? 5 : gs == 64 ? 6 : 7;
   if (epi.bias || epi.act != MLXQ_ACT_NONE)
-    hipLaunchKernelGGL((qmm_f32_kernel<XT, SB, BITS, GS, WAVES, BN, BK, true>), dim3((unsigned)tiles),
-                       dim3(WAVES * 64), 0, st, (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N,
+    hipLaunchKernelGGL((qmm_f32_kernel<XT, SB, BITS, WAVES, BN, BK, true>), dim3((unsigned)tiles),
+                       dim3(WAVES * 64), 0, st, (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N, gs_log2,
                        (float*)y, epi);
   else
-    hipLaunchKernelGGL((qmm_f32_kernel<XT, SB, BITS, GS, WAVES, BN, BK, false>), dim3((unsigned)tiles),
-                       dim3(WAVES * 64), 0, st, (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N,
+    hipLaunchKernelGGL((qmm_f32_kernel<XT, SB, BITS, WAVES, BN, BK, false>), dim3((unsigned)tiles),
+                       dim3(WAVES * 64), 0, st, (const XT*)x, M, K, wq, (const SB*)s, (const SB*)b, N, gs_log2,
                        (float*)y, epi);
   return check_launch("qmm_f32");
 }
@@ -461,10 +462,10 @@ template <typename XT, typename SB>
 static int qmm_f32_bits_gs(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                            const void* b, int64_t N, int gs, int bits, void* y, const F32Epilogue& epi,
                            hipStream_t st) {
-#define MLXQ_F(B, G) \
-  if (bits == B && gs == G) return launch_qmm_f32<XT, SB, B, G>(x, M, K, wq, s, b, N, y, epi, st);
-  MLXQ_F(4, 32) MLXQ_F(4, 64) MLXQ_F(4, 128) MLXQ_F(8, 32) MLXQ_F(8, 64) MLXQ_F(8, 128)
-#undef MLXQ_F
+  if (gs == 32 || gs == 64 || gs == 128) {
+    if (bits == 4) return launch_qmm_f32<XT, SB, 4>(x, M, K, wq, s, b, N, gs, y, epi, st);
+    if (bits == 8) return launch_qmm_f32<XT, SB, 8>(x, M, K, wq, s, b, N, gs, y, epi, st);
+  }
   return set_error(MLXQ_EINVAL, "qmm_f32: unsupported bits=%d group_size=%d", bits, gs);
 }
 
@@ -501,8 +502,8 @@ int run_dense_f32(const void* x, int x_dtype, int64_t M, int64_t K, const void* 
   if (tiles > 0x7fffffff) return set_error(MLXQ_EINVAL, "dense product: problem too large");
   const F32Epilogue none{};
 #define MLXQ_D(XT, WT)                                                                                    \
-  hipLaunchKernelGGL((qmm_f32_kernel<XT, float, 4, 32, WAVES, BN, BK, false, WT>), dim3((unsigned)tiles), \
-                     dim3(WAVES * 64), 0, st, (const XT*)x, M, K, (const uint32_t*)d, nullptr, nullptr, N, y, none)
+  hipLaunchKernelGGL((qmm_f32_kernel<XT, float, 4, WAVES, BN, BK, false, WT>), dim3((unsigned)tiles), \
+                     dim3(WAVES * 64), 0, st, (const XT*)x, M, K, (const uint32_t*)d, nullptr, nullptr, N, 5, y, none)
   if (x_dtype == MLXQ_BFLOAT16) {
     if (d_dtype == MLXQ_BFLOAT16) MLXQ_D(uint16_t, uint16_t);
     else MLXQ_D(uint16_t, float);
