@@ -234,8 +234,7 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
         xr[i][q] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rx, x_off[i] + at + 16u * q, 0, 0));
   };
   float* const xtab = reinterpret_cast<float*>(lds + OFF_X);
-  constexpr int XPASS = BM / NS > 16 ? BM / NS / 16 : 1;
-  float xrun[XF32 ? A_LD : XPASS];  // GS 128: a row's sum over its group's first step
+  float xrun[XF32 ? A_LD : 1];  // GS 128: a row's sum over its group's first step
   // X of group g for tile row `row`; the lanes that share a row write the same value.
   auto put_x = [&](int row, int g, float v) { xtab[(g & 7) * BM + row] = v; };
   // f32: split step t's registers into its stage and leave the group sums.  POS: t's position in its
@@ -275,12 +274,11 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     }
   };
   // fp16 / bf16: the group sums of step t from its landed stage, BM / NS rows per wave, four lanes a
-  // row (two chunks each), 16 rows at a time.
+  // row (two chunks each).
   auto sum_x = [&](int t, auto POS) {
     constexpr int RW = BM / NS;
-#pragma unroll
-    for (int ps = 0; ps < XPASS; ++ps) {
-    const int row = wave * RW + 16 * ps + ((lane >> 2) & (RW < 16 ? RW - 1 : 15)), q = lane & 3;
+    static_assert(RW == 16 || RW == 8, "rows of a wave: all its lanes, or twice over");
+    const int row = wave * RW + ((lane >> 2) & (RW - 1)), q = lane & 3;
     const unsigned char* const base = stage_at(t) + row * 128;
     float part[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -305,9 +303,8 @@ __global__ __launch_bounds__(512) void qmm_f32_strip_kernel(const XT* __restrict
     } else {
       sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4e, 0xf, 0xf, true));
       if constexpr (GS == 64) put_x(row, t, sum);
-      else if constexpr (decltype(POS)::value == 0) xrun[ps] = sum;
-      else put_x(row, t >> 1, xrun[ps] + sum);
-    }
+      else if constexpr (decltype(POS)::value == 0) xrun[0] = sum;
+      else put_x(row, t >> 1, xrun[0] + sum);
     }
   };
 
