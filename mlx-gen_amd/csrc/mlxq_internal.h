@@ -66,8 +66,8 @@ int run_quantize_batched(const void* const* w, int count, int dtype, int64_t N, 
                          uint32_t* const* wq, void* const* s, void* const* b, hipStream_t st);
 int run_dequantize(const uint32_t* wq, const void* s, const void* b, int dtype, int64_t N, int64_t K,
                    int gs, int bits, void* out, hipStream_t st);
-// The f32-dequant product; y in promote(x_dtype, sb_dtype): the GEMV for M <= 8 (exact f32), the
-// split-bf16 GEMM for larger M (f32 operands, within ~1e-5 relative of the f32 product).
+// The f32-dequant product; y in promote(x_dtype, sb_dtype): a GEMV for M <= 8 (exact f32 dequantization),
+// run_qmm_f32 for larger M (f32 or fp16 x and / or f32 scales; bf16 against bf16 is refused there).
 int run_qmv(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
             const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, hipStream_t st);
 int run_qmm(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void* s, const void* b,
@@ -117,8 +117,9 @@ struct F32Epilogue {
   int R = 0;                   // padded rank, 0 = no LoRA
   float lora_scale = 1.0f;
 };
-// Large-M GEMM for operands MLX computes in f32 (f32 x and/or f32 scales), f32 y, as three bf16
-// MFMA passes over two-term bf16 splits of x and of the f32-dequantized weights.
+// Large-M GEMM for operands MLX computes in f32 (fp16 or f32 x and/or f32 scales), f32 y: the factored
+// kernel where it takes the problem (qmm_f32_strip_fits), else three bf16 MFMA passes over two-term
+// bf16 splits of x and of the f32-dequantized weights (no LoRA residual).
 int run_qmm_f32(const void* x, int x_dtype, int64_t M, int64_t K, const uint32_t* wq, const void* s,
                 const void* b, int sb_dtype, int64_t N, int gs, int bits, void* y, hipStream_t st,
                 const F32Epilogue& epi = F32Epilogue{});

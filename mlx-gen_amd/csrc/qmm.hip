@@ -297,8 +297,8 @@ int run_qmm(const void* x, int64_t M, int64_t K, const uint32_t* wq, const void*
   if (K % 64 == 0 && (wide_tiles >= 128 || narrow_tiles >= 128 || mid_tiles >= kQmmMidMinTiles) &&
       qmm_wide_fits(M, K, N, gs, bits, sb_dtype == MLXQ_BFLOAT16 ? 2 : 4))
     return run_qmm_wide(x, M, K, wq, s, b, sb_dtype, N, gs, bits, y, epi, st);
-  // Small grids with a long K: the K-split kernel (64x64 tiles, 8 waves each taking a slice of
-  // K).  Measured against the tile kernel on N = K = 3072 (Q4 g64): 13 vs 59 us at M = 256,
+  // Small grids with a long K: the K-split kernel (64x64 tiles, 8 or 4 waves each taking a slice
+  // of K).  Measured against the tile kernel on N = K = 3072 (Q4 g64): 13 vs 59 us at M = 256,
   // 42 vs 72 us at M = 1024 (768 small tiles), 65 vs 73 us at M = 1536 (1152), 77 vs 75 us at
   // M = 2048 (1536); M = 512, N = 9216 with bias and GELU (1152) 86 vs 87 us.
   const int64_t small_tiles = ((M + 63) / 64) * ((N + 63) / 64);

@@ -17,9 +17,13 @@
 // Workgroup: 8 waves, tile BM (128 or 64) x 256 TN, K advanced 64 per step; wave w owns TN strips of 32
 // columns, all BM rows of them.  Small grids (strip_shape) take KS = 2 or 4 K-groups of 8 / KS
 // waves instead: each group walks its own share of K, with its own activation ring, over the same
-// 256 / KS columns, and the partial sums meet in LDS at the end.  What bounds it is the LDS port: a wave reads 1 KB of activations
-// per MFMA (32 cycles of one SIMD's matrix core; four SIMDs against 128 bytes per cycle).  Hence the
-// weights never pass through LDS: a lane loads its own column's packed words two steps ahead and
+// 256 / KS columns, and the partial sums meet in LDS at the end.  What bounds it is the vector and
+// matrix work of a SIMD's two waves: the code conversions and folds keep its vector unit busy about as
+// long as the MFMAs keep its matrix core (counters, share of the SIMD's cycles, matrix / vector: [4096,
+// 1280] fp16 x Q4 [10240, 1280]^T 37 / 48 %, [4608, 3072] f32 x Q4 [12288, 3072]^T 53 / 52 %), and two
+// waves overlap them only in part.  The LDS port, at 1 KB of activations a wave and MFMA, has room
+// (24 and 19 % of the CU's cycles).
+// The weights never pass through LDS: a lane loads its own column's packed words two steps ahead and
 // converts them straight into its MFMA operand, each code once per workgroup, and with the codes
 // as the MFMA's B side a lane holds 16 rows of ONE column, so the fold's scale is a single register.
 // fp16 and bf16 activations go global -> LDS by direct-to-LDS loads three steps ahead into a 4-stage
@@ -655,7 +659,8 @@ static int launch_strip(const void* x, int64_t M, int64_t K, const uint32_t* wq,
 }
 
 // Tile height and K-groups: 0: 128 rows; 1: 64 rows; 2: 64 rows in 2 K-groups; 3: 32 rows in 4.
-// One workgroup runs per CU, so a shape costs its rounds of tiles times its chain of K steps: the
+// One workgroup runs per CU (512 threads at 141 registers or more, or 84 KB of LDS or more: a second one fits
+// beside none of the four), so a shape costs its rounds of tiles times its chain of K steps: the
 // shape with the least rounds * (steps * t + 5 us), with t, the measured time of a step (us), 0.95 /
 // 0.63 / 0.71 / 0.63 for one pass and 1.7 / 0.95 / 1.2 / 1.25 for two.  Measured, us for shapes 0..3
 // (Q4 g64 unless stated): fp16 77 x 1280 x 5120 Q8 26.4 / 19.1 / 13.9 / 9.3, 77 x 5120 x 1280 81.7 /
@@ -689,11 +694,12 @@ static int strip_tile(const void* x, int64_t M, int64_t K, const uint32_t* wq, c
   switch (strip_shape(M, K, N, GS, std::is_same<XT, float>::value)) {
     case 0:
       // f32 activations, Q4, more than a round and a half of tiles: 64 x 512 instead of 128 x 256, two
-      // strips per wave.  Both activation parts are then read from LDS for two strips' MFMAs instead of
-      // one (half the LDS reads), for twice the code conversions.  Same-process A/B, 128 x 256 ->
+      // strips per wave: half the LDS reads of activations, for twice the code conversions, which two passes'
+      // MFMAs hide.  Same-process A/B, 128 x 256 ->
       // 64 x 512: 4608 x 3072 x 12288 694 -> 648 us, 4608 x 12288 x 3072 748 -> 713, 4608 x 3072 x 3072
       // g128 175 -> 164; 1024 x 3072 x 12288 (1.5 rounds) 171 -> 174.  Q8 needs twice the weight
-      // registers and spills (4608 x 3072 x 9216 597 -> 630); fp16's one pass has no second use.
+      // registers and spills (4608 x 3072 x 9216 597 -> 630).  fp16 has one pass and loses by the
+      // conversions (4096 x 1280 x 10240 152 -> 166, 2048 x 3072 x 12288 190 -> 204; 233 registers, no spill).
       if constexpr (std::is_same<XT, float>::value && BITS == 4) {
         if (((M + 63) / 64) * ((N + 511) / 512) * 2 > device_cu_count() * 3)
           return launch_strip<XT, SB, BITS, GS, 64, 1, 2>(x, M, K, wq, s, b, N, y, epi, st);

@@ -656,7 +656,7 @@ struct QmvArgs {
 // Rows per workgroup of one tile: 16 for SwiGLU; for one matrix, of 16, 12 and 8 the count whose
 // busiest CU streams the fewest rows (the MFMA columns past the count load nothing).  The down
 // projection of a decode MLP (N = 3072) takes 12 rows: 256 workgroups, every CU, where 16-row tiles
-// left 64 CUs idle.
+// left 64 CUs idle.  Stacked experts choose as one of them alone would.
 inline int qmv_tile_rows(int64_t N, int nmat) {
   if (nmat == 2) return 16;
   const int64_t cus = device_cu_count();

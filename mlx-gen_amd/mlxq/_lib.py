@@ -142,7 +142,7 @@ _fast = None
 
 
 def fast():
-    """The native call path of the operators (_fast.so, host/fast.cpp): each function returns None for
+    """The native call path of the operators (host/fast.cpp): each function returns None for
     a call whose operands need preparation or that is refused, and the caller takes its general path; a
     device error is raised as MlxqError.  It only saves host time: where it is not built for this
     Python and torch, every call takes its general path."""

@@ -14,7 +14,7 @@ is f32); a bias add or a LoRA residual in f32 promotes the result to f32.  Every
 against x before anything is launched, as MLX's quantized_matmul checks them; failures raise
 ``MlxqError`` with status MLXQ_EINVAL, and library errors carry the library's status and message.
 The decode-sized calls go through the native module (_lib.fast) when their operands need no
-preparation; the code here is the general path and the one that reports errors.
+preparation; the code here is the general path and reports what is refused.
 """
 from __future__ import annotations
 
@@ -256,8 +256,9 @@ def qmv(x, wq, scales, biases, group_size: int = DEFAULT_GROUP_SIZE, bits: int =
 
 
 def qmv_valu(x, wq, scales, biases, group_size: int = DEFAULT_GROUP_SIZE, bits: int = 4, out=None):
-    """Force the VALU GEMV (no matrix cores; M <= 8), the kernel quantized_matmul runs for f32
-    operands and group size 32, on any operand dtypes."""
+    """Force the VALU GEMV (no matrix cores; M <= 8), the kernel quantized_matmul runs for
+    fp16 and f32 operands, K past the matrix-core kernels' reach and a few one-row bf16 shapes, on any
+    operand dtypes."""
     return _mm("mlxq_qmv_valu", x, wq, scales, biases, group_size, bits, out=out)
 
 

@@ -1,10 +1,11 @@
-"""GPU parity of the f32 large-M GEMM (qmm_f32.hip): operands MLX computes in f32 at M > 8.
+"""GPU parity of the f32 large-M GEMMs (qmm_f32_strip.h, qmm_f32.hip): operands MLX computes in f32 at M > 8.
 
 FLUX.1's residual stream is f32 (mlx-gen-flux/src/model.rs:407-410) and quantized_matmul takes the
 activations as they come (src/adapters.rs:301-317), so an f32 x against bf16 (or f32) scales is
 an f32 product: x, scales and biases cast to f32, weights dequantized in f32, f32 accumulation.
-The kernel carries both operands as two-term bf16 splits and adds three bf16 MFMA products.  The
-checks hold it to the exact f32 oracle (fp64 over the f32-dequantized weights) at relFro < 1e-4,
+The factored kernel carries f32 activations as two-term bf16 splits against the exact codes (two bf16
+MFMA products; one for bf16 activations); the three-pass kernel, which serves f32 activations at group
+size 32 and K that is no multiple of 64, carries both operands as two-term splits.  The checks hold it to the exact f32 oracle (fp64 over the f32-dequantized weights) at relFro < 1e-4,
 and to at least ten times closer than the same product with x rounded to bf16 — what a single
 bf16 pass would give — so a missing correction pass fails them.
 """
@@ -30,10 +31,9 @@ def _tdt(name):
 
 
 # (M, N, K, gs, bits, x dtype, scales dtype): ragged M and N (N % 4 != 0), every group size,
-# Q4 and Q8, f32 or bf16 scales, bf16 x against f32 scales, the M = 9 boundary.  Group sizes 64
-# and 128 run the factored kernel; with bf16 scales and K / gs a multiple of 16 its bias term goes
-# through the batched MFMA (the last four cases: one, three, two and one 16-group batches, the
-# last at the M = 9 boundary).
+# Q4 and Q8, f32 or bf16 scales, bf16 x against f32 scales, the M = 9 boundary.  f32 x at group
+# size 32 runs the three-pass kernel, the rest the factored one (the last four cases with 16, 48, 32
+# and 16 groups along K, the last at the M = 9 boundary).
 CASES = [
     (200, 198, 512, 64, 4, "f32", "bf16"),
     (130, 264, 1024, 32, 8, "f32", "f32"),
