@@ -17,12 +17,12 @@
 // Workgroup: 8 waves, tile BM (128 or 64) x 256 TN, K advanced 64 per step; wave w owns TN strips of 32
 // columns, all BM rows of them.  Small grids (strip_shape) take KS = 2 or 4 K-groups of 8 / KS
 // waves instead: each group walks its own share of K, with its own activation ring, over the same
-// 256 / KS columns, and the partial sums meet in LDS at the end.  What bounds it is the vector and
-// matrix work of a SIMD's two waves: the code conversions and folds keep its vector unit busy about as
-// long as the MFMAs keep its matrix core (counters, share of the SIMD's cycles, matrix / vector: [4096,
-// 1280] fp16 x Q4 [10240, 1280]^T 37 / 48 %, [4608, 3072] f32 x Q4 [12288, 3072]^T 53 / 52 %), and two
-// waves overlap them only in part.  The LDS port, at 1 KB of activations a wave and MFMA, has room
-// (24 and 19 % of the CU's cycles).
+// 256 / KS columns, and the partial sums meet in LDS at the end.  No unit is
+// saturated; what bounds it is how far a SIMD's two waves overlap the matrix work with the vector work
+// (code conversions, folds), which takes about as long (counters, share of the SIMDs' cycles, matrix /
+// vector at 4 cycles an instruction, and of the CUs' cycles, LDS at 8 cycles a KB: [4096, 1280] fp16 x Q4
+// [10240, 1280]^T 37 / 44 / 41 %, [4608, 3072] f32 x Q4 [12288, 3072]^T 53 / 46 / 31 %).  Trading LDS
+// reads for conversions moves it by less than 10 % either way (strip_tile).
 // The weights never pass through LDS: a lane loads its own column's packed words two steps ahead and
 // converts them straight into its MFMA operand, each code once per workgroup, and with the codes
 // as the MFMA's B side a lane holds 16 rows of ONE column, so the fold's scale is a single register.
